@@ -88,3 +88,39 @@ def test_cutout_cleaning_chain_matches_oracle():
     g = torch.from_numpy(x.copy()).cuda()
     rfi.kadane_f(rfi.zdot(g), td, fd, 5.0, wl)
     assert np.array_equal(g.cpu().numpy().view(np.uint32), ref.view(np.uint32))
+
+
+def same_bits(a, b):
+    """Equal bit for bit, a NaN equal to any NaN."""
+    nan = np.isnan(b)
+    return np.array_equal(np.isnan(a), nan) and np.array_equal(
+        np.where(nan, 0, a).view(np.uint32), np.where(nan, 0, b).view(np.uint32))
+
+
+# around the time-major kernels' edges: 32 channels a workgroup (31 takes the
+# general kernels, 33 overlaps two groups), 128 samples a chunk, 32 samples
+# and 128 channels a normalisation tile
+@pytest.mark.parametrize("nchan,nsamp,nf", [(31, 70, 1), (32, 128, 2), (33, 129, 1), (64, 1, 1), (95, 127, 1),
+                                            (129, 257, 2), (300, 33, 1)])
+def test_time_major_zdot_and_kadanef_edges(nchan, nsamp, nf):
+    import torch
+
+    from transientx_amd import rfi
+
+    say("case time-major nchan", nchan, "nsamp", nsamp, "frames", nf)
+    x = frames(5 * nchan + nsamp, nf, nchan, max(nsamp, 8))[:, :, :nsamp].copy()
+    x[0, 3, nsamp // 2] = np.inf if nchan % 2 else np.nan
+    ref = np.stack([oracle.zdot(x[f]) for f in range(nf)])
+    t = torch.from_numpy(np.ascontiguousarray(x.transpose(0, 2, 1))).cuda()
+    rfi.zdot(t, layout="time")
+    assert same_bits(np.ascontiguousarray(t.cpu().numpy().transpose(0, 2, 1)), ref)
+    for td, fd in ((1, 1), (2, 1), (1, 2)):
+        y = np.nan_to_num(ref, nan=1.5, posinf=2.0, neginf=-2.0)
+        y[0, 5, :] = -np.abs(y[0, 5, :])  # a channel whose sum only falls
+        y[0, 6, nsamp // 3] = np.inf
+        y[0, 7, nsamp // 4] = np.nan
+        wl = [2 * f for f in range(nf)]
+        r = np.stack([oracle.kadanef(y[f], td, fd, 3.0, wl[f]) for f in range(nf)])
+        t = torch.from_numpy(np.ascontiguousarray(y.transpose(0, 2, 1))).cuda()
+        rfi.kadane_f(t, td, fd, 3.0, wl, layout="time")
+        assert same_bits(np.ascontiguousarray(t.cpu().numpy().transpose(0, 2, 1)), r), (td, fd)

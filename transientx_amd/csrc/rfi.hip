@@ -261,133 +261,311 @@ __global__ __launch_bounds__(256) void k_zdot_rows(Frames F, const double *s, co
     (void)j;
 }
 
-// Time-major frames (cstride 1): lanes are consecutive channels (coalesced
-// at every sample); each lane keeps U loads in flight ahead of its
-// sequential sums.  A block has only nchan such threads (64 wavefronts at
-// 4096 channels), so memory parallelism comes from U.
-template <bool FIT>
-__global__ __launch_bounds__(256) void k_zdot_cols(Frames F, const double *s, const double *sess)
+// ---- Time-major frames (cstride 1), the DataBuffer layout.  A channel's sums
+// run over all its samples one after the other, so a search block (26,123
+// samples of 4096 channels) is 4096 chains of 26,123 dependent FP64 adds and
+// nothing shorter; what can be chosen is what a step of the chain costs.  On
+// gfx950 a dependent FP64 add or FMA issues every 4.5 cycles and a
+// conversion every 5.5 (measured), so the chains get a wave of their own
+// (wave 0 of the workgroup, which only reads LDS, converts and adds) and
+// four helper waves bring the samples: 32 channels (one 128-byte line of a
+// sample) per workgroup, so that 4096 channels use 128 CUs, and both of a
+// channel's sums in the same wave (lane l and lane l + 32).  The helpers keep
+// two chunks of kColT samples in registers on their way from HBM while a
+// third is written to LDS and a fourth is summed.
+constexpr int kColCh = 32, kColT = 128, kColThreads = 64 + 256;
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4))); // 4-byte aligned 16-byte access
+
+// n steps of a chain, 16 at a time: get(i) reads the operands of 16 steps while
+// the 16 before them run (the scheduling barriers keep the reads ahead).
+template <int n, class T, class Get, class Step>
+__device__ __forceinline__ void chain16(Get get, Step step)
 {
-    constexpr int U = 32;
-    const long g = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= (long)F.nframes * F.nchan) return;
-    const long f = g / F.nchan, j = g % F.nchan;
-    float *col = F.x + f * F.fstride + j;
-    const long ts = F.tstride, N = F.nsamp;
-    const double *sf = s + f * N; // read only when FIT
-    // One sweep over the column in batches of U samples; the next batch's
-    // loads are issued before the current batch is processed, so they
-    // overlap it.  body(i, v, sv) handles samples i..i+U-1 in order.
-    auto sweep = [&](auto body, auto tail) {
-        long i = 0;
-        if (N >= U) {
-            float nx[U];
-            double snx[U];
+    T x0[16], x1[16];
+    auto fetch = [&](T(&x)[16], int i) {
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int u = 0; u < U; u++) {
-                nx[u] = col[u * ts];
-                if (FIT) snx[u] = sf[u];
-            }
-            for (; i + U <= N; i += U) {
-                float v[U];
-                double sv[U];
-#pragma unroll
-                for (int u = 0; u < U; u++) {
-                    v[u] = nx[u];
-                    if (FIT) sv[u] = snx[u];
-                }
-                if (i + 2 * U <= N) {
-#pragma unroll
-                    for (int u = 0; u < U; u++) {
-                        nx[u] = col[(i + U + u) * ts];
-                        if (FIT) snx[u] = sf[i + U + u];
-                    }
-                }
-                body(i, v, sv);
-            }
-        }
-        for (; i < N; i++) tail(i);
+        for (int u = 0; u < 16; u++) x[u] = get(i + u);
+        __builtin_amdgcn_sched_barrier(0);
     };
-    double a = 0., b = 0.;
-    sweep(
-        [&](long i, const float *v, const double *sv) {
+    fetch(x0, 0);
 #pragma unroll
-            for (int u = 0; u < U; u++) {
-                a += v[u];
-                if (FIT) b = fma((double)v[u], sv[u], b);
-                else b += v[u] * v[u];
-            }
-        },
-        [&](long i) {
-            const float v = col[i * ts];
-            a += v;
-            if (FIT) b = fma((double)v, sf[i], b);
-            else b += v * v;
-        });
-    double m = 0., sd = 1., alpha = 0., beta = 0.;
-    if (!FIT) {
-        m = a / N;
-        sd = b / N;
-        sd = fma(-m, m, sd);
-        sd = sqrt(sd);
-        if (sd == 0.) sd = 1.;
-    } else {
-        const double se = sess[2 * f], ss = sess[2 * f + 1], nb = (double)N;
-        const double tmp = fma(se, se, -(ss * nb));
-        if (tmp != 0) {
-            alpha = fma(a, se, -(b * nb)) / tmp;
-            beta = fma(b, se, -(a * ss)) / tmp;
-        }
+    for (int i = 0; i < n; i += 32) {
+        fetch(x1, i + 16);
+#pragma unroll
+        for (int u = 0; u < 16; u++) step(i + u, x0[u]);
+        if (i + 32 < n) fetch(x0, i + 32);
+#pragma unroll
+        for (int u = 0; u < 16; u++) step(i + 16 + u, x1[u]);
     }
-    auto update = [&](float v, double sv) {
-        if (FIT) return (float)((double)v - fma(alpha, sv, beta));
-        return (float)((double)((float)((double)v - m)) / sd);
-    };
-    sweep(
-        [&](long i, const float *v, const double *sv) {
-#pragma unroll
-            for (int u = 0; u < U; u++) col[(i + u) * ts] = update(v[u], FIT ? sv[u] : 0.);
-        },
-        [&](long i) { col[i * ts] = update(col[i * ts], FIT ? sf[i] : 0.); });
 }
 
-// The channel mean for time-major frames: a workgroup takes 64 samples;
-// 64-channel tiles of their rows pass through LDS, each lane (sample) then
-// sums its row's channels in order.
-__global__ __launch_bounds__(64) void k_zdot_s_rows(Frames F, double *s)
+// The streaming part: chunks of kColT samples of 32 columns (ts floats from
+// sample to sample, N samples) pass through buf; put(k, v) of a helper
+// thread (h < 256) stores columns q4 .. q4 + 3 of its samples r0 + 32*u
+// of chunk k, chain(k) of wave 0 works on chunk k, buf half k & 1.
+struct ColChunk {
+    f4u v[4];
+    double s;
+};
+template <class Put, class Chain>
+__device__ __forceinline__ void stream_columns(const float *__restrict__ col, const double *__restrict__ sf, long N,
+                                               long ts, Put put, Chain chain)
 {
-    __shared__ float T[64][65];
-    const int lane = threadIdx.x;
-    const long g0 = (long)blockIdx.x * 64; // first (frame, sample)
-    const long ntot = (long)F.nframes * F.nsamp;
-    const int nrow = (int)min((long)64, ntot - g0);
-    double a = 0.;
-    auto rowp = [&](int r) -> const float * {
-        const long gr = g0 + r;
-        return F.x + (gr / F.nsamp) * F.fstride + (gr % F.nsamp) * F.tstride;
+    const int tid = threadIdx.x, h = tid - 64, q4 = (h & 7) * 4, r0 = h >> 3;
+    const int nk = (int)((N + kColT - 1) / kColT);
+    auto load = [&](int k, ColChunk &c) { // past the end: a sample that exists, unused
+        const long t0 = (long)k * kColT;
+#pragma unroll
+        for (int u = 0; u < 4; u++) c.v[u] = *(const f4u *)(col + min(t0 + r0 + 32 * u, N - 1) * ts + q4);
+        if (sf) c.s = sf[min(t0 + (h & (kColT - 1)), N - 1)];
     };
-    for (int c0 = 0; c0 < F.nchan; c0 += 64) {
-        const int n = min(64, F.nchan - c0);
-        const int cl = c0 + min(lane, n - 1);
-        // 16 row loads in flight (addresses clamped to rows and channels that exist)
-        for (int r0 = 0; r0 < nrow; r0 += 16) {
-            float v[16];
-#pragma unroll
-            for (int u = 0; u < 16; u++) v[u] = rowp(min(r0 + u, nrow - 1))[cl];
-#pragma unroll
-            for (int u = 0; u < 16; u++)
-                if (r0 + u < nrow && lane < n) T[r0 + u][lane] = v[u];
+    ColChunk A, B;
+    if (tid >= 64) {
+        load(0, A);
+        load(1, B);
+        put(0, A);
+        load(2, A);
+    } else {
+        __builtin_amdgcn_s_setprio(3); // the chain wave goes first on its SIMD
+    }
+    __syncthreads();
+    for (int k = 0; k < nk; k += 2) {
+        if (tid < 64) {
+            chain(k);
+        } else {
+            put(k + 1, B);
+            load(k + 3, B);
         }
         __syncthreads();
-        if (lane < nrow)
-            for (int c = 0; c < n; c++) a += T[lane][c];
+        if (k + 1 >= nk) break;
+        if (tid < 64) {
+            chain(k + 1);
+        } else {
+            put(k + 2, A);
+            load(k + 4, A);
+        }
         __syncthreads();
     }
-    if (lane < nrow) s[g0 + lane] = a / F.nchan;
+}
+
+// FIT = false: mean and standard deviation of each channel (candidate.cpp:837-851)
+// into stat[2*(f*nchan + j)].  FIT = true: sum x and sum x*s of each
+// (already normalised) channel (:870-880) into the same place, and, in one
+// extra workgroup per frame, sum s and sum s^2 into sess.  4096 channels x
+// 26,123 samples (428 MB): 177 us and 214 us, 16 and 20 cycles a sample; one
+// lane per channel loading for itself took 1.9 and 1.4 ms (with the update).
+template <bool FIT>
+__global__ __launch_bounds__(kColThreads) void k_zdot_chain(Frames F, const double *__restrict__ s, double *stat,
+                                                            double *sess)
+{
+    constexpr int RS = FIT ? kColCh : 2 * kColCh; // floats per sample: x, or x then x*x
+    __shared__ __attribute__((aligned(16))) float buf[2][kColT * RS];
+    __shared__ double mult[FIT ? 2 : 1][FIT ? kColT : 1][2]; // {1, s} per sample
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int per = (F.nchan + kColCh - 1) / kColCh + (FIT ? 1 : 0); // workgroups per frame
+    const long f = blockIdx.x / per;
+    const int g = (int)(blockIdx.x % per);
+    const long N = F.nsamp;
+    const double *sf = s + f * N; // read only when FIT
+
+    struct VM {
+        double v, m;
+    };
+    struct XM {
+        float x;
+        double m;
+    };
+    if (FIT && g == per - 1) {
+        // sum s (lane 0: fma(s, 1, a) is a + s) and sum s^2 (lane 1); the
+        // next 128 values are on their way while these are summed
+        if (tid >= 64) return;
+        double a = 0., n0 = sf[min((long)lane, N - 1)], n1 = sf[min(lane + 64L, N - 1)];
+        for (long t0 = 0; t0 < N; t0 += kColT) {
+            const int n = (int)min((long)kColT, N - t0);
+            mult[0][lane][0] = mult[0][lane + 64][0] = 1.;
+            mult[0][lane][1] = n0;
+            mult[0][lane + 64][1] = n1;
+            n0 = sf[min(t0 + kColT + lane, N - 1)];
+            n1 = sf[min(t0 + kColT + lane + 64, N - 1)];
+            __builtin_amdgcn_wave_barrier();
+            if (n == kColT)
+                chain16<kColT, VM>([&](int i) { return VM{mult[0][i][1], mult[0][i][lane & 1]}; },
+                                   [&](int, const VM &x) { a = fma(x.v, x.m, a); });
+            else
+                for (int i = 0; i < n; i++) a = fma(mult[0][i][1], mult[0][i][lane & 1], a);
+            __builtin_amdgcn_wave_barrier();
+        }
+        if (lane < 2) sess[2 * f + lane] = a;
+        return;
+    }
+
+    // the last group ends at the last channel (the channels it shares with
+    // the group before come out the same in both)
+    const int c0 = min(g * kColCh, F.nchan - kColCh);
+    const int h = tid - 64, q4 = (h & 7) * 4, r0 = h >> 3;
+    double acc = 0.;
+    const int sel = lane >> 5;
+    const int ls = FIT ? (lane & 31) : lane;
+    auto put = [&](int k, const ColChunk &c) {
+        float *b = buf[k & 1];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            float *d = b + (r0 + 32 * u) * RS + q4;
+            const f4u &v = c.v[u];
+            *(float4 *)d = make_float4(v[0], v[1], v[2], v[3]);
+            if (!FIT) // a float product, as data[]*data[] is
+                *(float4 *)(d + kColCh) = make_float4(v[0] * v[0], v[1] * v[1], v[2] * v[2], v[3] * v[3]);
+        }
+        if (FIT && h < kColT) {
+            mult[k & 1][h][0] = 1.;
+            mult[k & 1][h][1] = c.s;
+        }
+    };
+    auto chain = [&](int k) {
+        const float *b = buf[k & 1] + ls;
+        const int n = (int)min((long)kColT, N - (long)k * kColT);
+        if (n == kColT) {
+            if (FIT)
+                chain16<kColT, XM>([&](int i) { return XM{b[i * RS], mult[k & 1][FIT ? i : 0][sel]}; },
+                                   [&](int, const XM &x) { acc = fma((double)x.x, x.m, acc); });
+            else
+                chain16<kColT, float>([&](int i) { return b[i * RS]; }, [&](int, float x) { acc += (double)x; });
+        } else {
+            for (int i = 0; i < n; i++)
+                acc = FIT ? fma((double)b[i * RS], mult[k & 1][i][sel], acc) : acc + (double)b[i * RS];
+        }
+    };
+    stream_columns(F.x + f * F.fstride + c0, FIT ? sf : nullptr, N, F.tstride, put, chain);
+    if (tid >= 64) return;
+    double *out = stat + 2 * (f * F.nchan + c0);
+    if (FIT) {
+        out[2 * ls + sel] = acc;
+    } else {
+        const double other = __shfl_xor(acc, 32, 64);
+        const double m = acc / N;
+        double sd = other / N;
+        sd = fma(-m, m, sd); // tmpstd -= tmpmean*tmpmean
+        sd = sqrt(sd);
+        if (sd == 0.) sd = 1.;
+        if (lane < kColCh) {
+            out[2 * lane] = m;
+            out[2 * lane + 1] = sd;
+        }
+    }
+}
+
+// The time-major frame normalised in place with the channels' (mean, sd)
+// (candidate.cpp:853-859), and each sample's channel mean s, summed in
+// channel order (:858, 862-865).  A workgroup takes 32 samples and walks the
+// channels 128 at a time: four helper waves load, normalise, store and
+// leave the values in LDS, while wave 4 (lane = sample) adds the tile before
+// in channel order.  250 us for 856 MB at 4096 channels x 26,123 samples.
+constexpr int kNsT = 32, kNsC = 128;
+__global__ __launch_bounds__(320) void k_zdot_norm_s(Frames F, const double *__restrict__ stat, double *s)
+{
+    __shared__ float T[2][kNsC][kNsT + 1];
+    const long per = (F.nsamp + kNsT - 1) / kNsT;
+    const long f = blockIdx.x / per, t0 = (blockIdx.x % per) * kNsT;
+    const int nt = (int)min((long)kNsT, F.nsamp - t0);
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    float *blk = F.x + f * F.fstride + t0 * F.tstride;
+    const double *st = stat + 2 * f * F.nchan;
+    const int nk = (F.nchan + kNsC - 1) / kNsC;
+    double a = 0.;
+    // channels c0 + lane + 64*i, samples w + 4*u, and the channels' mean and sd
+    struct Tile {
+        float v[2][8];
+        double m[2], sd[2];
+    } A, B;
+    auto load = [&](int k, Tile &t) { // past the end: values that exist, unused
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const int c = min(k * kNsC + lane + 64 * i, F.nchan - 1);
+            t.m[i] = st[2 * c];
+            t.sd[i] = st[2 * c + 1];
+#pragma unroll
+            for (int u = 0; u < 8; u++) t.v[i][u] = blk[min(w + 4 * u, nt - 1) * F.tstride + c];
+        }
+    };
+    // the next tile's loads go out before this one's stores: a wait for
+    // loads then has no stores ahead of it
+    auto norm = [&](int k, const Tile &t, Tile &next) {
+        load(k + 1, next);
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const int cc = lane + 64 * i, c = k * kNsC + cc;
+#pragma unroll
+            for (int u = 0; u < 8; u++) {
+                float x = (float)((double)t.v[i][u] - t.m[i]);
+                x = (float)((double)x / t.sd[i]);
+                T[k & 1][cc][w + 4 * u] = x;
+                if (c < F.nchan && w + 4 * u < nt) blk[(w + 4 * u) * F.tstride + c] = x;
+            }
+        }
+    };
+    if (w < 4) load(0, A);
+    for (int k = 0; k <= nk; k++) {
+        if (w < 4) {
+            if (k < nk) {
+                if (k & 1)
+                    norm(k, B, A);
+                else
+                    norm(k, A, B);
+            }
+        } else if (k > 0 && lane < kNsT) {
+            const float(*Tk)[kNsT + 1] = T[(k - 1) & 1];
+            const int n = min(kNsC, F.nchan - (k - 1) * kNsC);
+            if (n == kNsC) {
+                chain16<kNsC, float>([&](int j) { return Tk[j][lane]; }, [&](int, float x) { a += (double)x; });
+            } else {
+                for (int j = 0; j < n; j++) a += Tk[j][lane];
+            }
+        }
+        __syncthreads();
+    }
+    if (w == 4 && lane < nt) s[f * F.nsamp + t0 + lane] = a / F.nchan;
+}
+
+// The time-major frame less each channel's fit alpha*s + beta
+// (candidate.cpp:881-896); fit[2*(f*nchan + j)] = (sum x, sum x*s).  One
+// thread per channel and 32 samples: one read and one write of the frame
+// (131 us for 856 MB).
+constexpr int kUpT = 32;
+__global__ __launch_bounds__(256) void k_zdot_update(Frames F, const double *__restrict__ s,
+                                                     const double *__restrict__ fit,
+                                                     const double *__restrict__ sess)
+{
+    const long nct = (F.nchan + 255) / 256, per = nct * ((F.nsamp + kUpT - 1) / kUpT);
+    const long f = blockIdx.x / per, r = blockIdx.x % per;
+    const int j = (int)(r % nct) * 256 + threadIdx.x;
+    const long t0 = r / nct * kUpT;
+    if (j >= F.nchan) return;
+    const int n = (int)min((long)kUpT, F.nsamp - t0);
+    float *col = F.x + f * F.fstride + t0 * F.tstride + j;
+    const double *sf = s + f * F.nsamp + t0;
+    const double xe = fit[2 * (f * F.nchan + j)], xs = fit[2 * (f * F.nchan + j) + 1];
+    const double se = sess[2 * f], ss = sess[2 * f + 1], nb = (double)F.nsamp;
+    const double tmp = fma(se, se, -(ss * nb));
+    double alpha = 0., beta = 0.;
+    if (tmp != 0) {
+        alpha = fma(xe, se, -(xs * nb)) / tmp;
+        beta = fma(xs, se, -(xe * ss)) / tmp;
+    }
+    if (n == kUpT) {
+        float v[kUpT];
+#pragma unroll
+        for (int u = 0; u < kUpT; u++) v[u] = col[u * F.tstride];
+#pragma unroll
+        for (int u = 0; u < kUpT; u++) col[u * F.tstride] = (float)((double)v[u] - fma(alpha, sf[u], beta));
+    } else {
+        for (int u = 0; u < n; u++) col[u * F.tstride] = (float)((double)col[u * F.tstride] - fma(alpha, sf[u], beta));
+    }
 }
 
 // kadaneF 1: the td x fd downsampled frame, each output summed in float
-// over k < fd (outer) and n < td (inner) (candidate.cpp:724-739)
+// over k < fd (outer) and n < td (inner) (candidate.cpp:724-739); ds element
+// (jd, id) of frame f is ds[f*ncd*nsd + jd*js + id*is]
 __global__ void k_kad_down(Frames F, int td, int fd, int ncd, long nsd, float *ds)
 {
     const long g = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -400,63 +578,151 @@ __global__ void k_kad_down(Frames F, int td, int fd, int ncd, long nsd, float *d
     ds[g] = a;
 }
 
-// The maximum-sum contiguous run of sg*a[0..n) (the XLibs kadane<float>;
-// declared: the running sum restarts after it drops below zero, strict '>'
-// keeps the earliest maximum); returns the sum.
-__device__ inline float kadane_run(const float *a, long n, float sg, long *start, long *end)
+// The same for time-major frames, into ds [f][id][jd]: a thread takes one
+// downsampled channel and 8 downsampled samples, so that a wavefront's reads
+// and writes are consecutive channels of one sample (127 us for 428 MB at
+// td 4, fd 2; 1.7 ms with a wavefront along time).
+constexpr int kKdT = 8;
+__global__ __launch_bounds__(256) void k_kad_down_tm(Frames F, int td, int fd, int ncd, long nsd,
+                                                     float *__restrict__ ds)
 {
-    float best = -INFINITY, cur = 0.f;
-    long s = 0, bs = 0, be = 0;
-    auto step = [&](long i, float v) {
-        cur += sg * v;
-        if (cur > best) {
-            best = cur;
-            bs = s;
-            be = i;
-        }
-        if (cur < 0.f) {
-            cur = 0.f;
-            s = i + 1;
-        }
-    };
-    long i = 0;
-    for (; i + 16 <= n; i += 16) { // 16 loads in flight
-        float v[16];
+    const long nct = (ncd + 255) / 256, per = nct * ((nsd + kKdT - 1) / kKdT);
+    const long f = blockIdx.x / per, r = blockIdx.x % per;
+    const int jd = (int)(r % nct) * 256 + threadIdx.x;
+    const long id0 = r / nct * kKdT;
+    if (jd >= ncd) return;
+    const float *x = F.x + f * F.fstride + (long)jd * fd;
+    float a[kKdT];
 #pragma unroll
-        for (int u = 0; u < 16; u++) v[u] = a[i + u];
+    for (int u = 0; u < kKdT; u++) a[u] = 0.f;
+    for (int k = 0; k < fd; k++)
+#pragma unroll 4
+        for (int n = 0; n < td; n++) {
+            float v[kKdT]; // samples past the end are clamped, unused
 #pragma unroll
-        for (int u = 0; u < 16; u++) step(i + u, v[u]);
-    }
-    for (; i < n; i++) step(i, a[i]);
-    *start = bs;
-    *end = be;
-    return best;
+            for (int u = 0; u < kKdT; u++) v[u] = x[(min(id0 + u, nsd - 1) * td + n) * F.tstride + k];
+#pragma unroll
+            for (int u = 0; u < kKdT; u++) a[u] += v[u];
+        }
+#pragma unroll
+    for (int u = 0; u < kKdT; u++)
+        if (id0 + u < nsd) ds[(f * nsd + id0 + u) * ncd + jd] = a[u];
 }
 
+// The maximum-sum contiguous run of the values stepped through it (the
+// XLibs kadane<float>; declared: the running sum restarts after it drops
+// below zero, strict '>' keeps the earliest maximum).  sg is 1, or -1 for the
+// strongest negative run (the product is exact, so the FMA is one add).
+struct Kadane {
+    float best = -INFINITY, cur = 0.f;
+    int s = 0, bs = 0, be = 0;
+    __device__ __forceinline__ void step(int i, float sg, float v)
+    {
+        cur = fmaf(sg, v, cur);
+        const bool up = cur > best;
+        best = up ? cur : best;
+        bs = up ? s : bs;
+        be = up ? i : be;
+        const bool low = cur < 0.f;
+        cur = low ? 0.f : cur;
+        s = low ? i + 1 : s;
+    }
+    // the zapped samples [z[0], z[1]): a run longer than wl whose
+    // S/N^2 = sum^2/(wn*td*fd) exceeds threshold^2, empty otherwise
+    // (candidate.cpp:752-827)
+    __device__ void zap(int td, int fd, int wl, float thre, long *z) const
+    {
+        const long wn = (long)be - bs + 1;
+        float snr2 = 0.f;
+        if (wn > wl) snr2 = best * best / ((float)wn * (float)(td * fd));
+        const bool hit = snr2 > thre * thre;
+        z[0] = hit ? (long)bs * td : 0;
+        z[1] = hit ? ((long)be + 1) * td : 0;
+    }
+};
+
 // kadaneF 2: per (frame, downsampled channel) the strongest positive and
-// negative runs; a run longer than wnlimit whose S/N^2 = sum^2/(wn*td*fd)
-// exceeds threshold^2 is zapped over its samples [start*td, (end+1)*td)
-// (candidate.cpp:752-827).  zap[4*g..]: positive then negative range, empty
-// when not zapped.
+// negative runs.  zap[4*g..]: positive then negative range, empty when not
+// zapped.  ds as k_kad_down leaves it.
 __global__ void k_kad_scan(int nframes, int ncd, long nsd, int td, int fd, float thre, const int *wnlimit,
                            const float *ds, long *zap)
 {
     const long g = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (g >= (long)nframes * ncd) return;
-    const long f = g / ncd;
     const float *ch = ds + g * nsd;
-    const int wl = wnlimit[f];
-    const float var = (float)(td * fd);
-    for (int p = 0; p < 2; p++) {
-        long s = 0, e = 0;
-        const float box = kadane_run(ch, nsd, p ? -1.f : 1.f, &s, &e);
-        const long wn = e - s + 1;
-        float snr2 = 0.f;
-        if (wn > wl) snr2 = box * box / ((float)wn * var);
-        const bool hit = snr2 > thre * thre;
-        zap[4 * g + 2 * p] = hit ? s * td : 0;
-        zap[4 * g + 2 * p + 1] = hit ? (e + 1) * td : 0;
+    Kadane p, m;
+    long i = 0;
+    for (; i + 16 <= nsd; i += 16) { // 16 loads in flight
+        float v[16];
+#pragma unroll
+        for (int u = 0; u < 16; u++) v[u] = ch[i + u];
+#pragma unroll
+        for (int u = 0; u < 16; u++) {
+            p.step((int)(i + u), 1.f, v[u]);
+            m.step((int)(i + u), -1.f, v[u]);
+        }
     }
+    for (; i < nsd; i++) {
+        p.step((int)i, 1.f, ch[i]);
+        m.step((int)i, -1.f, ch[i]);
+    }
+    const int wl = wnlimit[g / ncd];
+    p.zap(td, fd, wl, thre, zap + 4 * g);
+    m.zap(td, fd, wl, thre, zap + 4 * g + 2);
+}
+
+// The same over ds [f][id][jd] (k_kad_down_tm): 32 consecutive downsampled
+// channels per workgroup, their positive runs in the lower half of wave 0 and
+// their negative ones in the upper.  A run's scan is one chain over nsd
+// samples (6,530 for a search block at td = 4) of eight instructions each,
+// and only ncd/32 such waves exist, so helper waves stream the samples as
+// they do for the sums of zdot: 212 us for 2048 channels x 6,530 samples,
+// 78 cycles a sample (one thread per channel took 1.1 ms).
+__global__ __launch_bounds__(kColThreads) void k_kad_scan_tm(int ncd, long nsd, int td, int fd, float thre,
+                                                             const int *wnlimit, const float *__restrict__ ds,
+                                                             long *zap)
+{
+    __shared__ __attribute__((aligned(16))) float buf[2][kColT * kColCh];
+    const int per = (ncd + kColCh - 1) / kColCh, tid = threadIdx.x, lane = tid & 63;
+    const long f = blockIdx.x / per;
+    const int c0 = min((int)(blockIdx.x % per) * kColCh, ncd - kColCh);
+    const int h = tid - 64, q4 = (h & 7) * 4, r0 = h >> 3;
+    const float sg = lane < 32 ? 1.f : -1.f;
+    Kadane p;
+    auto put = [&](int k, const ColChunk &c) {
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+            *(float4 *)(buf[k & 1] + (r0 + 32 * u) * kColCh + q4) =
+                make_float4(c.v[u][0], c.v[u][1], c.v[u][2], c.v[u][3]);
+    };
+    auto chain = [&](int k) {
+        const float *b = buf[k & 1] + (lane & 31);
+        const int i0 = k * kColT, n = (int)min((long)kColT, nsd - i0);
+        if (n == kColT) {
+            constexpr int U = 16;
+            float x0[U], x1[U];
+            auto get = [&](float(&x)[U], int i) {
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int u = 0; u < U; u++) x[u] = b[(i + u) * kColCh];
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            get(x0, 0);
+#pragma unroll 1
+            for (int i = 0; i < kColT; i += 2 * U) {
+                get(x1, i + U);
+#pragma unroll
+                for (int u = 0; u < U; u++) p.step(i0 + i + u, sg, x0[u]);
+                get(x0, (i + 2 * U) & (kColT - 1)); // the last one reads sample 0 again, unused
+#pragma unroll
+                for (int u = 0; u < U; u++) p.step(i0 + i + U + u, sg, x1[u]);
+            }
+        } else {
+            for (int i = 0; i < n; i++) p.step(i0 + i, sg, b[i * kColCh]);
+        }
+    };
+    stream_columns(ds + f * nsd * ncd + c0, nullptr, nsd, ncd, put, chain);
+    if (tid < 64) p.zap(td, fd, wnlimit[f], thre, zap + 4 * (f * ncd + c0 + (lane & 31)) + (lane < 32 ? 0 : 2));
 }
 
 // kadaneF 3: zero the zapped runs of every channel of each downsampled
@@ -471,6 +737,23 @@ __global__ void k_kad_zero(Frames F, int fd, int ncd, const long *zap)
     const long *z = zap + 4 * (f * ncd + j / fd);
     for (int p = 0; p < 2; p++)
         for (long i = z[2 * p]; i < z[2 * p + 1]; i++) F.at(f, j, i) = 0.f;
+}
+
+// The same for time-major frames: one thread per channel and 64 samples, so
+// that a long run is written by many workgroups and a wavefront's stores are
+// consecutive channels.
+constexpr int kKzT = 64;
+__global__ __launch_bounds__(256) void k_kad_zero_tm(Frames F, int fd, int ncd, const long *zap)
+{
+    const int nch = ncd * fd;
+    const long nct = (nch + 255) / 256, per = nct * ((F.nsamp + kKzT - 1) / kKzT);
+    const long f = blockIdx.x / per, r = blockIdx.x % per;
+    const int j = (int)(r % nct) * 256 + threadIdx.x;
+    const long t0 = r / nct * kKzT, t1 = min(t0 + kKzT, F.nsamp);
+    if (j >= nch) return;
+    const long *z = zap + 4 * (f * ncd + j / fd);
+    for (int p = 0; p < 2; p++)
+        for (long i = max(t0, z[2 * p]); i < min(t1, z[2 * p + 1]); i++) F.at(f, j, i) = 0.f;
 }
 
 inline unsigned blocks_for(long n) { return (unsigned)((n + 255) / 256); }
@@ -489,7 +772,7 @@ int check_frames(const Frames &F)
 extern "C" size_t tx_rfi_work_bytes(int op, int nframes, int nchan, long nsamp, int td, int fd)
 {
     if (nframes < 0 || nchan < 1 || nsamp < 1) return 0;
-    if (op == TX_RFI_ZDOT) return (size_t)nframes * (nsamp + 2) * sizeof(double);
+    if (op == TX_RFI_ZDOT) return (size_t)nframes * (nsamp + 2 + 2 * (size_t)nchan) * sizeof(double);
     if (op == TX_RFI_KADANEF) {
         if (td < 1 || fd < 1) return 0;
         const size_t ncd = nchan / fd, nsd = nsamp / td;
@@ -509,7 +792,7 @@ extern "C" int tx_rfi_zdot(void *stream, float *data, int nframes, long fstride,
     if (!work || work_bytes < tx_rfi_work_bytes(TX_RFI_ZDOT, nframes, nchan, nsamp, 1, 1))
         return set_error(TX_EINVAL, "rfi: work buffer smaller than tx_rfi_work_bytes");
     hipStream_t st = (hipStream_t)stream;
-    double *s = (double *)work, *sess = s + (size_t)nframes * nsamp;
+    double *s = (double *)work, *sess = s + (size_t)nframes * nsamp, *stat = sess + 2 * (size_t)nframes;
     const long nfc = (long)nframes * nchan, nfs = (long)nframes * nsamp;
     const double *cs = s, *css = sess;
     if (tstride == 1 && fstride == (long)nchan * nsamp && cstride == nsamp) {
@@ -519,15 +802,17 @@ extern "C" int tx_rfi_zdot(void *stream, float *data, int nframes, long fstride,
         hipLaunchKernelGGL(k_zdot_s, dim3(blocks_for(nfs)), dim3(256), 0, st, F, s);
         hipLaunchKernelGGL(k_zdot_ss, dim3(blocks_for(nframes)), dim3(256), 0, st, F, cs, sess);
         hipLaunchKernelGGL(k_zdot_rows<true>, dim3(nb), dim3(256), 0, st, F, cs, css);
-    } else if (cstride == 1 && fstride == (long)nchan * nsamp && tstride == nchan) {
+    } else if (cstride == 1 && fstride == (long)nchan * nsamp && tstride == nchan && nchan >= kColCh) {
         // the DataBuffer layout [nframes][nsamp][nchan]
-        // one wavefront per workgroup: the few channel threads spread over
-        // as many CUs as there are wavefronts
-        const unsigned nw = (unsigned)((nfc + 63) / 64);
-        hipLaunchKernelGGL(k_zdot_cols<false>, dim3(nw), dim3(64), 0, st, F, cs, css);
-        hipLaunchKernelGGL(k_zdot_s_rows, dim3((unsigned)((nfs + 63) / 64)), dim3(64), 0, st, F, s);
-        hipLaunchKernelGGL(k_zdot_ss, dim3(blocks_for(nframes)), dim3(256), 0, st, F, cs, sess);
-        hipLaunchKernelGGL(k_zdot_cols<true>, dim3(nw), dim3(64), 0, st, F, cs, css);
+        const unsigned ng = (unsigned)((nchan + kColCh - 1) / kColCh);
+        hipLaunchKernelGGL(k_zdot_chain<false>, dim3(ng * nframes), dim3(kColThreads), 0, st, F, cs, stat, sess);
+        hipLaunchKernelGGL(k_zdot_norm_s, dim3((unsigned)((nsamp + kNsT - 1) / kNsT * nframes)), dim3(320), 0, st,
+                           F, (const double *)stat, s);
+        hipLaunchKernelGGL(k_zdot_chain<true>, dim3((ng + 1) * nframes), dim3(kColThreads), 0, st, F, cs, stat,
+                           sess);
+        hipLaunchKernelGGL(k_zdot_update,
+                           dim3((unsigned)(((nchan + 255) / 256) * ((nsamp + kUpT - 1) / kUpT) * nframes)), dim3(256),
+                           0, st, F, cs, (const double *)stat, css);
     } else {
         hipLaunchKernelGGL(k_zdot_norm, dim3(blocks_for(nfc)), dim3(256), 0, st, F);
         hipLaunchKernelGGL(k_zdot_s, dim3(blocks_for(nfs)), dim3(256), 0, st, F, s);
@@ -557,12 +842,23 @@ extern "C" int tx_rfi_kadanef(void *stream, float *data, int nframes, long fstri
     hipStream_t st = (hipStream_t)stream;
     float *ds = (float *)work;
     long *zap = (long *)((char *)work + ((size_t)nframes * ncd * nsd * sizeof(float) + 255) / 256 * 256);
-    hipLaunchKernelGGL(k_kad_down, dim3(blocks_for((long)nframes * ncd * nsd)), dim3(256), 0, st, F, td, fd,
-                       ncd, nsd, ds);
-    hipLaunchKernelGGL(k_kad_scan, dim3(blocks_for((long)nframes * ncd)), dim3(256), 0, st, nframes, ncd, nsd,
-                       td, fd, threshold, wnlimit, (const float *)ds, zap);
-    hipLaunchKernelGGL(k_kad_zero, dim3(blocks_for((long)nframes * ncd * fd)), dim3(256), 0, st, F, fd, ncd,
-                       (const long *)zap);
+    if (cstride == 1 && fstride == (long)nchan * nsamp && tstride == nchan && ncd >= kColCh) {
+        // the DataBuffer layout [nframes][nsamp][nchan]
+        const long nct = (ncd + 255) / 256, nzt = ((long)ncd * fd + 255) / 256;
+        hipLaunchKernelGGL(k_kad_down_tm, dim3((unsigned)(nct * ((nsd + kKdT - 1) / kKdT) * nframes)), dim3(256), 0,
+                           st, F, td, fd, ncd, nsd, ds);
+        hipLaunchKernelGGL(k_kad_scan_tm, dim3((unsigned)((ncd + kColCh - 1) / kColCh * nframes)), dim3(kColThreads), 0,
+                           st, ncd, nsd, td, fd, threshold, wnlimit, (const float *)ds, zap);
+        hipLaunchKernelGGL(k_kad_zero_tm, dim3((unsigned)(nzt * ((nsamp + kKzT - 1) / kKzT) * nframes)), dim3(256), 0,
+                           st, F, fd, ncd, (const long *)zap);
+    } else {
+        hipLaunchKernelGGL(k_kad_down, dim3(blocks_for((long)nframes * ncd * nsd)), dim3(256), 0, st, F, td, fd,
+                           ncd, nsd, ds);
+        hipLaunchKernelGGL(k_kad_scan, dim3(blocks_for((long)nframes * ncd)), dim3(256), 0, st, nframes, ncd, nsd,
+                           td, fd, threshold, wnlimit, (const float *)ds, zap);
+        hipLaunchKernelGGL(k_kad_zero, dim3(blocks_for((long)nframes * ncd * fd)), dim3(256), 0, st, F, fd, ncd,
+                           (const long *)zap);
+    }
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return set_error(TX_EHIP, std::string("rfi kadaneF: ") + hipGetErrorString(e));
     return TX_OK;
