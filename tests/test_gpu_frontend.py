@@ -245,3 +245,30 @@ def test_beam_rfi_chain_matches_oracle(td, fd, source):
             beam.build_graph(7.0)  # graph pipelines refuse a beam with filters
     finally:
         beam.close()
+
+
+# the 32-bit loads of td = fd = 1: multiples of 4 channels around the 64- and
+# 256-quad workgroups, lengths around the 8- and 512-sample tiles, and a block
+# off a 4-byte boundary, which takes the byte loads
+@pytest.mark.parametrize("ns,nch,shift", [(1, 4, 0), (8, 256, 0), (511, 260, 0), (513, 1028, 0), (1029, 12, 0),
+                                          (130, 64, 1), (130, 64, 2)])
+def test_frontend_word_loads(ns, nch, shift):
+    import torch
+
+    from transientx_amd import frontend
+
+    rng = np.random.default_rng(ns + nch)
+    x = rng.integers(0, 256, size=(ns, nch)).astype(np.uint8)
+    x[:, 1] = 255
+    say("case front end words ns", ns, "nch", nch, "shift", shift)
+    buf = torch.zeros(ns * nch + shift, dtype=torch.uint8, device="cuda")
+    g = buf[shift:].view(ns, nch)
+    g.copy_(torch.from_numpy(x))
+    off, gain = frontend.stats(g, 1, 1)
+    ro, rg = oracle.frontend_stats(x, 1, 1)
+    assert np.array_equal(off.cpu().numpy().view(np.uint32), ro.view(np.uint32))
+    assert np.array_equal(gain.cpu().numpy().view(np.uint32), rg.view(np.uint32))
+    for mask in (None, (rng.random(nch) > 0.2).astype(np.uint8)):
+        out = frontend.apply(g, 1, 1, off, gain, chan_mask=mask).cpu().numpy()
+        ref = oracle.frontend_u8(x, 1, 1, ro, rg, mask if mask is not None else np.ones(nch, np.uint8))
+        assert np.array_equal(out.view(np.uint32), ref.view(np.uint32))

