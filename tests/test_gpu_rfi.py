@@ -124,3 +124,22 @@ def test_time_major_zdot_and_kadanef_edges(nchan, nsamp, nf):
         t = torch.from_numpy(np.ascontiguousarray(y.transpose(0, 2, 1))).cuda()
         rfi.kadane_f(t, td, fd, 3.0, wl, layout="time")
         assert same_bits(np.ascontiguousarray(t.cpu().numpy().transpose(0, 2, 1)), r), (td, fd)
+
+
+# channel-major zdot around the tiles of rows in LDS: 32 rows to 600 samples,
+# fewer for longer rows, none past about 2,400 (the row kernels), and rows of no
+# whole 16-byte lines; few frames (a tile per workgroup) and many (a frame each)
+@pytest.mark.parametrize("nchan,nbin,nf", [(33, 31, 2), (32, 32, 130), (5, 1, 3), (70, 601, 1), (40, 605, 129),
+                                           (20, 1023, 2), (9, 2049, 1), (4, 2600, 1), (37, 65, 128)])
+def test_channel_major_zdot_tiles(nchan, nbin, nf):
+    import torch
+
+    from transientx_amd import rfi
+
+    say("case channel-major nchan", nchan, "nbin", nbin, "frames", nf)
+    x = frames(3 * nchan + nbin, nf, nchan, max(nbin, 8))[:, :, :nbin].copy()
+    x[nf - 1, 3, nbin // 2] = np.nan if nchan % 2 else np.inf
+    ref = np.stack([oracle.zdot(x[f]) for f in range(nf)])
+    g = torch.from_numpy(x).cuda()
+    rfi.zdot(g, layout="channel")
+    assert same_bits(g.cpu().numpy(), ref)

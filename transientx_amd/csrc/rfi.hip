@@ -23,12 +23,15 @@
 #include <string>
 
 #include "../../include/txgpu.h"
+#include "device_util.h"
 
 #pragma clang fp contract(off)
 
 namespace txgpu {
 int set_error(int code, const std::string &msg);
 }
+using txgpu::lds_fill;
+using txgpu::lds_fill16;
 using txgpu::set_error;
 
 namespace {
@@ -261,21 +264,6 @@ __global__ __launch_bounds__(256) void k_zdot_rows(Frames F, const double *s, co
     (void)j;
 }
 
-// ---- Time-major frames (cstride 1), the DataBuffer layout.  A channel's sums
-// run over all its samples one after the other, so a search block (26,123
-// samples of 4096 channels) is 4096 chains of 26,123 dependent FP64 adds and
-// nothing shorter; what can be chosen is what a step of the chain costs.  On
-// gfx950 a dependent FP64 add or FMA issues every 4.5 cycles and a
-// conversion every 5.5 (measured), so the chains get a wave of their own
-// (wave 0 of the workgroup, which only reads LDS, converts and adds) and
-// four helper waves bring the samples: 32 channels (one 128-byte line of a
-// sample) per workgroup, so that 4096 channels use 128 CUs, and both of a
-// channel's sums in the same wave (lane l and lane l + 32).  The helpers keep
-// two chunks of kColT samples in registers on their way from HBM while a
-// third is written to LDS and a fourth is summed.
-constexpr int kColCh = 32, kColT = 128, kColThreads = 64 + 256;
-typedef float f4u __attribute__((ext_vector_type(4), aligned(4))); // 4-byte aligned 16-byte access
-
 // n steps of a chain, 16 at a time: get(i) reads the operands of 16 steps while
 // the 16 before them run (the scheduling barriers keep the reads ahead).
 template <int n, class T, class Get, class Step>
@@ -299,6 +287,318 @@ __device__ __forceinline__ void chain16(Get get, Step step)
         for (int u = 0; u < 16; u++) step(i + 16 + u, x1[u]);
     }
 }
+
+// ---- Channel-major frames whose rows fit LDS: one read of the frame for the
+// statistics and the channel mean, one read and one write for the fit.  A
+// workgroup keeps RB rows (32 at 512 samples, two workgroups per CU) in LDS;
+// one wave runs the rows' chains, lanes r and RB + r the two sums of row r
+// over the same 16-byte LDS reads (the row pitch is an odd multiple of 4
+// floats, so 16 lanes' reads cover the 64 banks), and all the waves
+// normalise and update along time.  Eight waves, since a tile's phases follow
+// one another and only the other workgroup's fill the gaps (four waves: 1.28
+// and 1.07 ms where eight take 1.10 and 0.86; 16-row tiles, four workgroups
+// a CU: 1.33 and 1.32; the next tile loaded into registers ahead: no
+// faster).  1024 frames of 1024 x 512 samples (2.1 GB): statistics and mean
+// 0.86 ms, fit 1.10 ms (3.9 TB/s); tiles of 64 samples per pass took 3.0 and
+// 2.5.
+constexpr int kTileThreads = 512, kTileWaves = kTileThreads / 64;
+struct RowTile {
+    int RB, st; // rows per tile, row pitch in LDS (floats)
+};
+__host__ __device__ inline int row_pitch(long nsamp) { return (int)(((nsamp + 3) / 4) | 1) * 4; }
+// LDS of a tile: the rows, 16 bytes per sample (the fit's {1, s}; the
+// statistics kernel needs half of it) and 32 per row
+inline size_t tile_lds(int RB, long nsamp)
+{
+    return (size_t)RB * row_pitch(nsamp) * 4 + (size_t)nsamp * 16 + (size_t)RB * 32;
+}
+constexpr size_t kTileLds = 80 * 1024; // two workgroups per CU
+inline RowTile row_tile(long nsamp)
+{
+    for (int RB = 32; RB >= 8; RB >>= 1)
+        if (nsamp <= 16384 && tile_lds(RB, nsamp) <= kTileLds) return {RB, row_pitch(nsamp)};
+    return {0, 0};
+}
+
+// Rows j0 .. j0 + nr of frame f into LDS.  Whole 16-byte lines: up to 3
+// floats past a row's end are read from the next row, never past the frames.
+__device__ __forceinline__ void tile_load(const Frames &F, long f, int j0, int nr, const RowTile &R, float *T)
+{
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int n = (int)F.nsamp;
+    for (int r = w; r < nr; r += kTileWaves) {
+        const long g = f * F.nchan + j0 + r;
+        const uint32_t *src = (const uint32_t *)(F.x + g * n);
+        if ((n & 3) && g + 1 == (long)F.nframes * F.nchan)
+            lds_fill(src, (uint32_t *)(T + r * R.st), n, 0, 1, lane);
+        else
+            lds_fill16(src, (uint32_t *)(T + r * R.st), n, 0, 1, lane);
+    }
+}
+
+// The wave that runs a tile's chains: another one for each of the workgroups
+// that a CU is given in turn (every 256th), so that co-resident workgroups'
+// chains sit on different SIMDs.
+__device__ __forceinline__ int chain_wave() { return (int)(blockIdx.x >> 8) & 3; }
+
+// step(i, x) over the n samples of an LDS row in order, 16-byte reads 16
+// samples ahead.
+template <class Step>
+__device__ __forceinline__ void row_chain(const float *row, int n, Step step)
+{
+    const float4 *p = (const float4 *)row;
+    float4 x0[4], x1[4];
+    auto get = [&](float4(&x)[4], int q) {
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < 4; u++) x[u] = p[q + u];
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto run = [&](const float4(&x)[4], int i) {
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            step(i + 4 * u, x[u].x);
+            step(i + 4 * u + 1, x[u].y);
+            step(i + 4 * u + 2, x[u].z);
+            step(i + 4 * u + 3, x[u].w);
+        }
+    };
+    int i = 0;
+    if (n >= 32) {
+        get(x0, 0);
+#pragma unroll 1
+        for (; i + 32 <= n; i += 32) {
+            get(x1, i / 4 + 4);
+            run(x0, i);
+            get(x0, i + 64 <= n ? i / 4 + 8 : 0); // the last one reads the row's start, unused
+            run(x1, i + 16);
+        }
+    }
+    for (; i < n; i++) step(i, row[i]);
+}
+
+// zdot's normalisation (candidate.cpp:853-859)
+__device__ __forceinline__ float zdot_norm(float v, double m, double sd)
+{
+    v = (float)((double)v - m);
+    return (float)((double)v / sd);
+}
+
+// The same for U values v[u] of channels with (m, sd, 1/sd) = ch(u), by one
+// FP64 product each where that must give the same float, else by the
+// division (an FP64 division is a dozen instructions, the product and its
+// check five).  The product d*(1/sd) is within 2^-52 of d/sd, so it and the
+// rounded quotient are at most 3 units of the last of 53 bits apart, and they
+// round to the same float unless a boundary between floats lies within 3
+// units: for normal floats that is a low part (29 bits) of 0x10000000, kept
+// away from by 4 units.  Values whose magnitude is below 2^-126, infinite or
+// NaN are divided, and sd outside [2^-400, 2^400] has NaN as its reciprocal.
+__device__ __forceinline__ double zdot_rcp(double sd)
+{
+    return sd >= 0x1p-400 && sd <= 0x1p400 ? 1. / sd : (double)NAN;
+}
+template <int U, class Ch>
+__device__ __forceinline__ void zdot_norms(float (&v)[U], Ch ch)
+{
+    unsigned low = ~0u, mag = 0u; // the low part above the boundary's 4 units, the magnitude above 2^-126
+    float x[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+        const auto c = ch(u);
+        const double q = (double)(float)((double)v[u] - c.m) * c.r;
+        const unsigned long long b = (unsigned long long)__double_as_longlong(q);
+        low = min(low, ((unsigned)b << 3) + (0u - (0x0FFFFFFCu << 3)));
+        mag = max(mag, ((unsigned)(b >> 32) << 1) + (0u - 2u * 0x38100000u));
+        x[u] = (float)q;
+    }
+    if (low <= 8u << 3 || mag >= 2u * (0x7FF00000u - 0x38100000u)) {
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const auto c = ch(u);
+            x[u] = zdot_norm(v[u], c.m, c.sd);
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++) v[u] = x[u];
+}
+struct ChanStat {
+    double m, sd, r;
+};
+
+// Mean and standard deviation of each channel (candidate.cpp:837-851) into
+// stat[2*(f*nchan + j)].  MEAN: one workgroup per frame, which walks the
+// channels in order and so also forms the channel mean s of the normalised
+// samples (:858, 862-865) and the sums of s and s^2 (:879-880) from the same
+// read; without MEAN one workgroup per tile of rows.
+template <bool MEAN>
+__global__ __launch_bounds__(kTileThreads) void k_zdot_tile_stats(Frames F, RowTile R, double *stat, double *s, double *sess)
+{
+    extern __shared__ __attribute__((aligned(16))) float T[]; // [RB][st]
+    const int n = (int)F.nsamp, tid = threadIdx.x, lane = tid & 63, RB = R.RB;
+    double *sacc = (double *)(T + RB * R.st); // [n]
+    ChanStat *ms = (ChanStat *)(sacc + n);    // [RB]
+    const int ntile = (F.nchan + RB - 1) / RB;
+    const long f = MEAN ? blockIdx.x : blockIdx.x / ntile;
+    for (int jt = MEAN ? 0 : (int)(blockIdx.x % ntile); jt < ntile; jt++) {
+        const int j0 = jt * RB, nr = min(RB, F.nchan - j0);
+        __syncthreads(); // the tile before has been used
+        tile_load(F, f, j0, nr, R, T);
+        txgpu::lds_fill_done();
+        if (tid >> 6 == chain_wave()) {
+            const bool sq = lane >= RB && lane < 2 * RB; // the lane of sum x^2
+            double a = 0.;
+            row_chain(T + (lane & (RB - 1)) * R.st, n, [&](int, float x) {
+                a += (double)(x * (sq ? x : 1.f)); // a float product, as data[]*data[] is
+            });
+            const double b = __shfl(a, (lane + RB) & 63, 64);
+            const double m = a / F.nsamp;
+            double sd = b / F.nsamp;
+            sd = fma(-m, m, sd); // tmpstd -= tmpmean*tmpmean
+            sd = sqrt(sd);
+            if (sd == 0.) sd = 1.;
+            if (lane < nr) {
+                ms[lane] = {m, sd, zdot_rcp(sd)};
+                stat[2 * (f * F.nchan + j0 + lane)] = m;
+                stat[2 * (f * F.nchan + j0 + lane) + 1] = sd;
+            }
+        }
+        if (!MEAN) return;
+        __syncthreads();
+        for (int t = tid; t < n; t += kTileThreads) {
+            double a = jt ? sacc[t] : 0.;
+            int r = 0;
+            for (; r + 8 <= nr; r += 8) {
+                float v[8];
+#pragma unroll
+                for (int u = 0; u < 8; u++) v[u] = T[(r + u) * R.st + t];
+                zdot_norms(v, [&](int u) { return ms[r + u]; });
+#pragma unroll
+                for (int u = 0; u < 8; u++) a += (double)v[u];
+            }
+            for (; r < nr; r++) a += (double)zdot_norm(T[r * R.st + t], ms[r].m, ms[r].sd);
+            sacc[t] = a;
+        }
+    }
+    if (!MEAN) return;
+    for (int t = tid; t < n; t += kTileThreads) { // each thread its own samples
+        const double a = sacc[t] / F.nchan;
+        sacc[t] = a;
+        s[f * F.nsamp + t] = a;
+    }
+    __syncthreads();
+    if (tid < 2) { // sum s (lane 0: fma(s, 1, a) is a + s) and sum s^2 (lane 1)
+        double a = 0.;
+        int i = 0;
+        for (; i + 16 <= n; i += 16) {
+            double v[16];
+#pragma unroll
+            for (int u = 0; u < 16; u++) v[u] = sacc[i + u];
+#pragma unroll
+            for (int u = 0; u < 16; u++) a = fma(v[u], tid ? v[u] : 1., a);
+        }
+        for (; i < n; i++) a = fma(sacc[i], tid ? sacc[i] : 1., a);
+        sess[2 * f + tid] = a;
+    }
+}
+
+// The channel mean from the raw frame and the channels' statistics, one lane
+// per sample: for batches of too few frames to give every CU one.
+__global__ __launch_bounds__(64) void k_zdot_norm_mean(Frames F, const double *__restrict__ stat, double *s)
+{
+    const int per = (int)((F.nsamp + 63) / 64);
+    const long f = blockIdx.x / per, t = (long)(blockIdx.x % per) * 64 + threadIdx.x;
+    const float *x = F.x + f * F.fstride + min(t, F.nsamp - 1);
+    const double *st = stat + 2 * f * F.nchan;
+    double a = 0.;
+    int j = 0;
+    for (; j + 8 <= F.nchan; j += 8) {
+        float v[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) v[u] = x[(long)(j + u) * F.nsamp];
+#pragma unroll
+        for (int u = 0; u < 8; u++) a += (double)zdot_norm(v[u], st[2 * (j + u)], st[2 * (j + u) + 1]);
+    }
+    for (; j < F.nchan; j++) a += (double)zdot_norm(x[(long)j * F.nsamp], st[2 * j], st[2 * j + 1]);
+    if (t < F.nsamp) s[f * F.nsamp + t] = a / F.nchan;
+}
+
+// The rows of a tile normalised in LDS, their least-squares fit to s, and
+// the frame less that fit (candidate.cpp:870-896).
+__global__ __launch_bounds__(kTileThreads) void k_zdot_tile_fit(Frames F, RowTile R, const double *__restrict__ stat,
+                                                       const double *__restrict__ s, const double *__restrict__ sess)
+{
+    extern __shared__ __attribute__((aligned(16))) float T[]; // [RB][st]
+    const int n = (int)F.nsamp, tid = threadIdx.x, lane = tid & 63, w = tid >> 6, RB = R.RB;
+    double(*mult)[2] = (double(*)[2])(T + RB * R.st); // [n] {1, s}
+    double *ms = &mult[n][0];                         // [RB][2]
+    double *ab = ms + 2 * RB;                         // [RB][2]
+    const int ntile = (F.nchan + RB - 1) / RB;
+    const long f = blockIdx.x / ntile;
+    const int j0 = (int)(blockIdx.x % ntile) * RB, nr = min(RB, F.nchan - j0);
+    tile_load(F, f, j0, nr, R, T);
+    for (int t = tid; t < n; t += kTileThreads) {
+        mult[t][0] = 1.;
+        mult[t][1] = s[f * F.nsamp + t];
+    }
+    if (tid < 2 * nr) ms[tid] = stat[2 * (f * F.nchan + j0) + tid];
+    txgpu::lds_fill_done();
+    for (int r = w; r < nr; r += kTileWaves) {
+        const double m = ms[2 * r], sd = ms[2 * r + 1];
+        const ChanStat c{m, sd, zdot_rcp(sd)};
+        float *row = T + r * R.st;
+        int t = lane;
+        for (; t - lane + 256 <= n; t += 256) {
+            float v[4];
+#pragma unroll
+            for (int u = 0; u < 4; u++) v[u] = row[t + 64 * u];
+            zdot_norms(v, [&](int) { return c; });
+#pragma unroll
+            for (int u = 0; u < 4; u++) row[t + 64 * u] = v[u];
+        }
+        for (; t < n; t += 64) row[t] = zdot_norm(row[t], m, sd);
+    }
+    __syncthreads();
+    if (w == chain_wave()) {
+        const int sel = lane >= RB && lane < 2 * RB; // the lane of sum x*s
+        double a = 0.;
+        row_chain(T + (lane & (RB - 1)) * R.st, n, [&](int i, float x) { a = fma((double)x, mult[i][sel], a); });
+        const double b = __shfl(a, (lane + RB) & 63, 64);
+        const double se = sess[2 * f], ss = sess[2 * f + 1], nb = (double)F.nsamp;
+        const double tmp = fma(se, se, -(ss * nb));
+        double alpha = 0., beta = 0.;
+        if (tmp != 0) {
+            alpha = fma(a, se, -(b * nb)) / tmp;
+            beta = fma(b, se, -(a * ss)) / tmp;
+        }
+        if (lane < nr) {
+            ab[2 * lane] = alpha;
+            ab[2 * lane + 1] = beta;
+        }
+    }
+    __syncthreads();
+    for (int r = w; r < nr; r += kTileWaves) {
+        const double alpha = ab[2 * r], beta = ab[2 * r + 1];
+        const float *row = T + r * R.st;
+        float *out = F.x + (f * F.nchan + j0 + r) * F.nsamp;
+#pragma unroll 4
+        for (int t = lane; t < n; t += 64) out[t] = (float)((double)row[t] - fma(alpha, mult[t][1], beta));
+    }
+}
+
+// ---- Time-major frames (cstride 1), the DataBuffer layout.  A channel's sums
+// run over all its samples one after the other, so a search block (26,123
+// samples of 4096 channels) is 4096 chains of 26,123 dependent FP64 adds and
+// nothing shorter; what can be chosen is what a step of the chain costs.  On
+// gfx950 a dependent FP64 add or FMA issues every 4.5 cycles and a
+// conversion every 5.5 (measured), so the chains get a wave of their own
+// (wave 0 of the workgroup, which only reads LDS, converts and adds) and
+// four helper waves bring the samples: 32 channels (one 128-byte line of a
+// sample) per workgroup, so that 4096 channels use 128 CUs, and both of a
+// channel's sums in the same wave (lane l and lane l + 32).  The helpers keep
+// two chunks of kColT samples in registers on their way from HBM while a
+// third is written to LDS and a fourth is summed.
+constexpr int kColCh = 32, kColT = 128, kColThreads = 64 + 256;
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4))); // 4-byte aligned 16-byte access
 
 // The streaming part: chunks of kColT samples of 32 columns (ts floats from
 // sample to sample, N samples) pass through buf; put(k, v) of a helper
@@ -490,15 +790,16 @@ __global__ __launch_bounds__(320) void k_zdot_norm_s(Frames F, const double *__r
     };
     // the next tile's loads go out before this one's stores: a wait for
     // loads then has no stores ahead of it
-    auto norm = [&](int k, const Tile &t, Tile &next) {
+    auto norm = [&](int k, Tile &t, Tile &next) {
         load(k + 1, next);
 #pragma unroll
         for (int i = 0; i < 2; i++) {
             const int cc = lane + 64 * i, c = k * kNsC + cc;
+            const ChanStat cs{t.m[i], t.sd[i], zdot_rcp(t.sd[i])};
+            zdot_norms(t.v[i], [&](int) { return cs; });
 #pragma unroll
             for (int u = 0; u < 8; u++) {
-                float x = (float)((double)t.v[i][u] - t.m[i]);
-                x = (float)((double)x / t.sd[i]);
+                const float x = t.v[i][u];
                 T[k & 1][cc][w + 4 * u] = x;
                 if (c < F.nchan && w + 4 * u < nt) blk[(w + 4 * u) * F.tstride + c] = x;
             }
@@ -725,6 +1026,75 @@ __global__ __launch_bounds__(kColThreads) void k_kad_scan_tm(int ncd, long nsd, 
     if (tid < 64) p.zap(td, fd, wnlimit[f], thre, zap + 4 * (f * ncd + c0 + (lane & 31)) + (lane < 32 ? 0 : 2));
 }
 
+// kadaneF of channel-major frames in one pass: a workgroup takes 64
+// downsampled channels (fd rows each), reads their samples once (lane = a
+// downsampled sample), keeps the downsampled rows in LDS, scans them (wave 0
+// the positive runs, wave 1 the negative ones, a lane per row) and zeroes
+// what is zapped.  Reading the frames is all that is left: 0.49 ms for 2.1 GB
+// (1024 frames of 1024 x 512, td 4, fd 2), 0.82 ms with the downsampled
+// frames in memory and a kernel per step.
+constexpr size_t kKrLds = 40 * 1024; // four workgroups per CU
+inline int kad_rows(long nsd) // rows per workgroup, 0: a row does not fit
+{
+    for (int G = 64; G >= 4; G >>= 1)
+        if (nsd <= 65536 && (size_t)G * (nsd | 1) * 4 <= kKrLds) return G;
+    return 0;
+}
+__global__ __launch_bounds__(256) void k_kad_rows(Frames F, int td, int fd, int ncd, int nsd, int G, float thre,
+                                                  const int *__restrict__ wnlimit)
+{
+    extern __shared__ float ds[]; // [G][pitch], pitch odd
+    __shared__ long z[64][4];
+    const int pitch = nsd | 1, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int per = (ncd + G - 1) / G;
+    const long f = blockIdx.x / per;
+    const int g0 = (int)(blockIdx.x % per) * G, ng = min(G, ncd - g0);
+    const float *x = F.x + f * F.fstride + (long)g0 * fd * F.nsamp;
+    // each output in float over k < fd (outer) and n < td (inner) (candidate.cpp:724-739)
+    auto down = [&](int r, int id) {
+        const float *q = x + (long)r * fd * F.nsamp + (long)id * td;
+        float a = 0.f;
+        for (int k = 0; k < fd; k++)
+            for (int n = 0; n < td; n++) a += q[k * F.nsamp + n];
+        return a;
+    };
+    if (td == 4 && F.nsamp % 4 == 0 && ((uintptr_t)F.x & 15) == 0) {
+        for (int r = w; r < ng; r += 4)
+            for (int id = lane; id < nsd; id += 64) {
+                const float4 *q = (const float4 *)(x + (long)r * fd * F.nsamp) + id;
+                float a = 0.f;
+#pragma unroll 4
+                for (int k = 0; k < fd; k++) {
+                    const float4 v = q[k * (F.nsamp / 4)];
+                    a += v.x;
+                    a += v.y;
+                    a += v.z;
+                    a += v.w;
+                }
+                ds[r * pitch + id] = a;
+            }
+    } else {
+        for (int r = w; r < ng; r += 4)
+            for (int id = lane; id < nsd; id += 64) ds[r * pitch + id] = down(r, id);
+    }
+    __syncthreads();
+    if (w < 2 && lane < ng) {
+        const float sg = w ? -1.f : 1.f;
+        const float *row = ds + lane * pitch;
+        Kadane p;
+#pragma unroll 8
+        for (int i = 0; i < nsd; i++) p.step(i, sg, row[i]);
+        p.zap(td, fd, wnlimit[f], thre, &z[lane][2 * w]);
+    }
+    __syncthreads();
+    for (int c = w; c < ng * fd; c += 4) {
+        const long *q = z[c / fd];
+        float *row = F.x + f * F.fstride + ((long)g0 * fd + c) * F.nsamp;
+        for (int p = 0; p < 2; p++)
+            for (long i = q[2 * p] + lane; i < q[2 * p + 1]; i += 64) row[i] = 0.f;
+    }
+}
+
 // kadaneF 3: zero the zapped runs of every channel of each downsampled
 // channel (channels past ncd*fd are left as they are); one thread per
 // channel, which writes only its zapped samples (zaps are rare)
@@ -797,11 +1167,34 @@ extern "C" int tx_rfi_zdot(void *stream, float *data, int nframes, long fstride,
     const double *cs = s, *css = sess;
     if (tstride == 1 && fstride == (long)nchan * nsamp && cstride == nsamp) {
         // the Candidate layout [nframes][nchan][nsamp]
-        const unsigned nb = (unsigned)((nfc + 255) / 256);
-        hipLaunchKernelGGL(k_zdot_rows<false>, dim3(nb), dim3(256), 0, st, F, cs, css);
-        hipLaunchKernelGGL(k_zdot_s, dim3(blocks_for(nfs)), dim3(256), 0, st, F, s);
-        hipLaunchKernelGGL(k_zdot_ss, dim3(blocks_for(nframes)), dim3(256), 0, st, F, cs, sess);
-        hipLaunchKernelGGL(k_zdot_rows<true>, dim3(nb), dim3(256), 0, st, F, cs, css);
+        const RowTile R = row_tile(nsamp);
+        if (R.RB) {
+            const size_t shm = tile_lds(R.RB, nsamp);
+            const unsigned nt = (unsigned)((nchan + R.RB - 1) / R.RB) * nframes;
+            auto fit = k_zdot_tile_fit;
+            (void)hipFuncSetAttribute((const void *)fit, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kTileLds);
+            // a frame per workgroup reads the frames once less; with fewer
+            // frames than fill the CUs, a tile per workgroup is the faster
+            if (nframes >= 128) {
+                auto k = k_zdot_tile_stats<true>;
+                (void)hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kTileLds);
+                hipLaunchKernelGGL(k, dim3((unsigned)nframes), dim3(kTileThreads), shm, st, F, R, stat, s, sess);
+            } else {
+                auto k = k_zdot_tile_stats<false>;
+                (void)hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kTileLds);
+                hipLaunchKernelGGL(k, dim3(nt), dim3(kTileThreads), shm, st, F, R, stat, s, sess);
+                hipLaunchKernelGGL(k_zdot_norm_mean, dim3((unsigned)((nsamp + 63) / 64 * nframes)), dim3(64), 0, st,
+                                   F, (const double *)stat, s);
+                hipLaunchKernelGGL(k_zdot_ss, dim3(blocks_for(nframes)), dim3(256), 0, st, F, cs, sess);
+            }
+            hipLaunchKernelGGL(fit, dim3(nt), dim3(kTileThreads), shm, st, F, R, (const double *)stat, cs, css);
+        } else {
+            const unsigned nb = (unsigned)((nfc + 255) / 256);
+            hipLaunchKernelGGL(k_zdot_rows<false>, dim3(nb), dim3(256), 0, st, F, cs, css);
+            hipLaunchKernelGGL(k_zdot_s, dim3(blocks_for(nfs)), dim3(256), 0, st, F, s);
+            hipLaunchKernelGGL(k_zdot_ss, dim3(blocks_for(nframes)), dim3(256), 0, st, F, cs, sess);
+            hipLaunchKernelGGL(k_zdot_rows<true>, dim3(nb), dim3(256), 0, st, F, cs, css);
+        }
     } else if (cstride == 1 && fstride == (long)nchan * nsamp && tstride == nchan && nchan >= kColCh) {
         // the DataBuffer layout [nframes][nsamp][nchan]
         const unsigned ng = (unsigned)((nchan + kColCh - 1) / kColCh);
@@ -851,6 +1244,10 @@ extern "C" int tx_rfi_kadanef(void *stream, float *data, int nframes, long fstri
                            st, ncd, nsd, td, fd, threshold, wnlimit, (const float *)ds, zap);
         hipLaunchKernelGGL(k_kad_zero_tm, dim3((unsigned)(nzt * ((nsamp + kKzT - 1) / kKzT) * nframes)), dim3(256), 0,
                            st, F, fd, ncd, (const long *)zap);
+    } else if (const int G = tstride == 1 && fstride == (long)nchan * nsamp && cstride == nsamp ? kad_rows(nsd) : 0) {
+        // the Candidate layout [nframes][nchan][nsamp]
+        hipLaunchKernelGGL(k_kad_rows, dim3((unsigned)((ncd + G - 1) / G * nframes)), dim3(256),
+                           (size_t)G * (nsd | 1) * 4, st, F, td, fd, ncd, (int)nsd, G, threshold, wnlimit);
     } else {
         hipLaunchKernelGGL(k_kad_down, dim3(blocks_for((long)nframes * ncd * nsd)), dim3(256), 0, st, F, td, fd,
                            ncd, nsd, ds);
