@@ -630,3 +630,38 @@ def test_htr_4096ch_16us_four_rows_first_ready_block():
         dm_peak = rows[r][0] + i * rows[r][1]
         say("row", r, "points", pts.size, "peak DM", dm_peak, "S", float(S[i, t]))
         assert abs(dm_peak - burst_dm[r]) <= 3 * rows[r][1] + 0.02 * burst_dm[r], r
+
+
+@pytest.mark.parametrize("dtype", ["u8", "f32"])
+@pytest.mark.parametrize("shape", range(1, 7))
+def test_stage2_passes_of_many_and_few_rows(shape, dtype):
+    """Stage 2 fills a pass's packed rows as one run of 1 KB chunks: passes of
+    the 64 rows that fit a wavefront's lanes and of the few that fit 16 KB,
+    a group that leaves waves and DM slots empty, rows and tiles of no whole
+    16-byte line."""
+    ndump, nblocks = 517, 4
+    obs = Observation(nchans=96, fbot=1200, ftop=1500, tsamp=1e-3, nsamp=ndump * nblocks, sd=10, seed=shape,
+                      pulses=[Pulse(dm=37.0, t0=0.9, fwhm=6e-3, snr=30)])
+    x = generate(obs)
+    vwn = width_ladder(1e-3, 1e-3, 0.05, 0.1)
+    kw = dict(freqs=obs.freqs, tsamp=obs.tsamp, dms=0.0, ddm=1.5, ndm=61, vwn=vwn, overlap=0.25, nsub=96, group=27)
+    op = oracle_plan(obs, ndump, kw)
+    xo = x.astype(np.float32) - 128
+    if dtype == "f32":
+        xo = (xo * np.float32(0.37)).astype(np.float32)
+    for lds in (163840, 20480):
+        say("stage-2 shape", shape, "LDS", lds, dtype)
+        seen = []
+
+        def check(b, plan, ready):
+            assert np.array_equal(all_tim(plan), op.dedisperse(xo, op.window_start(b))), f"block {b}"
+            seen.append(b)
+            return ready
+
+        try:
+            stream(x if dtype == "u8" else xo, 96, ndump, nblocks, dict(kw, shapes={"s2_shape": shape, "s2_lds": lds}),
+                   beam_kw=dict(dtype=dtype), check=check)
+        except Exception as e:  # a tile of 2048 samples does not fit 20 KB
+            assert "does not fit" in str(e) and lds == 20480, e
+            continue
+        assert len(seen) == nblocks

@@ -93,11 +93,11 @@ struct Stage2Args {
     long spitch, Lsub;
     const int *d2;    // [ndm][nsub]
     const int *d2min;  // [ngroups*nblk][nsub] lowest delay of each DM block
-    const int *d2span; // [ngroups*nblk][nsub] highest minus lowest delay of each DM block
-    const int *d2off;  // [ngroups*nblk][nsub][8 waves][DPW] delay - d2min of each DM slot
+    const int *d2off;  // [ngroups*nblk][nsub][8 waves][DPW] LDS offset (floats) of each DM slot's first sample
     const int *ldsoff; // [ngroups*nblk][nsub] LDS offset (floats) of each sub-band row in its pass
     const int *npass;  // [ngroups*nblk] passes of each DM block
     const int *pstart; // [ngroups*nblk][pstride] first sub-band of each pass (+ end)
+    const int *pused;  // [ngroups*nblk][pstride] floats of each pass's rows
     int pstride;
     int half;          // floats per LDS buffer (two buffers)
     int nsub;
@@ -112,7 +112,8 @@ struct Stage2Args {
     const long *clock; // graph pipelines: w0 = *clock + ndump - maxdelay - N
     long ndump, maxdelay;
 };
-// Workgroups of 8 waves; DPW fine DMs per wave, R samples per lane.
+// Workgroups of kS2Waves waves; DPW fine DMs per wave, R samples per lane.
+constexpr int kS2Waves = 8;
 extern const int kStage2Shapes[][2];
 extern const int kNumStage2Shapes;
 int launch_stage2(hipStream_t st, const Stage2Args &a, int DPW, int R, LaunchSink *sink = nullptr);

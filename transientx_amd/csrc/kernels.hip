@@ -784,58 +784,79 @@ int launch_stage1_fe(hipStream_t st, const Stage1Args &a, int NCC, int Q, Launch
 // (direct global->LDS loads) while pass p is added.  Lanes own consecutive
 // samples, so LDS reads are conflict-free and each read feeds one FP32 add.
 // Sub-bands are added in ascending order.
+//
+// What bounds it: at 1000 DMs x 64 sub-bands x 28,735 samples (1.84 G adds,
+// 307 MB of rows, 115 MB of series) the (4, 8) shape takes 176 us at 80 KB;
+// without its fills 0.92 of that, without the LDS reads 0.8, without either
+// and without barriers 0.75: waves wait for one another at pass ends and for
+// their own first reads, not for one resource.  A pass's fill as one run of
+// chunks and slots read ahead of their adds took it from 199 us, 133 to 118
+// (500 DMs), 176 to 155 (300 DMs x 128 sub-bands) and 88 to 78 (1000 DMs x
+// 32 sub-bands x 22,379 samples).  Not faster: other wave counts than 8 (they
+// leave SIMDs uneven), three workgroups a CU by fewer registers (spills),
+// integer rows added two at a time, offsets read from LDS.
 
-// Per-pass lane tables: chunk j holds, lane l, the delay offset of DM slot
-// l % DPW for sub-band s0 + j*(64/DPW) + l / DPW, and the LDS row start of
-// sub-band s0 + j*(64/DPW) + l.  A pass spans at most 4 chunks.
-struct S2Tab {
-    int off[4], row[4];
-};
-
+// Per-pass lane tables.  off: chunk j holds, lane l, the LDS offset of DM slot
+// l % DPW's first sample in the row of sub-band s0 + j*(64/DPW) + l / DPW.  A
+// pass spans at most 4 chunks and 64 sub-bands.
 template <int DPW>
 __device__ __forceinline__ void stage2_tab(const Stage2Args &a, long bs, int s0, int s1, int wave, int lane,
-                                           S2Tab &t)
+                                           int (&off)[4])
 {
     constexpr int SC = 64 / DPW;
 #pragma unroll
     for (int j = 0; j < 4; j++) {
         const int c0 = s0 + j * SC, cn = min(SC, s1 - c0);
-        t.off[j] = lane < cn * DPW ? a.d2off[((bs + c0 + lane / DPW) * 8 + wave) * DPW + lane % DPW] : 0;
-        t.row[j] = lane < cn ? a.ldsoff[bs + c0 + lane] : 0;
+        off[j] = lane < cn * DPW ? a.d2off[((bs + c0 + lane / DPW) * kS2Waves + wave) * DPW + lane % DPW] : 0;
     }
 }
 
 // Adds the staged sub-band rows [s0, s1) of one pass into the wave's first
-// NA DM slots, taking offsets and row starts from the lane tables with
-// v_readlane (no memory wait between sub-bands).  All NA*R LDS reads of a
-// sub-band are issued before its adds.
+// NA DM slots, taking their LDS offsets from the lane tables with v_readlane
+// (no memory wait between sub-bands).  A slot's samples are added and the
+// slot is at once read for the next sub-band, so that a wave's other slots'
+// adds cover the reads.
 template <int DPW, int NA, int R>
-__device__ __forceinline__ void stage2_pass(const float *buf, int lane, int s0, int s1, const S2Tab &t,
+__device__ __forceinline__ void stage2_pass(const float *buf, int lane, int s0, int s1, const int (&off)[4],
                                             float (&acc)[DPW][R])
 {
     constexpr int SC = 64 / DPW;
+    float v[NA][R];
+    // slot d's samples of the sub-band whose lane-table entries start at e
+    auto get = [&](int d, int o, int e) {
+        const float *pd = buf + lane + __builtin_amdgcn_readlane(o, e + d);
+#pragma unroll
+        for (int r = 0; r < R; r++) v[d][r] = pd[64 * r];
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // adds slot d and at once reads it for the next sub-band
+    auto step = [&](int o, int e) {
+#pragma unroll
+        for (int d = 0; d < NA; d++) {
+#pragma unroll
+            for (int r = 0; r < R; r++) acc[d][r] += v[d][r];
+            __builtin_amdgcn_sched_barrier(0);
+            get(d, o, e);
+        }
+    };
+#pragma unroll
+    for (int d = 0; d < NA; d++) get(d, off[0], 0);
 #pragma unroll
     for (int j = 0; j < 4; j++) {
         const int cn = min(SC, s1 - (s0 + j * SC));
-        for (int q = 0; q < cn; q++) {
-            const float *row = buf + __builtin_amdgcn_readlane(t.row[j], q) + lane;
-            float v[NA][R];
-#pragma unroll
-            for (int d = 0; d < NA; d++) {
-                const float *pd = row + __builtin_amdgcn_readlane(t.off[j], q * DPW + d);
-#pragma unroll
-                for (int r = 0; r < R; r++) v[d][r] = pd[64 * r];
-            }
-#pragma unroll
-            for (int d = 0; d < NA; d++)
-#pragma unroll
-                for (int r = 0; r < R; r++) acc[d][r] += v[d][r];
-        }
+#pragma unroll 1
+        for (int q = 1; q < cn; q++) step(off[j], q * DPW);
+        if (j == 3 || s0 + (j + 1) * SC >= s1) break;
+        step(off[j < 3 ? j + 1 : 3], 0);
     }
+#pragma unroll
+    for (int d = 0; d < NA; d++)
+#pragma unroll
+        for (int r = 0; r < R; r++) acc[d][r] += v[d][r];
 }
 
 template <int DPW, int R>
-__global__ __launch_bounds__(512) void k_stage2(Stage2Args a)
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k_stage2(Stage2Args a)
 {
     extern __shared__ float lds2[]; // two buffers of a.half floats
     if (a.clock) a.w0 = *a.clock + a.ndump - a.maxdelay - a.N;
@@ -846,11 +867,12 @@ __global__ __launch_bounds__(512) void k_stage2(Stage2Args a)
     const int k = (int)(lid / a.nblk / a.ntile);
     const int blk = k * a.nblk + bx;
     const long gend = min((long)(k + 1) * a.group, a.ndm);
+    constexpr int nw = kS2Waves;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6); // uniform per wavefront
-    const long ibase = (long)k * a.group + (long)bx * 8 * DPW + wave; // DMs ibase + 8*d
+    const long ibase = (long)k * a.group + (long)bx * nw * DPW + wave; // DMs ibase + nw*d
     const long bs = (long)blk * a.nsub;
-    const long base = lmod(a.w0 + t0, a.Lsub);
+    const int base = (int)lmod(a.w0 + t0, a.Lsub), Lsub = (int)a.Lsub; // ring slots fit 32 bits
     const float *grp = a.sub + (long)k * a.nsub * a.spitch;
     const long pb = (long)blk * a.pstride;
     const int np = ldc(a.npass, blk);
@@ -860,35 +882,58 @@ __global__ __launch_bounds__(512) void k_stage2(Stage2Args a)
 #pragma unroll
         for (int r = 0; r < R; r++) acc[d][r] = 0.f;
 
-    int nact = 0; // live DM slots of this wave (wave-uniform): slot d is DM ibase + 8*d
+    int nact = 0; // live DM slots of this wave (wave-uniform): slot d is DM ibase + nw*d
 #pragma unroll
-    for (int d = 0; d < DPW; d++) nact += (ibase + 8 * d < gend) ? 1 : 0;
+    for (int d = 0; d < DPW; d++) nact += (ibase + (long)nw * d < gend) ? 1 : 0;
 
-    // rows of pass p into buffer p&1
-    auto fill = [&](int p) {
-        float *buf = lds2 + (p & 1) * a.half;
+    // The fill of a pass: its rows lie back to back in LDS, so the pass is one
+    // run of 1 KB chunks (64 lanes x 16 bytes) dealt to the waves; a chunk
+    // holds parts of at most two rows (a row is at least 64*R >= 256 floats).
+    // Lane l holds row l's LDS start and its source slot less that start.
+    struct Rows {
+        int off, min;
+    };
+    auto rows_of = [&](int p, Rows &t) {
         const int s0 = ldc(a.pstart, pb + p), s1 = ldc(a.pstart, pb + p + 1);
-        for (int s = s0; s < s1; s++) {
-            long start = base + ldc(a.d2min, bs + s);
-            if (start >= a.Lsub) start -= a.Lsub;
-            const float *src = grp + (long)s * a.spitch + start;
-            const int len = ldc(a.d2span, bs + s) + 64 * R; // spread of the block's delays + tile
-            // 16 bytes per lane: rows start 16-byte aligned with room for
-            // len rounded up to 4, and the ring's mirror covers the source
-            lds_fill16((const uint32_t *)src, (uint32_t *)(buf + ldc(a.ldsoff, bs + s)), len, wave, 8, lane);
+        const long i = bs + min(s0 + lane, s1 - 1);
+        t.off = a.ldsoff[i];
+        t.min = a.d2min[i];
+    };
+    auto fill = [&](int p, const Rows &t) {
+        float *buf = lds2 + (p & 1) * a.half;
+        const int s0 = ldc(a.pstart, pb + p), nr = ldc(a.pstart, pb + p + 1) - s0, used = ldc(a.pused, pb + p);
+        int x = base + t.min;
+        x -= x >= Lsub ? Lsub : 0;
+        x -= t.off;
+        for (int c = wave * 256; c < used; c += nw * 256) {
+            // the last row that starts at or before the chunk
+            const int r = __popcll(__ballot(lane < nr && t.off <= c)) - 1;
+            const int r1 = min(r + 1, nr - 1);
+            const int xa = __builtin_amdgcn_readlane(x, r);
+            const int xb = __builtin_amdgcn_readlane(x, r1) + (int)a.spitch;
+            const int end = r1 > r ? __builtin_amdgcn_readlane(t.off, r1) : used;
+            const int pos = c + 4 * lane;
+            const unsigned o = (unsigned)(pos + (pos < end ? xa : xb)); // >= 0: pos is in the row it is taken from
+            const float *src = grp + (long)(s0 + r) * a.spitch;
+            if (pos < used)
+                __builtin_amdgcn_global_load_lds((const uint32_t *)src + o, (uint32_t *)(buf + c), 16, 0, 0);
         }
     };
-    S2Tab cur, nxt;
+    int cur[4], nxt[4] = {0, 0, 0, 0};
+    Rows rows;
+    rows_of(0, rows);
     stage2_tab<DPW>(a, bs, ldc(a.pstart, pb), ldc(a.pstart, pb + 1), wave, lane, cur);
-    fill(0);
+    fill(0, rows);
+    if (np > 1) rows_of(1, rows);
     for (int p = 0; p < np; p++) {
         // pass p (rows and lane tables) has landed; every wave is done with
         // pass p-1's buffer, which pass p+1 now streams into
         lds_fill_done();
         const int s0 = ldc(a.pstart, pb + p), s1 = ldc(a.pstart, pb + p + 1);
         if (p + 1 < np) {
+            fill(p + 1, rows);
             stage2_tab<DPW>(a, bs, s1, ldc(a.pstart, pb + p + 2), wave, lane, nxt);
-            fill(p + 1);
+            if (p + 2 < np) rows_of(p + 2, rows);
         }
         const float *buf = lds2 + (p & 1) * a.half;
         // only the wave's live DM slots (a prefix of d) read and add
@@ -898,22 +943,22 @@ __global__ __launch_bounds__(512) void k_stage2(Stage2Args a)
             stage2_pass<DPW, (DPW > 1 ? DPW - 1 : 1), R>(buf, lane, s0, s1, cur, acc);
         } else if (nact > 0) { // ragged group ends
             for (int s = s0; s < s1; s++) {
-                const float *row = buf + ldc(a.ldsoff, bs + s) + lane;
 #pragma unroll
                 for (int d = 0; d < DPW; d++)
                     if (d < nact) {
-                        const float *q = row + ldc(a.d2off, ((bs + s) * 8 + wave) * DPW + d);
+                        const float *q = buf + lane + ldc(a.d2off, ((bs + s) * nw + wave) * DPW + d);
 #pragma unroll
                         for (int r = 0; r < R; r++) acc[d][r] += q[64 * r];
                     }
             }
         }
-        cur = nxt;
+#pragma unroll
+        for (int j = 0; j < 4; j++) cur[j] = nxt[j];
     }
     const int tile = (int)(t0 / (64 * R));
 #pragma unroll
     for (int d = 0; d < DPW; d++) {
-        const long i = ibase + 8 * d;
+        const long i = ibase + (long)nw * d;
         if (i >= gend) continue;
         float *out = a.tim + i * a.N;
         double s1 = 0., s2 = 0.;
@@ -946,7 +991,7 @@ static int launch_s2(hipStream_t st, const Stage2Args &a, LaunchSink *sink)
     const size_t shm = (size_t)2 * a.half * 4;
     (void)hipFuncSetAttribute((const void *)k_stage2<DPW, R>,
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
-    kemit(sink, st, k_stage2<DPW, R>, grid, dim3(512), shm, b);
+    kemit(sink, st, k_stage2<DPW, R>, grid, dim3(64 * kS2Waves), shm, b);
     return 0;
 }
 

@@ -163,7 +163,7 @@ struct tx_plan {
     int *d_ldsoff = nullptr, *d_npass = nullptr, *d_pstart = nullptr;
     // device buffers
     int *d_d1 = nullptr, *d_d1min = nullptr, *d_d1sel = nullptr, *d_d2 = nullptr, *d_d2min = nullptr;
-    int *d_d2span = nullptr, *d_d2off = nullptr;
+    int *d_d2off = nullptr, *d_pused = nullptr;
     int *d_vwn = nullptr, *d_whi = nullptr;
     float *d_fcnt = nullptr;
     float *d_sub = nullptr;
@@ -687,7 +687,7 @@ static void plan_free(tx_plan *p)
     hipFree(p->d_d1sel);
     hipFree(p->d_d2);
     hipFree(p->d_d2min);
-    hipFree(p->d_d2span);
+    hipFree(p->d_pused);
     hipFree(p->d_ldsoff);
     hipFree(p->d_npass);
     hipFree(p->d_pstart);
@@ -823,7 +823,7 @@ static int stage2_extents(const PlanMath &pm, int blk, int nblk, std::vector<int
 // `half` floats and `maxsub` sub-bands (the kernel's lane tables hold 4 chunks
 // of 64/DPW).  Returns false if one row alone does not fit.
 struct Stage2Plan {
-    std::vector<int> ldsoff, npass, pstart;
+    std::vector<int> ldsoff, npass, pstart, pused;
     int pstride = 0, maxrow = 0;
     long passes = 0;
 };
@@ -832,7 +832,7 @@ static bool stage2_passes(const PlanMath &pm, int nblkall, int T, const std::vec
 {
     pl.ldsoff.assign((size_t)nblkall * pm.nsub, 0);
     pl.npass.assign(nblkall, 0);
-    std::vector<std::vector<int>> starts(nblkall);
+    std::vector<std::vector<int>> starts(nblkall), fills(nblkall);
     pl.maxrow = 0;
     pl.passes = 0;
     for (int w = 0; w < nblkall; w++) {
@@ -844,24 +844,31 @@ static bool stage2_passes(const PlanMath &pm, int nblkall, int T, const std::vec
             if (len > half) return false;
             if (used + len > half || s - starts[w].back() >= maxsub) {
                 starts[w].push_back(s);
+                fills[w].push_back(used);
                 used = 0;
             }
             pl.ldsoff[(size_t)w * pm.nsub + s] = used;
             used += (len + 3) & ~3; // rows start 16-byte aligned
         }
         starts[w].push_back(pm.nsub);
+        fills[w].push_back(used);
         pl.npass[w] = (int)starts[w].size() - 1;
         if (nact[w]) pl.passes += pl.npass[w];
     }
     pl.pstride = 0;
     for (auto &v : starts) pl.pstride = std::max(pl.pstride, (int)v.size());
     pl.pstart.assign((size_t)nblkall * pl.pstride, pm.nsub);
-    for (int w = 0; w < nblkall; w++)
+    pl.pused.assign((size_t)nblkall * pl.pstride, 0);
+    for (int w = 0; w < nblkall; w++) {
         std::copy(starts[w].begin(), starts[w].end(), pl.pstart.begin() + (size_t)w * pl.pstride);
+        std::copy(fills[w].begin(), fills[w].end(), pl.pused.begin() + (size_t)w * pl.pstride);
+    }
     return true;
 }
 
-// Stage-2 shape: 8 waves, DPW fine DMs per wave, R samples per lane.  The
+static int stage2_maxsub(int DPW) { return std::min(64, 4 * (64 / DPW)); }
+
+// Stage-2 shape: DPW fine DMs per wave, R samples per lane.  The
 // cost of a shape counts, per time tile and DM block: one LDS read per
 // sample-add of its live DMs, the staging traffic of each sub-band row (the
 // block's delay extent + the tile, read from L2/HBM), and a fixed cost per
@@ -875,12 +882,12 @@ static bool choose_stage2(tx_plan *p, std::vector<int> &d2min, std::vector<int> 
     for (int c = 0; c < kNumStage2Shapes; c++) {
         if (force_shape > 0 && force_shape - 1 != c) continue;
         const int DPW = kStage2Shapes[c][0], R = kStage2Shapes[c][1];
-        const int blk = 8 * DPW, T = 64 * R;
+        const int blk = kS2Waves * DPW, T = 64 * R;
         const int nblk = (pm.group + blk - 1) / blk;
         std::vector<int> mn, sp, nact;
         stage2_extents(pm, blk, nblk, mn, sp, &nact);
         Stage2Plan pl;
-        if (!stage2_passes(pm, pm.ndmc * nblk, T, sp, nact, half, 4 * (64 / DPW), pl)) continue;
+        if (!stage2_passes(pm, pm.ndmc * nblk, T, sp, nact, half, stage2_maxsub(DPW), pl)) continue;
         const long ntile = (pm.nsamples + T - 1) / T;
         double cost = 0;
         for (size_t w = 0; w < nact.size(); w++) {
@@ -900,11 +907,11 @@ static bool choose_stage2(tx_plan *p, std::vector<int> &d2min, std::vector<int> 
     if (bi < 0) return false;
     p->DPW = kStage2Shapes[bi][0];
     p->R = kStage2Shapes[bi][1];
-    const int blk = 8 * p->DPW;
+    const int blk = kS2Waves * p->DPW;
     p->nblk = (pm.group + blk - 1) / blk;
     std::vector<int> nact;
     stage2_extents(pm, blk, p->nblk, d2min, d2span, &nact);
-    return stage2_passes(pm, pm.ndmc * p->nblk, 64 * p->R, d2span, nact, half, 4 * (64 / p->DPW), plan);
+    return stage2_passes(pm, pm.ndmc * p->nblk, 64 * p->R, d2span, nact, half, stage2_maxsub(p->DPW), plan);
 }
 
 template <typename T>
@@ -1080,29 +1087,30 @@ extern "C" int tx_plan_create(tx_beam *b, const tx_plan_desc *d, tx_plan **out)
     TRY(upload(&p->d_d1min, d1min));
     TRY(upload(&p->d_d2, pm.d2));
     {
-        // stage 2 reads, per (DM block, sub-band, wave), the DPW delays of
-        // its DM slots relative to the block's lowest delay; slots past the
-        // end of the group hold 0 (computed, never stored)
-        const int blk = 8 * p->DPW;
+        // stage 2 reads, per (DM block, sub-band, wave), where the DPW DM
+        // slots' first samples lie in the pass's LDS rows; slots past the
+        // end of the group hold the row's start (computed, never stored)
+        constexpr int NW = kS2Waves;
+        const int blk = NW * p->DPW;
         std::vector<int> off((size_t)pm.ndmc * p->nblk * pm.nsub * blk, 0);
         for (int k = 0; k < pm.ndmc; k++) {
             const long gend = std::min<long>((long)(k + 1) * pm.group, pm.ndm);
             for (int b = 0; b < p->nblk; b++) {
                 const size_t w = (size_t)k * p->nblk + b;
                 for (int s = 0; s < pm.nsub; s++)
-                    for (int wave = 0; wave < 8; wave++)
+                    for (int wave = 0; wave < NW; wave++)
                         for (int d = 0; d < p->DPW; d++) {
-                            const long i = (long)k * pm.group + (long)b * blk + wave + 8 * d;
-                            if (i < gend)
-                                off[((w * pm.nsub + s) * 8 + wave) * p->DPW + d] =
-                                    pm.d2[(size_t)i * pm.nsub + s] - d2min[w * pm.nsub + s];
+                            const long i = (long)k * pm.group + (long)b * blk + wave + NW * d;
+                            int &o = off[((w * pm.nsub + s) * NW + wave) * p->DPW + d];
+                            o = s2plan.ldsoff[w * pm.nsub + s];
+                            if (i < gend) o += pm.d2[(size_t)i * pm.nsub + s] - d2min[w * pm.nsub + s];
                         }
             }
         }
         TRY(upload(&p->d_d2off, off));
     }
     TRY(upload(&p->d_d2min, d2min));
-    TRY(upload(&p->d_d2span, d2span));
+    TRY(upload(&p->d_pused, s2plan.pused));
     TRY(upload(&p->d_ldsoff, s2plan.ldsoff));
     TRY(upload(&p->d_npass, s2plan.npass));
     TRY(upload(&p->d_pstart, s2plan.pstart));
@@ -1258,7 +1266,6 @@ static void stage2_args(tx_plan *p, long c, Stage2Args &a2)
     a2.Lsub = p->Lsub;
     a2.d2 = p->d_d2;
     a2.d2min = p->d_d2min;
-    a2.d2span = p->d_d2span;
     a2.d2off = p->d_d2off;
     a2.nsub = pm.nsub;
     a2.ndm = pm.ndm;
@@ -1270,6 +1277,7 @@ static void stage2_args(tx_plan *p, long c, Stage2Args &a2)
     a2.ldsoff = p->d_ldsoff;
     a2.npass = p->d_npass;
     a2.pstart = p->d_pstart;
+    a2.pused = p->d_pused;
     a2.pstride = p->pstride2;
     a2.half = p->half2;
     a2.tim = p->d_tim;
