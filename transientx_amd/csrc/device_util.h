@@ -28,6 +28,29 @@ __device__ inline void lds_fill16(const uint32_t *__restrict__ src, uint32_t *ds
         if (c + 4 * lane < len) __builtin_amdgcn_global_load_lds(src + c + 4 * lane, dst + c, 16, 0, 0);
 }
 
+// Rows packed back to back in LDS from buf on, as one run of chunks of 64
+// 16-byte lines dealt to the waves (walking the rows in every wave costs more
+// instructions than the loads).  Lane l holds row l's first word in LDS (off,
+// a multiple of 4) and its source's first word in the row of `pitch` words at
+// src + l*pitch (first); nr <= 64 rows of at least 256 words each, so that a
+// chunk holds parts of at most two, used words in all (a multiple of 4; a
+// row's source must be readable up to the next row's start in LDS).
+__device__ __forceinline__ void lds_fill_rows(const uint32_t *__restrict__ src, long pitch, int off, int first,
+                                              int nr, int used, uint32_t *buf, int wave, int nw, int lane)
+{
+    const int x = first - off;
+    for (int c = wave * 256; c < used; c += nw * 256) {
+        const int r = __popcll(__ballot(lane < nr && off <= c)) - 1; // the last row that starts at or before c
+        const int r1 = min(r + 1, nr - 1);
+        const int xa = __builtin_amdgcn_readlane(x, r);
+        const int xb = __builtin_amdgcn_readlane(x, r1) + (int)pitch;
+        const int end = r1 > r ? __builtin_amdgcn_readlane(off, r1) : used;
+        const int pos = c + 4 * lane;
+        const unsigned o = (unsigned)(pos + (pos < end ? xa : xb)); // >= 0: pos is in the row it is taken from
+        if (pos < used) __builtin_amdgcn_global_load_lds(src + (long)r * pitch + o, buf + c, 16, 0, 0);
+    }
+}
+
 __device__ inline void lds_fill_done()
 {
     __builtin_amdgcn_s_waitcnt(0); // vmcnt(0): every global->LDS load has landed

@@ -482,6 +482,11 @@ __device__ inline void stage1_clock(Stage1Args &a)
 // (channel, coarse DM) inside its row is fixed at plan time: the table d1sel
 // holds its perm selector and word-aligned byte offset, and the inner loop
 // spends one scalar add per (channel, coarse DM) instead of recomputing them.
+// A pass's rows are filled as one run of chunks (lds_fill_rows), not row by row
+// in every wave: (8, 1) 256 -> 227 us and (4, 2) 262 -> 234 at 1000 DMs of 4096
+// channels x 26,123 samples, (8, 2), which fills less per add, unchanged at
+// 220.  Bound by VALU issue: 77% of the cycles, 3 instructions per 4 samples of
+// a channel and coarse DM, the LDS pipe at 65%.
 template <int NCC, int Q>
 __global__ __launch_bounds__(256) void k_stage1_u8(Stage1Args a)
 {
@@ -500,6 +505,11 @@ __global__ __launch_bounds__(256) void k_stage1_u8(Stage1Args a)
     // workgroup, every later slot is a bounded offset from these
     const long in_base = lmod(tau0, a.Lin);
     const long sub_base = lmod(tau0, a.Lsub);
+    // lane l: the lowest delay of channel row l of the pass (the next pass's
+    // are loaded while one is summed)
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    auto mins = [&](int jc) { return (d1min + s * a.cps)[min(jc + lane, a.cps - 1)]; };
+    int dm = mins(0);
     uint32_t lo[NCC][Q], hi[NCC][Q];
 #pragma unroll
     for (int k = 0; k < NCC; k++)
@@ -509,14 +519,12 @@ __global__ __launch_bounds__(256) void k_stage1_u8(Stage1Args a)
     for (int jc = 0; jc < a.cps; jc += a.CH) {
         const int nch = min(a.CH, a.cps - jc);
         __syncthreads();
-        for (int jj = 0; jj < nch; jj++) {
-            const int j = s * a.cps + jc + jj;
-            long start = in_base + ldc(d1min, j);
-            if (start >= a.Lin) start -= a.Lin;
-            const uint32_t *src = (const uint32_t *)(ring + (long)j * a.pitch) + (start >> 2);
-            // RS is a multiple of 4 words; the ring's mirror covers the source
-            lds_fill16(src, lds_u + jj * a.RS, a.RS, tid >> 6, 4, tid & 63);
-        }
+        // RS is a multiple of 4 words; the ring's mirror covers the source
+        long start = in_base + dm;
+        if (start >= a.Lin) start -= a.Lin;
+        lds_fill_rows((const uint32_t *)(ring + (long)(s * a.cps + jc) * a.pitch), a.pitch >> 2, lane * a.RS,
+                      (int)(start >> 2), nch, nch * a.RS, lds_u, wave, 4, lane);
+        dm = mins(jc + a.CH);
         lds_fill_done();
         // channels two at a time: one v_add3_u32 adds both channels' 16-bit
         // pairs to an accumulator (integer sums, so the order is free); an
@@ -598,9 +606,54 @@ __global__ __launch_bounds__(256) void k_stage1_u8(Stage1Args a)
     }
 }
 
+// Adds n staged rows into SL slots (fine DMs in stage 2, coarse DMs in the f32
+// stage 1) of R samples each, STEP words apart from buf on: row i of slot d
+// starts at lane table off[j]'s entry (i - j*SC)*SL + d, SC = 64/SL rows per
+// table, taken with v_readlane (no memory wait between rows).  Only the first
+// NA slots read and add.  A slot's samples are added and the slot is at once
+// read for the next row, so that the other slots' adds cover the reads.
+// Rows are added in ascending order.
+template <int SL, int NA, int R, int STEP>
+__device__ __forceinline__ void add_rows(const float *buf, int n, const int (&off)[4], float (&acc)[SL][R])
+{
+    constexpr int SC = 64 / SL;
+    float v[NA][R];
+    // slot d's samples of the row whose lane-table entries start at e
+    auto get = [&](int d, int o, int e) {
+        const float *pd = buf + __builtin_amdgcn_readlane(o, e + d);
+#pragma unroll
+        for (int r = 0; r < R; r++) v[d][r] = pd[STEP * r];
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // adds slot d and at once reads it for the next row
+    auto step = [&](int o, int e) {
+#pragma unroll
+        for (int d = 0; d < NA; d++) {
+#pragma unroll
+            for (int r = 0; r < R; r++) acc[d][r] += v[d][r];
+            __builtin_amdgcn_sched_barrier(0);
+            get(d, o, e);
+        }
+    };
+#pragma unroll
+    for (int d = 0; d < NA; d++) get(d, off[0], 0);
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const int cn = min(SC, n - j * SC);
+#pragma unroll 1
+        for (int q = 1; q < cn; q++) step(off[j], q * SL);
+        if (j == 3 || (j + 1) * SC >= n) break;
+        step(off[j < 3 ? j + 1 : 3], 0);
+    }
+#pragma unroll
+    for (int d = 0; d < NA; d++)
+#pragma unroll
+        for (int r = 0; r < R; r++) acc[d][r] += v[d][r];
+}
+
 // f32 input: same tiling; each thread owns U = 4*Q output times strided by
 // 256 (consecutive lanes read consecutive LDS words).  Channels are summed
-// in ascending order, one FP32 add each, per output time.
+// in ascending order, one FP32 add each, per output time (add_rows).
 // FE: the ring holds 8-bit samples y (the front end's td = fd = 1 input) and
 // the LDS rows their values (y - fe_off[j]) * fe_gain[j]: each pass stages the
 // raw rows (RS bytes each, behind the CH f32 rows) and forms the floats once,
@@ -623,6 +676,31 @@ __global__ __launch_bounds__(256) void k_stage1_f32(Stage1Args a)
     const int *d1min = a.d1min + (long)kc * a.C;
     const long in_base = lmod(tau0, a.Lin);
     const long sub_base = lmod(tau0, a.Lsub);
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // up to 4 coarse DMs the offsets come from lane tables (add_rows) and a
+    // pass is one run of chunks, which keeps scalar loads and their waits out of
+    // the loops: 500 DMs of 4096 channels x 26,123 samples, (4, 1), 306 -> 277 us.
+    // With 8 the slots read ahead take the registers of a wave per SIMD (415
+    // against 375 us)
+    constexpr bool kScalar = NCC >= 8;
+    auto mins = [&](int jc) { return (d1min + s * a.cps)[min(jc + lane, a.cps - 1)]; }; // as in k_stage1_u8
+    int dml = kScalar ? 0 : mins(0);
+    // where coarse DM k of channel row i starts in LDS: lane (i % SC)*NCC + k of
+    // table i / SC (CH <= 16 rows in 4 tables)
+    constexpr int SC = 64 / NCC;
+    auto offs = [&](int jc, int(&o)[4]) {
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            const int i = t * SC + lane / NCC;
+            o[t] = 0;
+            if (i < a.CH && jc + i < a.cps) {
+                const int j = s * a.cps + jc + i;
+                o[t] = i * a.RS + a.d1[(long)j * a.d1pitch + k0 + lane % NCC] - d1min[j];
+            }
+        }
+    };
+    int off[4], noff[4];
+    if (!kScalar) offs(0, off);
     float acc[NCC][U];
 #pragma unroll
     for (int k = 0; k < NCC; k++)
@@ -634,20 +712,33 @@ __global__ __launch_bounds__(256) void k_stage1_f32(Stage1Args a)
     for (int jc = 0; jc < a.cps; jc += a.CH) {
         const int nch = min(a.CH, a.cps - jc);
         __syncthreads();
-        for (int jj = 0; jj < nch; jj++) {
-            const int j = s * a.cps + jc + jj;
-            long start = in_base + ldc(d1min, j);
-            if (start >= a.Lin) start -= a.Lin;
-            if (FE) {
-                // RS is a multiple of 16: whole 16-byte fills of RS bytes
-                const uint32_t *src = (const uint32_t *)((const uint8_t *)a.ring + (long)j * a.pitch + start);
-                lds_fill16(src, raw + jj * RW, RW, tid >> 6, 4, tid & 63);
-            } else {
-                const float *src = ring + (long)j * a.pitch + start;
-                // RS is a multiple of 4 floats: 16-byte fills, rows on 16-byte lines
-                lds_fill16((const uint32_t *)src, (uint32_t *)(lds_f + jj * a.RS), a.RS, tid >> 6, 4,
-                           tid & 63);
+        if (kScalar) {
+            for (int jj = 0; jj < nch; jj++) {
+                const int j = s * a.cps + jc + jj;
+                long start = in_base + ldc(d1min, j);
+                if (start >= a.Lin) start -= a.Lin;
+                if (FE) {
+                    // RS is a multiple of 16: whole 16-byte fills of RS bytes
+                    const uint32_t *src = (const uint32_t *)((const uint8_t *)a.ring + (long)j * a.pitch + start);
+                    lds_fill16(src, raw + jj * RW, RW, wave, 4, lane);
+                } else {
+                    const float *src = ring + (long)j * a.pitch + start;
+                    // RS is a multiple of 4 floats: 16-byte fills, rows on 16-byte lines
+                    lds_fill16((const uint32_t *)src, (uint32_t *)(lds_f + jj * a.RS), a.RS, wave, 4, lane);
+                }
             }
+        } else {
+            long start = in_base + dml;
+            if (start >= a.Lin) start -= a.Lin;
+            const long j0 = (long)(s * a.cps + jc) * a.pitch;
+            if (FE)
+                lds_fill_rows((const uint32_t *)((const uint8_t *)a.ring + j0), a.pitch >> 2, lane * RW,
+                              (int)(start >> 2), nch, nch * RW, raw, wave, 4, lane);
+            else
+                lds_fill_rows((const uint32_t *)(ring + j0), a.pitch, lane * a.RS, (int)start, nch, nch * a.RS,
+                              (uint32_t *)lds_f, wave, 4, lane);
+            dml = mins(jc + a.CH);
+            offs(jc + a.CH, noff);
         }
         lds_fill_done();
         if (FE) {
@@ -677,25 +768,31 @@ __global__ __launch_bounds__(256) void k_stage1_f32(Stage1Args a)
             }
             __syncthreads();
         }
-        for (int jj = 0; jj < nch; jj++) {
-            const int j = s * a.cps + jc + jj;
-            const int dmn = ldc(d1min, j);
-            const float *row = lds_f + jj * a.RS + tid;
-            const long dj = (long)j * a.d1pitch + k0;
-            // every LDS read of the channel issued before the adds (one
-            // wait per channel instead of one per read); each accumulator
-            // still takes the channels in ascending order
-            float v[NCC][U];
+        if constexpr (kScalar) {
+            for (int jj = 0; jj < nch; jj++) {
+                const int j = s * a.cps + jc + jj;
+                const int dmn = ldc(d1min, j);
+                const float *row = lds_f + jj * a.RS + tid;
+                const long dj = (long)j * a.d1pitch + k0;
+                // every LDS read of the channel issued before the adds (one
+                // wait per channel instead of one per read); each accumulator
+                // still takes the channels in ascending order
+                float v[NCC][U];
 #pragma unroll
-            for (int k = 0; k < NCC; k++) {
-                const float *p = row + (ldc(a.d1, dj + k) - dmn);
+                for (int k = 0; k < NCC; k++) {
+                    const float *p = row + (ldc(a.d1, dj + k) - dmn);
 #pragma unroll
-                for (int u = 0; u < U; u++) v[k][u] = p[u * 256];
+                    for (int u = 0; u < U; u++) v[k][u] = p[u * 256];
+                }
+#pragma unroll
+                for (int k = 0; k < NCC; k++)
+#pragma unroll
+                    for (int u = 0; u < U; u++) acc[k][u] += v[k][u];
             }
+        } else {
+            add_rows<NCC, NCC, U, 256>(lds_f + tid, nch, off, acc);
 #pragma unroll
-            for (int k = 0; k < NCC; k++)
-#pragma unroll
-                for (int u = 0; u < U; u++) acc[k][u] += v[k][u];
+            for (int t = 0; t < 4; t++) off[t] = noff[t];
         }
     }
 
@@ -811,50 +908,6 @@ __device__ __forceinline__ void stage2_tab(const Stage2Args &a, long bs, int s0,
     }
 }
 
-// Adds the staged sub-band rows [s0, s1) of one pass into the wave's first
-// NA DM slots, taking their LDS offsets from the lane tables with v_readlane
-// (no memory wait between sub-bands).  A slot's samples are added and the
-// slot is at once read for the next sub-band, so that a wave's other slots'
-// adds cover the reads.
-template <int DPW, int NA, int R>
-__device__ __forceinline__ void stage2_pass(const float *buf, int lane, int s0, int s1, const int (&off)[4],
-                                            float (&acc)[DPW][R])
-{
-    constexpr int SC = 64 / DPW;
-    float v[NA][R];
-    // slot d's samples of the sub-band whose lane-table entries start at e
-    auto get = [&](int d, int o, int e) {
-        const float *pd = buf + lane + __builtin_amdgcn_readlane(o, e + d);
-#pragma unroll
-        for (int r = 0; r < R; r++) v[d][r] = pd[64 * r];
-        __builtin_amdgcn_sched_barrier(0);
-    };
-    // adds slot d and at once reads it for the next sub-band
-    auto step = [&](int o, int e) {
-#pragma unroll
-        for (int d = 0; d < NA; d++) {
-#pragma unroll
-            for (int r = 0; r < R; r++) acc[d][r] += v[d][r];
-            __builtin_amdgcn_sched_barrier(0);
-            get(d, o, e);
-        }
-    };
-#pragma unroll
-    for (int d = 0; d < NA; d++) get(d, off[0], 0);
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-        const int cn = min(SC, s1 - (s0 + j * SC));
-#pragma unroll 1
-        for (int q = 1; q < cn; q++) step(off[j], q * DPW);
-        if (j == 3 || s0 + (j + 1) * SC >= s1) break;
-        step(off[j < 3 ? j + 1 : 3], 0);
-    }
-#pragma unroll
-    for (int d = 0; d < NA; d++)
-#pragma unroll
-        for (int r = 0; r < R; r++) acc[d][r] += v[d][r];
-}
-
 template <int DPW, int R>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k_stage2(Stage2Args a)
 {
@@ -886,10 +939,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
 #pragma unroll
     for (int d = 0; d < DPW; d++) nact += (ibase + (long)nw * d < gend) ? 1 : 0;
 
-    // The fill of a pass: its rows lie back to back in LDS, so the pass is one
-    // run of 1 KB chunks (64 lanes x 16 bytes) dealt to the waves; a chunk
-    // holds parts of at most two rows (a row is at least 64*R >= 256 floats).
-    // Lane l holds row l's LDS start and its source slot less that start.
+    // The rows of a pass: lane l holds row l's LDS start and its lowest delay.
     struct Rows {
         int off, min;
     };
@@ -900,24 +950,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
         t.min = a.d2min[i];
     };
     auto fill = [&](int p, const Rows &t) {
-        float *buf = lds2 + (p & 1) * a.half;
-        const int s0 = ldc(a.pstart, pb + p), nr = ldc(a.pstart, pb + p + 1) - s0, used = ldc(a.pused, pb + p);
+        const int s0 = ldc(a.pstart, pb + p), nr = ldc(a.pstart, pb + p + 1) - s0;
         int x = base + t.min;
         x -= x >= Lsub ? Lsub : 0;
-        x -= t.off;
-        for (int c = wave * 256; c < used; c += nw * 256) {
-            // the last row that starts at or before the chunk
-            const int r = __popcll(__ballot(lane < nr && t.off <= c)) - 1;
-            const int r1 = min(r + 1, nr - 1);
-            const int xa = __builtin_amdgcn_readlane(x, r);
-            const int xb = __builtin_amdgcn_readlane(x, r1) + (int)a.spitch;
-            const int end = r1 > r ? __builtin_amdgcn_readlane(t.off, r1) : used;
-            const int pos = c + 4 * lane;
-            const unsigned o = (unsigned)(pos + (pos < end ? xa : xb)); // >= 0: pos is in the row it is taken from
-            const float *src = grp + (long)(s0 + r) * a.spitch;
-            if (pos < used)
-                __builtin_amdgcn_global_load_lds((const uint32_t *)src + o, (uint32_t *)(buf + c), 16, 0, 0);
-        }
+        lds_fill_rows((const uint32_t *)(grp + (long)s0 * a.spitch), a.spitch, t.off, x, nr, ldc(a.pused, pb + p),
+                      (uint32_t *)(lds2 + (p & 1) * a.half), wave, nw, lane);
     };
     int cur[4], nxt[4] = {0, 0, 0, 0};
     Rows rows;
@@ -938,9 +975,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
         const float *buf = lds2 + (p & 1) * a.half;
         // only the wave's live DM slots (a prefix of d) read and add
         if (nact == DPW) {
-            stage2_pass<DPW, DPW, R>(buf, lane, s0, s1, cur, acc);
+            add_rows<DPW, DPW, R, 64>(buf + lane, s1 - s0, cur, acc);
         } else if (DPW > 1 && nact == DPW - 1) {
-            stage2_pass<DPW, (DPW > 1 ? DPW - 1 : 1), R>(buf, lane, s0, s1, cur, acc);
+            add_rows<DPW, (DPW > 1 ? DPW - 1 : 1), R, 64>(buf + lane, s1 - s0, cur, acc);
         } else if (nact > 0) { // ragged group ends
             for (int s = s0; s < s1; s++) {
 #pragma unroll
