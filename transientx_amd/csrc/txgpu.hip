@@ -717,9 +717,17 @@ static void plan_free(tx_plan *p)
 }
 
 // Stage-1 shape: NCC coarse DMs per workgroup (one input pass serves them
-// all), Q quads per thread, CH channel rows per LDS pass within budget.
-static bool choose_stage1(tx_plan *p, std::vector<int> &d1min, int lds_budget, int force_ncc,
-                          int force_q)
+// all), Q quads per thread, CH channel rows per LDS pass within an LDS budget
+// (f32 rows, four times the 8-bit ones: 24, 32 or 40 KB; 8-bit rows 24 KB, six
+// workgroups a CU).  The cost of a shape, in adds of one thread's quad:
+// per workgroup its adds (slots past the last coarse DM too), the words it
+// stages, its passes (barrier and fill latency) and its start, times
+// 1 + W/workgroups for the end of a launch that does not fill the CUs.  The
+// constants are fitted to the measured times of every shape on 23 rows (64 to
+// 4096 channels, 512 to 31,250 samples, 24 to 2500 DMs): the choice is within
+// 1% of the best shape on average, 8% at worst, where the widest NCC that
+// fits, the rule before, is 1.5 times slower on average.
+static bool choose_stage1(tx_plan *p, std::vector<int> &d1min, int force_ncc, int force_q)
 {
     const PlanMath &pm = p->pm;
     const bool u8 = p->beam->dtype == TX_DTYPE_U8;
@@ -727,7 +735,8 @@ static bool choose_stage1(tx_plan *p, std::vector<int> &d1min, int lds_budget, i
     int ncc0 = 1;
     while (ncc0 < pm.ndmc && ncc0 < maxncc) ncc0 <<= 1;
     if (force_ncc > maxncc) return false;
-    if (force_ncc > ncc0) ncc0 = force_ncc;
+    ncc0 = force_ncc > 0 ? force_ncc : std::min(ncc0, 8);
+    double best = 1e300;
     for (int NCC = ncc0; NCC >= 1; NCC >>= 1) {
         if (force_ncc > 0 && NCC != force_ncc) continue;
         const int nkc = (pm.ndmc + NCC - 1) / NCC;
@@ -749,6 +758,7 @@ static bool choose_stage1(tx_plan *p, std::vector<int> &d1min, int lds_budget, i
                 mn[(size_t)kc * pm.nchans + j] = lo;
                 spread = std::max(spread, hi - lo);
             }
+        bool kept = false;
         for (int Q = 2; Q >= 1; Q--) {
             if (force_q > 0 && Q != force_q) continue;
             // u8: words covering spread (from the word-aligned row start) +
@@ -757,19 +767,31 @@ static bool choose_stage1(tx_plan *p, std::vector<int> &d1min, int lds_budget, i
             // 8-bit ring are whole 16-byte fills
             // (rows a multiple of 4 words: 16-byte global->LDS fills)
             const int RS = u8 ? ((spread + 4 * 256 * Q + 8 + 3) / 4 + 3) & ~3 : (spread + 1024 * Q + 1 + 15) & ~15;
-            int CH = 0, CH_fe = 0;
-            for (int c = std::min(16, pm.cps); c >= 1; c--)
-                if (pm.cps % c == 0 && (long)c * RS * 4 <= lds_budget) {
-                    CH = c;
-                    break;
-                }
-            // the front end in the load: RS floats plus RS raw bytes per row
-            for (int c = std::min(16, pm.cps); c >= 1 && !u8; c--)
-                if (pm.cps % c == 0 && (long)c * RS * 5 <= lds_budget) {
-                    CH_fe = c;
-                    break;
-                }
-            if (CH >= std::min(4, pm.cps) || (NCC == 1 && Q == 1 && CH >= 1)) {
+            for (int kb : {24, 32, 40}) {
+                if (u8 && kb > 24) break;
+                const long lds_budget = std::min(p->beam->max_lds, kb * 1024);
+                int CH = 0, CH_fe = 0;
+                for (int c = std::min(16, pm.cps); c >= 1; c--)
+                    if (pm.cps % c == 0 && (long)c * RS * 4 <= lds_budget) {
+                        CH = c;
+                        break;
+                    }
+                // the front end in the load: RS floats plus RS raw bytes per row
+                for (int c = std::min(16, pm.cps); c >= 1 && !u8; c--)
+                    if (pm.cps % c == 0 && (long)c * RS * 5 <= lds_budget) {
+                        CH_fe = c;
+                        break;
+                    }
+                if (CH < std::min(4, pm.cps) && !(NCC == 1 && Q == 1 && CH >= 1)) continue;
+                const double nwg = (double)nkc * ((pm.ndump + 3 + 1024 * Q - 1) / (1024 * Q)) * pm.nsub;
+                double cost;
+                if (u8)
+                    cost = pm.cps * (NCC * Q * (NCC >= 8 ? 1.12 : 1.) + 0.0055 * RS + 9.5 / CH) + 227.;
+                else
+                    cost = pm.cps * (NCC * Q * (NCC >= 8 ? 0.93 : 1.) + 0.00525 * RS + 8. / CH) + 27.;
+                cost *= nwg * (1. + (u8 ? 1055. : 1353.) / nwg) * ((long)CH * RS * 4 > 24576 ? 1.07 : 1.);
+                if (cost >= best) continue;
+                best = cost;
                 p->NCC = NCC;
                 p->Q = Q;
                 p->CH = CH;
@@ -777,12 +799,12 @@ static bool choose_stage1(tx_plan *p, std::vector<int> &d1min, int lds_budget, i
                 p->RS = RS;
                 p->nkc = nkc;
                 p->read1 = u8 ? (long)RS * 4 + 4 : (long)RS + 1;
-                d1min.swap(mn);
-                return true;
+                kept = true;
             }
         }
+        if (kept) d1min = mn;
     }
-    return false;
+    return best < 1e300;
 }
 
 // Stage-2 delay extents of every DM block for blocks of `blk` fine DMs.
@@ -868,15 +890,23 @@ static bool stage2_passes(const PlanMath &pm, int nblkall, int T, const std::vec
 
 static int stage2_maxsub(int DPW) { return std::min(64, 4 * (64 / DPW)); }
 
-// Stage-2 shape: DPW fine DMs per wave, R samples per lane.  The
-// cost of a shape counts, per time tile and DM block: one LDS read per
-// sample-add of its live DMs, the staging traffic of each sub-band row (the
-// block's delay extent + the tile, read from L2/HBM), and a fixed cost per
-// pass (barrier and load latency the double buffer cannot hide).
+// Stage-2 shape (DPW fine DMs per wave, R samples per lane) and LDS per
+// workgroup: force_shape and force_lds, or where those are 0 every shape with
+// one to four workgroups' LDS per CU.  The cost of a choice counts, per time
+// tile and DM block: one LDS read and add per sample of its live DMs, each
+// sub-band row staged (the block's delay extent + the tile), its passes
+// (barrier and fill latency the double buffer does not cover) and its start
+// and end; times a factor for the workgroups that share a CU (shapes of 16
+// accumulators have the registers for three or four) plus the end of a launch
+// that does not fill the CUs.  Fitted to the measured times of every choice on
+// 23 rows (as for stage 1): within 2.5% of the best on average; one LDS size and
+// no cost for workgroups, the rule before, were 19% off on average and 1.9
+// times slower on the 16 us row.
 static bool choose_stage2(tx_plan *p, std::vector<int> &d2min, std::vector<int> &d2span,
-                          Stage2Plan &plan, int half, int force_shape)
+                          Stage2Plan &plan, int force_shape, int force_lds)
 {
     const PlanMath &pm = p->pm;
+    const int max_lds = p->beam->max_lds;
     double best = 1e300;
     int bi = -1;
     for (int c = 0; c < kNumStage2Shapes; c++) {
@@ -886,22 +916,30 @@ static bool choose_stage2(tx_plan *p, std::vector<int> &d2min, std::vector<int> 
         const int nblk = (pm.group + blk - 1) / blk;
         std::vector<int> mn, sp, nact;
         stage2_extents(pm, blk, nblk, mn, sp, &nact);
-        Stage2Plan pl;
-        if (!stage2_passes(pm, pm.ndmc * nblk, T, sp, nact, half, stage2_maxsub(DPW), pl)) continue;
-        const long ntile = (pm.nsamples + T - 1) / T;
-        double cost = 0;
+        double adds = 0, fill = 0, wgs = 0;
         for (size_t w = 0; w < nact.size(); w++) {
             if (!nact[w]) continue;
-            double fill = 0;
-            for (int s = 0; s < pm.nsub; s++) fill += sp[w * pm.nsub + s] + T;
-            cost += (double)ntile * ((double)nact[w] * T * pm.nsub + 2.0 * fill);
+            adds += (double)nact[w] * T * pm.nsub;
+            for (int s = 0; s < pm.nsub; s++) fill += (sp[w * pm.nsub + s] + T + 3) & ~3;
+            wgs++;
         }
-        cost += (double)ntile * pl.passes * 16384.0;
-        const double nwg = (double)ntile * pm.ndmc * nblk;
-        if (nwg < 1024) cost *= 1.0 + 0.5 * (1024 - nwg) / 1024; // too few workgroups to fill 256 CUs
-        if (cost < best) {
-            best = cost;
-            bi = c;
+        const double shape = DPW == 8 ? 1.97 : DPW * R < 32 ? 1. : DPW == 1 ? 0.93 : DPW == 2 ? 1.065 : 1.;
+        const double ntile = (double)((pm.nsamples + T - 1) / T);
+        for (int kb : {160, 80, 52, 40}) {
+            const int lds = force_lds > 0 ? std::min(max_lds, force_lds) : std::min(max_lds, kb * 1024);
+            Stage2Plan pl;
+            if (stage2_passes(pm, pm.ndmc * nblk, T, sp, nact, (lds / 8) & ~3, stage2_maxsub(DPW), pl)) {
+                const bool few = DPW * R < 32;
+                const double share = kb == 160 ? 1.15 : kb == 80 ? 1. : kb == 52 ? (few ? 0.86 : 1.03) : few ? 0.81 : 1.08;
+                const double cost = ntile * (adds * shape + 1.08 * fill + 14900. * pl.passes + 87000. * wgs) *
+                                    (share + 220. / (ntile * wgs));
+                if (cost < best) {
+                    best = cost;
+                    bi = c;
+                    p->half2 = (lds / 8) & ~3; // words per buffer (a multiple of 4): two buffers
+                }
+            }
+            if (force_lds > 0) break;
         }
     }
     if (bi < 0) return false;
@@ -911,7 +949,7 @@ static bool choose_stage2(tx_plan *p, std::vector<int> &d2min, std::vector<int> 
     p->nblk = (pm.group + blk - 1) / blk;
     std::vector<int> nact;
     stage2_extents(pm, blk, p->nblk, d2min, d2span, &nact);
-    return stage2_passes(pm, pm.ndmc * p->nblk, 64 * p->R, d2span, nact, half, stage2_maxsub(p->DPW), plan);
+    return stage2_passes(pm, pm.ndmc * p->nblk, 64 * p->R, d2span, nact, p->half2, stage2_maxsub(p->DPW), plan);
 }
 
 template <typename T>
@@ -1002,11 +1040,6 @@ extern "C" int tx_plan_create(tx_beam *b, const tx_plan_desc *d, tx_plan **out)
     std::vector<float> fcntf(pm.nsub);
     for (int s = 0; s < pm.nsub; s++) fcntf[s] = (float)p->fcnt[s];
 
-    // stage 1: 256-thread workgroups, ~6 per CU -> 24 KB of LDS each;
-    // stage 2: 512-thread workgroups, 2 per CU -> 80 KB each
-    const int budget1 = std::min(b->max_lds, 24576);
-    int budget2 = std::min(b->max_lds, 81920);
-    if (d->s2_lds > 0) budget2 = std::min(b->max_lds, d->s2_lds);
     if (d->s1_ncc < 0 || d->s1_ncc > 16 || (d->s1_ncc & (d->s1_ncc - 1)) || d->s1_q < 0 || d->s1_q > 2 ||
         d->s2_shape < 0 || d->s2_shape > kNumStage2Shapes || (d->s2_lds != 0 && d->s2_lds < 4096) ||
         d->s3_window < 0 || d->s3_window > 1) {
@@ -1014,25 +1047,17 @@ extern "C" int tx_plan_create(tx_beam *b, const tx_plan_desc *d, tx_plan **out)
         return fail(TX_EINVAL, "launch shape override out of range");
     }
     std::vector<int> d1min, d2min, d2span;
-    if (!choose_stage1(p, d1min, budget1, d->s1_ncc, d->s1_q)) {
+    if (!choose_stage1(p, d1min, d->s1_ncc, d->s1_q)) {
         delete p;
         return fail(TX_EINVAL, "stage-1 tile does not fit in LDS (delay spread too large)");
     }
     Stage2Plan s2plan;
-    bool fit2 = choose_stage2(p, d2min, d2span, s2plan, (budget2 / 8) & ~3, d->s2_shape);
-    if (!fit2 && d->s2_lds == 0 && b->max_lds > budget2) {
-        // rows whose DM step moves the low sub-bands by thousands of samples
-        // (high time resolution, high DM): one workgroup per CU, all its LDS
-        budget2 = b->max_lds;
-        fit2 = choose_stage2(p, d2min, d2span, s2plan, (budget2 / 8) & ~3, d->s2_shape);
-    }
-    if (!fit2) {
+    if (!choose_stage2(p, d2min, d2span, s2plan, d->s2_shape, d->s2_lds)) {
         delete p;
         return fail(TX_EINVAL, "stage-2 tile does not fit in LDS (delay spread too large)");
     }
     // >= 4096 so that a stage-1 tile (<= 2048 samples) wraps the ring at most once
     p->Lsub = std::max<long>(round_up(N + pm.D2 + 64, 64), 4096);
-    p->half2 = (budget2 / 8) & ~3; // floats per buffer (a multiple of 4): two buffers in budget2 bytes
     p->pstride2 = s2plan.pstride;
     p->maxrow2 = s2plan.maxrow;
     // a stage-2 row is read contiguously from its start slot
