@@ -90,3 +90,41 @@ def test_refine_without_maps_matches_with_maps():
     finally:
         R.close()
     assert a.tobytes() == b.tobytes()
+
+
+@pytest.mark.parametrize("nchan,nbin", [
+    (8, 2), (64, 31), (40, 32), (64, 33), (40, 64), (33, 65), (32, 129), (64, 256), (64, 260), (128, 511),
+    (64, 513), (16, 1023), (16, 1024), (16, 1028), (9, 2047), (8, 2048), (8, 2049)])
+def test_refine_row_lengths(nchan, nbin):
+    """Row lengths around every change of kernel and of samples per lane, with
+    and without maps, on noise, zeros, whole numbers (ties), negative rows and
+    an infinity."""
+    import torch
+
+    tbin = 98.304e-6
+    f = np.linspace(1500.0, 1200.0, nchan)
+    rng = np.random.default_rng(nbin)
+    x = rng.normal(size=(6, nchan, nbin)).astype(np.float32)
+    x[1] = 0.0
+    x[2] = rng.integers(0, 3, (nchan, nbin))
+    x[3] = -np.abs(x[3])
+    x[4, nchan // 2, nbin // 2] = np.inf
+    dm = rng.uniform(20, 300, 6)
+    R = Refiner(f, nbin, tbin, 0.1, max_batch=4)
+    try:
+        xt = torch.from_numpy(x).cuda()
+        say("case", nchan, nbin)
+        plain = R.run(xt, dm)
+        res, (dmt, snr, wid) = R.run(xt, dm, maps=True)
+        dmt, snr, wid = dmt.cpu().numpy(), snr.cpu().numpy(), wid.cpu().numpy()
+    finally:
+        R.close()
+    assert plain.tobytes() == res.tobytes()
+    for c in range(6):
+        odmt = oracle.refine_optimize(oracle.cand_dedisperse(x[c], f, dm[c], tbin), f, tbin, dm[c])[0]
+        assert np.array_equal(dmt[c].view(np.uint32), odmt.view(np.uint32)), f"dmtmap cand {c}"
+        S, W, j, i, s = oracle.refine_mf(odmt, 0.1)
+        assert np.array_equal(snr[c].view(np.uint32), S.view(np.uint32)), f"snr map cand {c}"
+        assert np.array_equal(wid[c], W), f"width map cand {c}"
+        assert (res[c]["maxdmid"], res[c]["maxtid"], res[c]["wn"]) == (j, i, W[j, i])
+        assert res[c]["snr"] == np.float32(s)

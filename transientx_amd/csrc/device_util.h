@@ -94,6 +94,35 @@ __device__ __forceinline__ double wave_scan_incl_d(double x)
 // Lane l - 1's value (0 on lane 0): wave_shr:1.
 __device__ __forceinline__ double wave_shr1_d(double x) { return dpp_d<0x138, 0xF, true>(x); }
 
+// Wavefront maximum of floats (NaNs lose) and minimum of ints, the same steps
+// as the scan's: lane 63 holds the result, which goes to every lane.
+__device__ __forceinline__ float wave_max_f(float x)
+{
+    auto step = [&](auto moved) { x = fmaxf(x, __int_as_float(moved)); };
+#define TXGPU_DPP(CTRL, MASK) __builtin_amdgcn_update_dpp(__float_as_int(x), __float_as_int(x), CTRL, MASK, 0xF, false)
+    step(TXGPU_DPP(0x111, 0xF));
+    step(TXGPU_DPP(0x112, 0xF));
+    step(TXGPU_DPP(0x114, 0xF));
+    step(TXGPU_DPP(0x118, 0xF));
+    step(TXGPU_DPP(0x142, 0xA));
+    step(TXGPU_DPP(0x143, 0xC));
+#undef TXGPU_DPP
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), 63));
+}
+
+__device__ __forceinline__ int wave_min_i(int x)
+{
+#define TXGPU_DPP(CTRL, MASK) x = min(x, __builtin_amdgcn_update_dpp(x, x, CTRL, MASK, 0xF, false))
+    TXGPU_DPP(0x111, 0xF);
+    TXGPU_DPP(0x112, 0xF);
+    TXGPU_DPP(0x114, 0xF);
+    TXGPU_DPP(0x118, 0xF);
+    TXGPU_DPP(0x142, 0xA);
+    TXGPU_DPP(0x143, 0xC);
+#undef TXGPU_DPP
+    return __builtin_amdgcn_readlane(x, 63);
+}
+
 typedef float f4v __attribute__((ext_vector_type(4)));
 
 // Four floats of LDS at a 16-byte aligned address, as one 128-bit read.

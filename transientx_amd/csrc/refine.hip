@@ -14,10 +14,13 @@
 //                    first pass loads the cutout (band order, padding and the
 //                    incoherent shift fused in); the last one writes the DM
 //                    rows in trial order.
-//   R2 k_mf          one lane per DM row for the sequential parts (FP64
-//                    mean/variance, the FP32 circular running sum, in the
-//                    reference's order), then the whole wavefront per row for
-//                    the width loop; per-row first maximum.
+//                    (k_tree_rows: rows of 32 to 2048 samples, a wave to a
+//                    pair of rows.)
+//   R2 k_mf_rows     rows in LDS: one lane per DM row for the sequential parts
+//                    (FP64 mean/variance, the FP32 circular running sum, in the
+//                    reference's order), then a wavefront per row for the width
+//                    loop; per-row first maximum.  Longer rows: k_mf_scan for
+//                    the sequential parts, k_mf_box for the widths.
 //   R3 k_argmax      first maximum of each cutout's S/N map (row-major).
 //
 // All sums are elementwise FP32 adds (tree) or sequential in the reference's
@@ -35,7 +38,13 @@
 namespace txgpu {
 int set_error(int code, const std::string &msg);
 }
+using txgpu::f4v;
+using txgpu::lds_f4;
 using txgpu::lds_fill;
+using txgpu::lds_fill16;
+using txgpu::ldc;
+using txgpu::wave_max_f;
+using txgpu::wave_min_i;
 using txgpu::lds_fill_done;
 using txgpu::set_error;
 
@@ -44,6 +53,21 @@ namespace {
 constexpr int kTreeLdsFloats = 16384; // 64 KB of rows per tree workgroup
 constexpr int kMaxItems = 16;         // pair items per thread per chunk (256 threads)
 constexpr int kMaxMfBox = 64;
+// Row lengths of k_tree_rows, beside k_tree_pass: the whole grid of 128 cutouts
+// of 1024 channels takes 226 us against 301 at 32 samples, 253 against 359 at
+// 64, 308 against 460 at 128; 64 cutouts 1256 against 1800 at 1000 samples, 32
+// cutouts 2783 against 2876 at 2048.  Shorter rows would leave most of a wave
+// idle, longer ones do not fit its registers.
+constexpr int kTreeRowsMin = 32, kTreeRowsMax = 2048;
+// Longest rows of k_mf_rows, beside k_mf_scan and k_mf_box, without and with
+// maps: the same grids take 253 us against 371 at 64 samples, 308 against 458 at
+// 128, 1256 against 1487 at 1000, 2783 against 3221 at 2048 without; with maps
+// 629 against 742 at 512 but 1092 against 1090 at 700 and 1643 against 1515 at
+// 1000 (too few rows fit LDS, and a width needs two reads a sample).
+constexpr int kMfRowsMax = 2048, kMfMapsMax = 512;
+// Bytes of LDS per k_mf_rows workgroup: three to a CU (512 samples, 256 cutouts:
+// 824 us; four to a CU 843, two 939).
+constexpr int kMfRowsLds = 52 * 1024;
 
 // include/candidate.h:116-119, no contraction (the reference computes it as written)
 __device__ __host__ inline double dmdelay(double dm, double fh, double fl)
@@ -193,6 +217,133 @@ __global__ __launch_bounds__(256) void k_tree_pass(TreeArgs A)
     }
 }
 
+// The same pass for rows of at most 64*U samples: a wave takes whole row pairs,
+// U columns a lane, all of a pair's reads in registers before its two rows
+// are written, so that the levels need one barrier each; the shifts of every
+// level are formed together at the start (their FP64 divisions are a long
+// chain, which each level used to wait for); rows go out 16 bytes a lane where
+// ncol allows.  P2: ncol is a power of two, and a wrap is a mask.
+// 256 cutouts of 1024 x 512, five levels a pass: 258 us a pass, k_tree_pass 865;
+// 1.07 GB read and written, 216 us at a copy's rate, bounds it.
+template <int U, bool P2>
+__global__ __launch_bounds__(512) void k_tree_rows(TreeArgs A)
+{
+    extern __shared__ float rows[]; // [G][ncol], then the shifts: G a level (or G row delays)
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int c = blockIdx.y;
+    const int G = 1 << (A.b - A.a);
+    int *sh = (int *)(rows + (size_t)G * A.ncol);
+    const int g = (int)(blockIdx.x >> A.a), rho = (int)(blockIdx.x & ((1u << A.a) - 1));
+    const int ncol = A.ncol;
+
+    // ---- load the group's G rows, as k_tree_pass does
+    if (A.first) {
+        for (int t = tid; t < G; t += 512) {
+            const int q = A.srcrow[g * G + t];
+            int d = 0;
+            if (q >= 0 && A.dedisperse) {
+                d = (int)round(dmdelay(A.dmc[c], A.fmax, A.fsrc[q]) / A.tbin);
+                d %= ncol;
+                if (d < 0) d += ncol;
+            }
+            sh[t] = d;
+        }
+        __syncthreads();
+        const float *cut = A.src + (size_t)c * A.nchan * ncol;
+        for (int t = wave; t < G; t += 8) {
+            const int q = A.srcrow[g * G + t];
+            float *dst = rows + (size_t)t * ncol;
+            if (q < 0) {
+                for (int i = lane; i < ncol; i += 64) dst[i] = 0.f;
+                continue;
+            }
+            const int d = sh[t]; // the row rotated left by d: [d, ncol) then [0, d)
+            const uint32_t *srow = (const uint32_t *)(cut + (size_t)q * ncol);
+            lds_fill(srow + d, (uint32_t *)dst, ncol - d, 0, 1, lane);
+            if (d) lds_fill(srow, (uint32_t *)dst + (ncol - d), d, 0, 1, lane);
+        }
+        __syncthreads(); // sh is free again
+    } else {
+        const float *in = A.src + (size_t)c * A.nrow * ncol;
+        for (int t = wave; t < G; t += 8)
+            lds_fill((const uint32_t *)(in + ((size_t)(g * G + t) * (1 << A.a) + rho) * ncol),
+                     (uint32_t *)(rows + (size_t)t * ncol), ncol, 0, 1, lane);
+    }
+    const int pairs = G / 2;
+    const double dms = A.dms[c], ddm = A.ddm[c], dm0 = A.dm0[c];
+    for (int e = tid; e < (A.b - A.a) * 2 * pairs; e += 512) {
+        const int l = A.a + e / (2 * pairs), q = (e % (2 * pairs)) >> 1;
+        const int hs = l - A.a, jl = q >> hs, t = q & ((1 << hs) - 1);
+        const int jg = (g << (A.b - l - 1)) + jl;
+        const int x0 = jg << (l + 1), x1 = x0 + (1 << l);
+        const int k = rho + (t << A.a) + ((e & 1) << l);
+        sh[e] = tree_shift(A.fP[x0], A.fP[x1], bitrev(k, A.n), dms, ddm, dm0, A.tbin, ncol);
+    }
+    lds_fill_done();
+
+    // ---- levels a .. b-1, in place
+    for (int l = A.a; l < A.b; l++) {
+        const int hs = l - A.a, half = 1 << hs;
+        for (int q = wave; q < pairs; q += 8) {
+            const int jl = q >> hs, t = q & (half - 1);
+            float *Ar = rows + (size_t)(2 * jl * half + t) * ncol;
+            float *Br = Ar + (size_t)half * ncol;
+            const int s0 = sh[hs * 2 * pairs + 2 * q], s1 = sh[hs * 2 * pairs + 2 * q + 1];
+            float av[U], b0[U], b1[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int i = lane + 64 * u;
+                int i0 = i + s0, i1 = i + s1;
+                if (P2) {
+                    i0 &= ncol - 1;
+                    i1 &= ncol - 1;
+                } else {
+                    i0 -= i0 >= ncol ? ncol : 0;
+                    i1 -= i1 >= ncol ? ncol : 0;
+                }
+                if (64 * U == ncol || i < ncol) {
+                    av[u] = Ar[i];
+                    b0[u] = Br[i0];
+                    b1[u] = Br[i1];
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int i = lane + 64 * u;
+                if (64 * U == ncol || i < ncol) {
+                    Ar[i] = av[u] + b0[u];
+                    Br[i] = av[u] + b1[u];
+                }
+            }
+        }
+        __syncthreads();
+    }
+
+    // ---- store: node layout, or DM order after the last level
+    float *out = A.dst + (size_t)c * A.nrow * ncol;
+    for (int t = wave; t < G; t += 8) {
+        const int k = rho + (t << A.a);
+        const int r = A.last ? bitrev(k, A.n) : g * (1 << A.b) + k;
+        const float *row = rows + (size_t)t * ncol;
+        float *o = out + (size_t)r * ncol;
+        if (ncol % 4 == 0 && ((uintptr_t)A.dst & 15) == 0) {
+            for (int i = 4 * lane; i < ncol; i += 256) *(float4 *)(o + i) = *(const float4 *)(row + i);
+        } else {
+            for (int i = lane; i < ncol; i += 64) o[i] = row[i];
+        }
+    }
+}
+
+auto tree_rows_kernel(int ncol) -> void (*)(TreeArgs)
+{
+    const bool p2 = (ncol & (ncol - 1)) == 0;
+    if (ncol <= 128) return p2 ? k_tree_rows<2, true> : k_tree_rows<2, false>;
+    if (ncol <= 256) return p2 ? k_tree_rows<4, true> : k_tree_rows<4, false>;
+    if (ncol <= 512) return p2 ? k_tree_rows<8, true> : k_tree_rows<8, false>;
+    if (ncol <= 1024) return p2 ? k_tree_rows<16, true> : k_tree_rows<16, false>;
+    return p2 ? k_tree_rows<32, true> : k_tree_rows<32, false>;
+}
+
 struct MfArgs {
     const float *dmt; // [rows][ncol]
     float *cs;        // [rows][2*ncol] circular running sums
@@ -205,6 +356,7 @@ struct MfArgs {
     int nbox;
     long nrows;
     int ncol;
+    const int *pick; // workgroup c takes row pick[c] of cutout c (nrows per cutout); else null
 };
 
 // Sequential parts of matched_filter: one 64-lane workgroup per 64 DM rows,
@@ -348,6 +500,259 @@ __global__ __launch_bounds__(256) void k_mf_box(MfArgs M)
     }
 }
 
+// Both parts in one kernel for rows short enough that a workgroup holds a few
+// of them in LDS: the running sums (2*ncol a row, written and read back between
+// the two kernels) never leave the chip.  A width needs samples j and j + wn of
+// the doubled row for every j < ncol, so the sums end at ncol + W, W the widest
+// width (rounded up to 4 words with V4), and a row is ncol + W words: it is
+// loaded with its first W samples behind the others, where the second lap finds
+// them, and the sums take the samples' places.  One wave forms the rows' means
+// and another their mean squares at the same time, a lane a row; the first then
+// runs the sums, and the four waves take the rows' widths, 64*CU samples at a
+// time.  256 cutouts of 1024 x 512 without maps: 824 us and 38 us for the 256
+// best rows, k_mf_scan and k_mf_box 684 + 1031.  The chains of FP64 conversions
+// and adds bound it (three a CU, as many as LDS has room for: 305 us without
+// them, 585 without the widths).
+struct MfRow {
+    int nrows;  // rows per workgroup
+    int pitch;  // words from row to row: odd, or an odd multiple of 4 with V4
+    int W;
+    int nchunk; // pieces of 64*CU samples
+};
+
+// f(i, the four samples from i) for i = 0, 4, ... of a run of LDS, read 16
+// ahead (the compiler would put each read before its use, and the wave wait).
+template <typename F> __device__ __forceinline__ void mf_walk4(const float *x, int len, F f)
+{
+    if (len <= 0) return;
+    f4v nx[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) nx[q] = lds_f4(x + min(4 * q, len - 4));
+    for (int i = 0; i < len; i += 16) {
+        f4v cur[4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            cur[q] = nx[q];
+            nx[q] = lds_f4(x + min(i + 16 + 4 * q, len - 4));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+            if (i + 4 * q < len) f(i + 4 * q, cur[q]);
+    }
+}
+
+// Sequential FP64 sum of the samples (SQ: of their squares).
+template <bool V4, bool SQ> __device__ __forceinline__ void mf_sum(const float *x, int len, double &acc)
+{
+    auto step = [&](float f) {
+        const double d = (double)f;
+        acc = SQ ? fma(d, d, acc) : acc + d;
+    };
+    if (V4) {
+        mf_walk4(x, len, [&](int, f4v c) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) step(c[e]);
+        });
+    } else {
+#pragma unroll 8
+        for (int i = 0; i < len; i++) step(x[i]);
+    }
+}
+
+// csump: (double)csum + (x - mean), rounded to float each step.
+template <bool V4> __device__ __forceinline__ void mf_csum(const float *x, float *out, int len, double m, float &csum)
+{
+    auto step = [&](float f) { return csum = (float)((double)csum + ((double)f - m)); };
+    if (V4) {
+        mf_walk4(x, len, [&](int i, f4v c) {
+            f4v o;
+#pragma unroll
+            for (int e = 0; e < 4; e++) o[e] = step(c[e]);
+            *(f4v *)__builtin_assume_aligned(out + i, 16) = o;
+        });
+    } else {
+        float nx[8];
+#pragma unroll
+        for (int q = 0; q < 8; q++) nx[q] = x[min(q, len - 1)];
+        for (int i = 0; i < len; i += 8) {
+            float cur[8];
+#pragma unroll
+            for (int q = 0; q < 8; q++) {
+                cur[q] = nx[q];
+                nx[q] = x[min(i + 8 + q, len - 1)];
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int q = 0; q < 8; q++)
+                if (i + q < len) out[i + q] = step(cur[q]);
+        }
+    }
+}
+
+template <int CU, bool V4, bool MAPS>
+__global__ __launch_bounds__(256) void k_mf_rows(MfArgs M, MfRow T)
+{
+    extern __shared__ float smem[];
+    __shared__ double smean[64], svar[64];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int ncol = M.ncol, W = T.W;
+    const long R0 = M.pick ? (long)blockIdx.x * M.nrows + M.pick[blockIdx.x] : (long)blockIdx.x * T.nrows;
+    // the waves of a workgroup go to the four SIMDs in order: the workgroups of
+    // a CU (256 apart) run their chains on different ones
+    const int chain = (blockIdx.x >> 8) & 3;
+    const int nr = M.pick ? 1 : (int)min((long)T.nrows, M.nrows - R0);
+    for (int t = wave; t < nr; t += 4) {
+        const uint32_t *x = (const uint32_t *)(M.dmt + (R0 + t) * ncol);
+        uint32_t *B = (uint32_t *)(smem + t * T.pitch);
+        if (V4) {
+            lds_fill16(x, B + ncol, W, 0, 1, lane);
+            lds_fill16(x + W, B + W, ncol - W, 0, 1, lane);
+        } else {
+            lds_fill(x, B + ncol, W, 0, 1, lane);
+            lds_fill(x + W, B + W, ncol - W, 0, 1, lane);
+        }
+    }
+    lds_fill_done();
+    float *row = smem + lane * T.pitch;
+    if (wave == chain && lane < nr) {
+        double m = 0.;
+        mf_sum<V4, false>(row + ncol, W, m);
+        mf_sum<V4, false>(row + W, ncol - W, m);
+        smean[lane] = m / ncol;
+    } else if (wave == (chain ^ 1) && lane < nr) {
+        double v = 0.;
+        mf_sum<V4, true>(row + ncol, W, v);
+        mf_sum<V4, true>(row + W, ncol - W, v);
+        svar[lane] = v / ncol;
+    }
+    __syncthreads();
+    if (wave == chain && lane < nr) {
+        const double m = smean[lane];
+        float csum = 0.f;
+        mf_csum<V4>(row + ncol, row, W, m, csum);
+        mf_csum<V4>(row + W, row + W, ncol - W, m, csum);
+        mf_csum<V4>(row + ncol, row + ncol, W, m, csum);
+        svar[lane] = fma(-m, m, svar[lane]);
+    }
+    __syncthreads();
+    const int nbox = M.nbox;
+    // every row's scales: row t's at scale[64*t]
+    float *scale = smem + (size_t)T.nrows * T.pitch + 64 * CU * T.nchunk;
+    for (int e = threadIdx.x; e < nr * nbox; e += 256) {
+        const int t = e / nbox, k = e - t * nbox;
+        scale[64 * t + k] = (float)sqrt(1. / (M.vwn[k] * svar[t]));
+    }
+    __syncthreads();
+    if (MAPS) {
+        for (int t = wave; t < nr; t += 4) {
+            const long r = R0 + t;
+            const float *B = smem + t * T.pitch;
+            float best = -INFINITY;
+            int bo = 0x7fffffff, bw = 0;
+            for (int h = 0; h < T.nchunk; h++) {
+                float vS[CU];
+                int vW[CU];
+#pragma unroll
+                for (int u = 0; u < CU; u++) {
+                    vS[u] = 0.f;
+                    vW[u] = 0;
+                }
+                const int h0 = h * 64 * CU + lane;
+                if (svar[t] > 0)
+                    for (int k = 0; k < nbox; k++) {
+                        const int wn = ldc(M.vwn, k), wl = wn / 2 + 1, wh = (wn - 1) / 2;
+                        const float temp = scale[64 * t + k];
+#pragma unroll
+                        for (int u = 0; u < CU; u++) {
+                            const int o = min(h0 + 64 * u, ncol - 1);
+                            const int i = o >= wl ? o : o + ncol;
+                            const float S = (B[i + wh] - B[i - wl]) * temp;
+                            if (S >= vS[u]) {
+                                vS[u] = S;
+                                vW[u] = wn;
+                            }
+                        }
+                    }
+#pragma unroll
+                for (int u = 0; u < CU; u++) {
+                    const int o = h0 + 64 * u;
+                    if (o < ncol) {
+                        if (M.snr) M.snr[r * ncol + o] = vS[u];
+                        if (M.wid) M.wid[r * ncol + o] = vW[u];
+                        if (vS[u] > best) {
+                            best = vS[u];
+                            bo = o;
+                            bw = vW[u];
+                        }
+                    }
+                }
+            }
+            // first maximum of the row: larger value, then smaller sample
+            const float rb = wave_max_f(best);
+            const int first = wave_min_i(best == rb ? bo : 0x7fffffff);
+            if (bo == first) {
+                const long w = M.pick ? blockIdx.x : r;
+                if (!M.pick) M.rowmax[r] = rb;
+                M.rowarg[w] = bo;
+                M.rowwid[w] = bw;
+            }
+        }
+        return;
+    }
+    // Without maps only a row's largest S/N is wanted (its time and width only
+    // for each cutout's best row, which is then taken once more).  A width's
+    // largest S/N is its largest difference times the scale (both roundings
+    // keep the order, and a NaN never counts), so the scale is applied once a
+    // lane; sample j of a width belongs to time (j + wl) mod ncol, and B[j]
+    // serves every width.
+    for (int t = wave; t < nr; t += 4) {
+        const float *B = smem + t * T.pitch;
+        float best = 0.f;
+        if (svar[t] > 0) {
+            const float *sc = scale + 64 * t;
+            for (int h = 0; h < T.nchunk; h++) {
+                const int j0 = h * 64 * CU + lane;
+                float c0[CU];
+#pragma unroll
+                for (int u = 0; u < CU; u++) c0[u] = j0 + 64 * u < ncol ? B[j0 + 64 * u] : INFINITY;
+                for (int k = 0; k < nbox; k += 2) {
+                    const int k2 = min(k + 1, nbox - 1);
+                    const float *B1 = B + j0 + ldc(M.vwn, k), *B2 = B + j0 + ldc(M.vwn, k2);
+                    const float t1 = sc[k], t2 = sc[k2];
+                    float c1[CU], c2[CU], d1 = -INFINITY, d2 = -INFINITY;
+#pragma unroll
+                    for (int u = 0; u < CU; u++) c1[u] = B1[64 * u];
+#pragma unroll
+                    for (int u = 0; u < CU; u++) c2[u] = B2[64 * u];
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int u = 0; u < CU; u++) d1 = fmaxf(d1, c1[u] - c0[u]);
+#pragma unroll
+                    for (int u = 0; u < CU; u++) d2 = fmaxf(d2, c2[u] - c0[u]);
+                    best = fmaxf(best, fmaxf(d1 * t1, d2 * t2));
+                }
+            }
+        }
+        best = wave_max_f(best);
+        if (lane == 0) M.rowmax[R0 + t] = best;
+    }
+}
+
+template <bool V4, bool MAPS> auto mf_rows_kernel(int cu) -> void (*)(MfArgs, MfRow)
+{
+    switch (cu) {
+    case 1: return k_mf_rows<1, V4, MAPS>;
+    case 2: return k_mf_rows<2, V4, MAPS>;
+    case 3: return k_mf_rows<3, V4, MAPS>;
+    case 4: return k_mf_rows<4, V4, MAPS>;
+    case 5: return k_mf_rows<5, V4, MAPS>;
+    case 6: return k_mf_rows<6, V4, MAPS>;
+    case 7: return k_mf_rows<7, V4, MAPS>;
+    default: return k_mf_rows<8, V4, MAPS>;
+    }
+}
+
 __global__ __launch_bounds__(256) void k_argmax(const float *rowmax, const int *rowarg,
                                                 const int *rowwid, int nrow, int *odm, int *ot,
                                                 float *os, int *ow)
@@ -381,9 +786,11 @@ __global__ __launch_bounds__(256) void k_argmax(const float *rowmax, const int *
     if (tid == 0) {
         const int j = sj[0];
         odm[c] = j;
-        ot[c] = rowarg[(size_t)c * nrow + j];
         os[c] = sv[0];
-        ow[c] = rowwid[(size_t)c * nrow + j];
+        if (rowarg) {
+            ot[c] = rowarg[(size_t)c * nrow + j];
+            ow[c] = rowwid[(size_t)c * nrow + j];
+        }
     }
 }
 
@@ -500,6 +907,9 @@ extern "C" int tx_refine_create(const tx_refine_desc *d, int max_batch, tx_refin
     }
     (void)hipFuncSetAttribute((const void *)k_tree_pass, hipFuncAttributeMaxDynamicSharedMemorySize,
                               kTreeLdsFloats * 4);
+    if (d->nbin >= kTreeRowsMin && d->nbin <= kTreeRowsMax)
+        (void)hipFuncSetAttribute((const void *)tree_rows_kernel(d->nbin), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  kTreeLdsFloats * 4 + 10 * 1024 * 4);
     const size_t B = (size_t)max_batch, rowsz = (size_t)nrow * d->nbin;
     bool ok = hipStreamCreate(&r->stream) == hipSuccess &&
               hipMalloc(&r->d_fP, nrow * sizeof(double)) == hipSuccess &&
@@ -509,7 +919,7 @@ extern "C" int tx_refine_create(const tx_refine_desc *d, int max_batch, tx_refin
               hipMalloc(&r->d_vwn, kMaxMfBox * sizeof(int)) == hipSuccess &&
               hipMalloc(&r->d_t1, B * rowsz * 4) == hipSuccess &&
               hipMalloc(&r->d_t2, B * rowsz * 4) == hipSuccess &&
-              hipMalloc(&r->d_cs, 2 * B * rowsz * 4) == hipSuccess &&
+              (d->nbin <= kMfMapsMax || hipMalloc(&r->d_cs, 2 * B * rowsz * 4) == hipSuccess) &&
               hipMalloc(&r->d_rowmax, B * nrow * 4) == hipSuccess &&
               hipMalloc(&r->d_rowarg, B * nrow * 4) == hipSuccess &&
               hipMalloc(&r->d_rowwid, B * nrow * 4) == hipSuccess &&
@@ -615,7 +1025,12 @@ extern "C" int tx_refine_run(tx_refiner *r, int ncand, const float *cutouts, con
             A.dst = dst;
             const int G = 1 << (A.b - A.a);
             dim3 grid((unsigned)((nrow >> A.b) << A.a), (unsigned)nc);
-            hipLaunchKernelGGL(k_tree_pass, grid, dim3(256), (size_t)G * nbin * 4, r->stream, A);
+            const size_t shm = (size_t)G * nbin * 4;
+            const size_t sht = (size_t)(A.b - A.a) * G * 4;
+            if (nbin >= kTreeRowsMin && nbin <= kTreeRowsMax)
+                hipLaunchKernelGGL(tree_rows_kernel(nbin), grid, dim3(512), shm + sht, r->stream, A);
+            else
+                hipLaunchKernelGGL(k_tree_pass, grid, dim3(256), shm, r->stream, A);
             RCHK(hipGetLastError());
             src = dst;
         }
@@ -632,24 +1047,63 @@ extern "C" int tx_refine_run(tx_refiner *r, int ncand, const float *cutouts, con
         M.nbox = (int)r->vwn.size();
         M.nrows = (long)nc * nrow;
         M.ncol = nbin;
-        hipLaunchKernelGGL(k_mf_scan, dim3((unsigned)((M.nrows + 63) / 64)), dim3(64), 64 * 65 * 4,
-                           r->stream, M);
-        RCHK(hipGetLastError());
-        const size_t shm = 4 * 2 * (size_t)nbin * 4;
-        const dim3 mg((unsigned)((M.nrows + 3) / 4));
-        if (nbin <= 512)
-            hipLaunchKernelGGL(k_mf_box<8>, mg, dim3(256), shm, r->stream, M);
-        else if (nbin <= 1024)
-            hipLaunchKernelGGL(k_mf_box<16>, mg, dim3(256), shm, r->stream, M);
-        else if (nbin <= 2048)
-            hipLaunchKernelGGL(k_mf_box<32>, mg, dim3(256), shm, r->stream, M);
-        else
-            hipLaunchKernelGGL(k_mf_box<64>, mg, dim3(256), shm, r->stream, M);
-        RCHK(hipGetLastError());
-        hipLaunchKernelGGL(k_argmax, dim3((unsigned)nc), dim3(256), 0, r->stream, r->d_rowmax,
-                           r->d_rowarg, r->d_rowwid, nrow, r->d_res_i, r->d_res_i + r->batch, r->d_res_s,
-                           r->d_res_i + 2 * r->batch);
-        RCHK(hipGetLastError());
+        M.pick = nullptr;
+        bool picked = false; // the results' times and widths are there
+        const bool maps = M.snr || M.wid;
+        if (nbin <= (maps ? kMfMapsMax : kMfRowsMax)) {
+            const bool v4 = nbin % 4 == 0 && ((uintptr_t)dmt_out & 15) == 0;
+            const int nu = (nbin + 63) / 64;
+            MfRow T;
+            T.nchunk = (nu + 7) / 8;
+            const int cu = (nu + T.nchunk - 1) / T.nchunk;
+            T.W = v4 ? (r->vwn.back() + 3) / 4 * 4 : r->vwn.back();
+            T.pitch = v4 ? ((nbin + T.W) / 4 | 1) * 4 : (nbin + T.W) | 1;
+            T.nrows = std::max(1, std::min(64, (kMfRowsLds / 4 - 64 * cu * T.nchunk) / (T.pitch + 64)));
+            // reads past a row's last sample (whose results do not count) stay in the allocation
+            const auto shm = [&] { return ((size_t)T.nrows * (T.pitch + 64) + 64 * cu * T.nchunk) * 4; };
+            auto kernel = [&](bool m) {
+                return v4 ? (m ? mf_rows_kernel<true, true>(cu) : mf_rows_kernel<true, false>(cu))
+                          : (m ? mf_rows_kernel<false, true>(cu) : mf_rows_kernel<false, false>(cu));
+            };
+            hipLaunchKernelGGL(kernel(maps), dim3((unsigned)((M.nrows + T.nrows - 1) / T.nrows)), dim3(256), shm(),
+                               r->stream, M, T);
+            RCHK(hipGetLastError());
+            if (!maps) {
+                hipLaunchKernelGGL(k_argmax, dim3((unsigned)nc), dim3(256), 0, r->stream, r->d_rowmax,
+                                   (const int *)nullptr, (const int *)nullptr, nrow, r->d_res_i,
+                                   r->d_res_i + r->batch, r->d_res_s, r->d_res_i + 2 * r->batch);
+                RCHK(hipGetLastError());
+                picked = true;
+                M.pick = r->d_res_i;
+                M.nrows = nrow;
+                M.rowarg = r->d_res_i + r->batch;
+                M.rowwid = r->d_res_i + 2 * r->batch;
+                T.nrows = 1;
+                hipLaunchKernelGGL(kernel(true), dim3((unsigned)nc), dim3(256), shm(), r->stream, M, T);
+                RCHK(hipGetLastError());
+            }
+        } else {
+            hipLaunchKernelGGL(k_mf_scan, dim3((unsigned)((M.nrows + 63) / 64)), dim3(64), 64 * 65 * 4,
+                               r->stream, M);
+            RCHK(hipGetLastError());
+            const size_t shm = 4 * 2 * (size_t)nbin * 4;
+            const dim3 mg((unsigned)((M.nrows + 3) / 4));
+            if (nbin <= 512)
+                hipLaunchKernelGGL(k_mf_box<8>, mg, dim3(256), shm, r->stream, M);
+            else if (nbin <= 1024)
+                hipLaunchKernelGGL(k_mf_box<16>, mg, dim3(256), shm, r->stream, M);
+            else if (nbin <= 2048)
+                hipLaunchKernelGGL(k_mf_box<32>, mg, dim3(256), shm, r->stream, M);
+            else
+                hipLaunchKernelGGL(k_mf_box<64>, mg, dim3(256), shm, r->stream, M);
+            RCHK(hipGetLastError());
+        }
+        if (!picked) {
+            hipLaunchKernelGGL(k_argmax, dim3((unsigned)nc), dim3(256), 0, r->stream, r->d_rowmax,
+                               r->d_rowarg, r->d_rowwid, nrow, r->d_res_i, r->d_res_i + r->batch, r->d_res_s,
+                               r->d_res_i + 2 * r->batch);
+            RCHK(hipGetLastError());
+        }
         std::vector<int> ri(3 * (size_t)r->batch);
         std::vector<float> rs(r->batch);
         RCHK(hipMemcpyAsync(ri.data(), r->d_res_i, ri.size() * 4, hipMemcpyDeviceToHost, r->stream));
