@@ -418,3 +418,49 @@ def test_gradient_refinement_at_the_refinement_workload():
     assert njev >= 10 * nev
     assert np.mean(close | tie) >= 0.99
     assert np.mean(close) >= 0.95
+
+
+@pytest.mark.parametrize("nchan,nbin", [
+    (1, 64), (3, 65), (5, 127), (17, 128), (18, 129), (33, 255), (30, 257), (31, 384), (32, 385), (15, 511),
+    (9, 513), (16, 768), (7, 769), (8, 1024), (9, 1025), (6, 2048), (5, 2049)])
+def test_row_lengths_and_few_channels(nchan, nbin):
+    """Row lengths around every change of samples per lane, and channel counts
+    that leave waves without a channel or with a ragged last step: S and every
+    gradient, with and without dS/dw, against the FP64 restatement."""
+    import torch
+
+    from transientx_amd.diff import DiffSNR
+
+    f, x, w, dm, t0, W, kf, tbin = make(nbin, 2, nchan=nchan, nbin=nbin)
+    w[:, 0] = 1.0
+    say("case nchan", nchan, "nbin", nbin)
+    m = DiffSNR(f, nbin, tbin, softness=1.0)
+    try:
+        xt, wt = torch.from_numpy(x).cuda(), torch.from_numpy(w).cuda()
+        F = lambda v: torch.tensor(v, dtype=torch.float32, device="cuda")
+        one = torch.ones(2, device="cuda")
+        snr, gdm, gt0, gwd, gw, _ = (v if v is None else v.cpu().numpy()
+                                     for v in m.adjoint(xt, wt, F(dm), F(t0), F(W), one))
+        gdm2 = m.adjoint(xt, wt, F(dm), F(t0), F(W), one, need_w=False)[1].cpu().numpy()
+        assert np.array_equal(snr, m.forward(xt, wt, F(dm), F(t0), F(W)).cpu().numpy())
+    finally:
+        m.close()
+    xd, wd = x.astype(np.float64), w.astype(np.float64)
+    for c in range(2):
+        args = [np.float64(np.float32(v[c])) for v in (dm, t0, W)]
+        s64 = snr64(xd[c], wd[c], *args, kf, 1.0)
+        assert abs(snr[c] - s64) <= 2e-5 * max(1.0, abs(s64)), (c, snr[c], s64)
+        for k, (got, h) in enumerate(((gdm[c], 1e-6), (gt0[c], 1e-5), (gwd[c], 1e-5))):
+            a1, a2 = list(args), list(args)
+            a1[k] += h
+            a2[k] -= h
+            ref = (snr64(xd[c], wd[c], *a1, kf, 1.0) - snr64(xd[c], wd[c], *a2, kf, 1.0)) / (2 * h)
+            assert abs(got - ref) <= 2e-3 * abs(ref) + 2e-3, (c, k, got, ref)
+            if k == 0:
+                assert abs(gdm2[c] - ref) <= 2e-3 * abs(ref) + 2e-3, (c, gdm2[c], ref)
+        for j in range(nchan):
+            w1, w2 = wd[c].copy(), wd[c].copy()
+            w1[j] += 1e-6
+            w2[j] -= 1e-6
+            ref = (snr64(xd[c], w1, *args, kf, 1.0) - snr64(xd[c], w2, *args, kf, 1.0)) / 2e-6
+            assert abs(gw[c, j] - ref) <= 2e-3 * abs(ref) + 2e-4, (c, j, gw[c, j], ref)

@@ -29,6 +29,7 @@ int set_error(int code, const std::string &msg);
 }
 using txgpu::set_error;
 using txgpu::wave_sum_d;
+using txgpu::wave_total_d;
 
 namespace {
 
@@ -69,6 +70,66 @@ __device__ inline double block_sum_d(double v, double *sh)
     return ((sh[0] + sh[1]) + sh[2]) + sh[3];
 }
 
+// f(j, w_j, x0, x1) for the channels j = wave, wave + 4, ... in order: lane l
+// gets x0[u] = X_j[(t + d_j) mod nbin] and x1[u], the sample after it, for
+// t = l + 64*u.  Few workgroups share a CU here, so that a channel's weight and
+// row, waited for one after the other, were all the time went to: the rows of
+// the next NB channels (and their weights, through the scalar cache) are
+// fetched before the current ones are used, and x1 comes from the neighbouring
+// lane (wave_shl:1; lane 63's is lane 0's of the next u).  512 evaluations of
+// 1024 x 512: forward 202 us (1069), with the adjoint 505 us (2229).  A
+// pass over the 1.07 GB: at 5.3 and 4.2 TB/s the memory bounds both.
+template <int U, typename F>
+__device__ __forceinline__ void channel_rows(const float *X, const float *W, const int *sd, int nchan, int nbin,
+                                             int lane, int wave, F f)
+{
+    constexpr int NB = U <= 8 ? 4 : U <= 16 ? 2 : 1;
+    typedef __attribute__((address_space(4))) const float const_float_t;
+    const int n = (nchan - wave + 3) / 4;
+    if (n <= 0) return;
+    float nx[NB][U], nw[NB];
+    auto fetch = [&](int s, float (&v)[U], float &w) {
+        const int j = wave + 4 * min(s, n - 1);
+        w = ((const_float_t *)W)[j];
+        const int d = __builtin_amdgcn_readfirstlane(sd[j]);
+        const float *row = X + (size_t)j * nbin;
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            int i0 = min(lane + 64 * u, nbin - 1) + d;
+            if (i0 >= nbin) i0 -= nbin;
+            v[u] = row[i0];
+        }
+    };
+#pragma unroll
+    for (int b = 0; b < NB; b++) fetch(b, nx[b], nw[b]);
+    for (int s = 0; s < n; s += NB) {
+        float x0[NB][U], w[NB];
+#pragma unroll
+        for (int b = 0; b < NB; b++) {
+            w[b] = nw[b];
+#pragma unroll
+            for (int u = 0; u < U; u++) x0[b][u] = nx[b][u];
+        }
+#pragma unroll
+        for (int b = 0; b < NB; b++) fetch(s + NB + b, nx[b], nw[b]);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int b = 0; b < NB; b++) {
+            if (s + b >= n) break;
+            float x1[U];
+            const int first = __builtin_amdgcn_readfirstlane(__float_as_int(x0[b][0]));
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int after = __builtin_amdgcn_readfirstlane(__float_as_int(x0[b][(u + 1) % U]));
+                const int nb =
+                    __builtin_amdgcn_update_dpp(after, __float_as_int(x0[b][u]), 0x130, 0xF, 0xF, false);
+                x1[u] = __int_as_float(lane + 64 * u == nbin - 1 ? first : nb);
+            }
+            f(wave + 4 * (s + b), w[b], x0[b], x1);
+        }
+    }
+}
+
 // One 256-thread workgroup per evaluation; U samples per lane (nbin <= 64*U).
 template <int U, bool ADJ>
 __global__ __launch_bounds__(256) void k_diff(DiffArgs A)
@@ -81,7 +142,7 @@ __global__ __launch_bounds__(256) void k_diff(DiffArgs A)
     // logical order: consecutive evaluations (which share a cutout) on one
     // XCD, so the cutout is fetched into one L2 rather than eight
     const int e = (int)txgpu::xcd_logical(blockIdx.x, gridDim.x);
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int nbin = A.nbin, nchan = A.nchan;
     const int c = A.cand ? A.cand[e] : e;
     const float *X = A.x + (size_t)c * nchan * nbin;
@@ -102,23 +163,12 @@ __global__ __launch_bounds__(256) void k_diff(DiffArgs A)
     float acc[U];
 #pragma unroll
     for (int u = 0; u < U; u++) acc[u] = 0.f;
-    for (int j = wave; j < nchan; j += 4) {
-        const float wj = W[j];
-        if (wj == 0.f) continue;
+    channel_rows<U>(X, W, sd, nchan, nbin, lane, wave, [&](int j, float wj, const float(&x0)[U], const float(&x1)[U]) {
+        if (wj == 0.f) return;
         const float al = sa[j];
-        const int d = sd[j];
-        const float *row = X + (size_t)j * nbin;
 #pragma unroll
-        for (int u = 0; u < U; u++) {
-            const int t = lane + 64 * u;
-            if (t < nbin) {
-                int i0 = t + d;
-                if (i0 >= nbin) i0 -= nbin;
-                const int i1 = i0 + 1 < nbin ? i0 + 1 : 0;
-                acc[u] += wj * ((1.f - al) * row[i0] + al * row[i1]);
-            }
-        }
-    }
+        for (int u = 0; u < U; u++) acc[u] += wj * ((1.f - al) * x0[u] + al * x1[u]);
+    });
 #pragma unroll
     for (int u = 0; u < U; u++) {
         const int t = lane + 64 * u;
@@ -215,50 +265,33 @@ __global__ __launch_bounds__(256) void k_diff(DiffArgs A)
     double gdm_w = 0.;
     if (!A.gw && !A.gx) {
         double lacc = 0.;
-        for (int j = wave; j < nchan; j += 4) {
-            const float wj = W[j];
-            if (wj == 0.f) continue;
-            const int d = sd[j];
-            const float *row = X + (size_t)j * nbin;
-            double b = 0.;
+        channel_rows<U>(X, W, sd, nchan, nbin, lane, wave,
+                        [&](int j, float wj, const float(&x0)[U], const float(&x1)[U]) {
+                            if (wj == 0.f) return;
+                            double b = 0.;
 #pragma unroll
-            for (int u = 0; u < U; u++) {
-                const int t = lane + 64 * u;
-                if (t < nbin) {
-                    int i0 = t + d;
-                    if (i0 >= nbin) i0 -= nbin;
-                    const int i1 = i0 + 1 < nbin ? i0 + 1 : 0;
-                    b += (double)G[u] * (double)(row[i1] - row[i0]);
-                }
-            }
-            lacc += (double)wj * A.kf[j] * b;
-        }
+                            for (int u = 0; u < U; u++)
+                                if (lane + 64 * u < nbin) b += (double)G[u] * (double)(x1[u] - x0[u]);
+                            lacc += (double)wj * A.kf[j] * b;
+                        });
         gdm_w = wave_sum_d(lacc);
     } else
-    for (int j = wave; j < nchan; j += 4) {
-        const float wj = W[j];
+    channel_rows<U>(X, W, sd, nchan, nbin, lane, wave, [&](int j, float wj, const float(&x0)[U], const float(&x1)[U]) {
         const float al = sa[j];
-        const int d = sd[j];
-        const float *row = X + (size_t)j * nbin;
         double a = 0., b = 0.;
 #pragma unroll
-        for (int u = 0; u < U; u++) {
-            const int t = lane + 64 * u;
-            if (t < nbin) {
-                int i0 = t + d;
-                if (i0 >= nbin) i0 -= nbin;
-                const int i1 = i0 + 1 < nbin ? i0 + 1 : 0;
-                const float x0 = row[i0], x1 = row[i1];
-                a += (double)G[u] * (double)((1.f - al) * x0 + al * x1);
-                b += (double)G[u] * (double)(x1 - x0);
+        for (int u = 0; u < U; u++)
+            if (lane + 64 * u < nbin) {
+                a += (double)G[u] * (double)((1.f - al) * x0[u] + al * x1[u]);
+                b += (double)G[u] * (double)(x1[u] - x0[u]);
             }
-        }
-        a = wave_sum_d(a);
-        b = wave_sum_d(b);
+        a = wave_total_d(a);
+        b = wave_total_d(b);
         if (A.gw && lane == 0) A.gw[(size_t)e * nchan + j] = (float)(gs * (a - S * (double)wj / sw2));
         gdm_w += (double)wj * A.kf[j] * b; // identical on every lane
         if (A.gx) {
             // dS/dx_j[k] = w_j*((1-a_j)*G(k-d_j) + a_j*G(k-d_j-1))
+            const int d = sd[j];
             float *gxr = A.gx + ((size_t)e * nchan + j) * nbin;
             for (int k = lane; k < nbin; k += 64) {
                 int t0i = k - d;
@@ -267,7 +300,7 @@ __global__ __launch_bounds__(256) void k_diff(DiffArgs A)
                 gxr[k] = (float)gs * wj * ((1.f - al) * pw[t0i] + al * pw[t1i]);
             }
         }
-    }
+    });
     __syncthreads();
     if (lane == 0) shd[wave] = gdm_w;
     __syncthreads();
@@ -700,8 +733,17 @@ int launch_diff(hipStream_t st, const DiffArgs &A, int neval)
         void *p[] = {(void *)&A};
         (void)hipLaunchKernel(f, g, b, p, shm, st);
     };
-    if (A.nbin <= 512)
+    // steps small enough that few of a wave's reads go to lanes past the row's end
+    if (A.nbin <= 128)
+        go((const void *)k_diff<2, ADJ>);
+    else if (A.nbin <= 256)
+        go((const void *)k_diff<4, ADJ>);
+    else if (A.nbin <= 384)
+        go((const void *)k_diff<6, ADJ>);
+    else if (A.nbin <= 512)
         go((const void *)k_diff<8, ADJ>);
+    else if (A.nbin <= 768)
+        go((const void *)k_diff<12, ADJ>);
     else if (A.nbin <= 1024)
         go((const void *)k_diff<16, ADJ>);
     else if (A.nbin <= 2048)
