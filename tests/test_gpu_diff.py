@@ -464,3 +464,30 @@ def test_row_lengths_and_few_channels(nchan, nbin):
             w2[j] -= 1e-6
             ref = (snr64(xd[c], w1, *args, kf, 1.0) - snr64(xd[c], w2, *args, kf, 1.0)) / 2e-6
             assert abs(gw[c, j] - ref) <= 2e-3 * abs(ref) + 2e-4, (c, j, gw[c, j], ref)
+
+
+@pytest.mark.parametrize("nchan,nbin", [(3, 65), (18, 128), (17, 257), (33, 385), (9, 513), (7, 769), (6, 1025)])
+def test_grid_row_lengths(nchan, nbin):
+    """The grid at row lengths around every change of samples per lane: each
+    trial's best S against the largest of tx_refine_fwd's (the tolerance of
+    the brute-force test above)."""
+    import torch
+
+    from transientx_amd.diff import DiffSNR
+
+    f, x, w, dm, t0, W, kf, tbin = make(nbin, 2, nchan=nchan, nbin=nbin)
+    w[:, 0] = 1.0
+    m = DiffSNR(f, nbin, tbin, softness=1.0)
+    try:
+        xt, wt = torch.from_numpy(x).cuda(), torch.from_numpy(w).cuda()
+        F = lambda v: torch.tensor(np.asarray(v), dtype=torch.float32, device="cuda")
+        wd = np.float32([2.5, 6.0])
+        best = m.grid(xt, wt, F(dm), F(t0), 3, 0.5, 2, 1.0, F(wd))[0].cpu().numpy()
+        for r in range(3):
+            d = F(np.float32(dm) + np.float32(r) * np.float32(0.5))
+            s = [m.forward(xt, wt, d, F(np.float32(t0) + np.float32(i)), F(np.full(2, v))).cpu().numpy()
+                 for i in range(2) for v in wd]
+            top = np.max(s, axis=0)
+            assert np.all(np.abs(best[:, r] - top) <= 1e-4 * np.abs(top) + 1e-5), (r, best[:, r], top)
+    finally:
+        m.close()

@@ -77,7 +77,8 @@ __device__ inline double block_sum_d(double v, double *sh)
 // the next NB channels (and their weights, through the scalar cache) are
 // fetched before the current ones are used, and x1 comes from the neighbouring
 // lane (wave_shl:1; lane 63's is lane 0's of the next u).  512 evaluations of
-// 1024 x 512: forward 202 us (1069), with the adjoint 505 us (2229).  A
+// 1024 x 512: forward 202 us (1069), with the adjoint 505 us (2229);
+// k_dgrid, 128 cutouts and 9 DM trials of that size: 343 us (810).  A
 // pass over the 1.07 GB: at 5.3 and 4.2 TB/s the memory bounds both.
 template <int U, typename F>
 __device__ __forceinline__ void channel_rows(const float *X, const float *W, const int *sd, int nchan, int nbin,
@@ -593,7 +594,7 @@ __global__ __launch_bounds__(256) void k_dgrid(GridArgs A)
     float *sa = (float *)(sd + A.nchan);    // [nchan] its fraction
     const unsigned lid = txgpu::xcd_logical(blockIdx.x, gridDim.x);
     const int c = (int)(lid / A.ndm), m = (int)(lid % A.ndm);
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int nbin = A.nbin, nchan = A.nchan;
     const float *X = A.x + (size_t)c * nchan * nbin;
     const float *W = A.w + (size_t)c * nchan;
@@ -611,23 +612,12 @@ __global__ __launch_bounds__(256) void k_dgrid(GridArgs A)
     float acc[U];
 #pragma unroll
     for (int u = 0; u < U; u++) acc[u] = 0.f;
-    for (int j = wave; j < nchan; j += 4) {
-        const float wj = W[j];
-        if (wj == 0.f) continue;
+    channel_rows<U>(X, W, sd, nchan, nbin, lane, wave, [&](int j, float wj, const float(&x0)[U], const float(&x1)[U]) {
+        if (wj == 0.f) return;
         const float al = sa[j];
-        const int d = sd[j];
-        const float *row = X + (size_t)j * nbin;
 #pragma unroll
-        for (int u = 0; u < U; u++) {
-            const int t = lane + 64 * u;
-            if (t < nbin) {
-                int i0 = t + d;
-                if (i0 >= nbin) i0 -= nbin;
-                const int i1 = i0 + 1 < nbin ? i0 + 1 : 0;
-                acc[u] += wj * ((1.f - al) * row[i0] + al * row[i1]);
-            }
-        }
-    }
+        for (int u = 0; u < U; u++) acc[u] += wj * ((1.f - al) * x0[u] + al * x1[u]);
+    });
 #pragma unroll
     for (int u = 0; u < U; u++) {
         const int t = lane + 64 * u;
@@ -974,8 +964,17 @@ extern "C" int tx_refine_grid(tx_diff *r, int ncut, const float *x, const float 
         void *p[] = {(void *)&A};
         (void)hipLaunchKernel(f, g, b, p, shm, r->stream);
     };
-    if (A.nbin <= 512)
+    // as k_diff
+    if (A.nbin <= 128)
+        go((const void *)k_dgrid<2>);
+    else if (A.nbin <= 256)
+        go((const void *)k_dgrid<4>);
+    else if (A.nbin <= 384)
+        go((const void *)k_dgrid<6>);
+    else if (A.nbin <= 512)
         go((const void *)k_dgrid<8>);
+    else if (A.nbin <= 768)
+        go((const void *)k_dgrid<12>);
     else if (A.nbin <= 1024)
         go((const void *)k_dgrid<16>);
     else if (A.nbin <= 2048)
