@@ -97,9 +97,9 @@ def same_bits(a, b):
         np.where(nan, 0, a).view(np.uint32), np.where(nan, 0, b).view(np.uint32))
 
 
-# around the time-major kernels' edges: 32 channels a workgroup (31 takes the
-# general kernels, 33 overlaps two groups), 128 samples a chunk, 32 samples
-# and 128 channels a normalisation tile
+# around the time-major kernels' edges: 32 channels a workgroup (33 overlaps two
+# groups; below 32 zdot takes its narrow form and kadaneF the general kernels),
+# 128 samples a chunk, 32 samples and 128 channels a normalisation tile
 @pytest.mark.parametrize("nchan,nsamp,nf", [(31, 70, 1), (32, 128, 2), (33, 129, 1), (64, 1, 1), (95, 127, 1),
                                             (129, 257, 2), (300, 33, 1)])
 def test_time_major_zdot_and_kadanef_edges(nchan, nsamp, nf):
@@ -143,3 +143,58 @@ def test_channel_major_zdot_tiles(nchan, nbin, nf):
     g = torch.from_numpy(x).cuda()
     rfi.zdot(g, layout="channel")
     assert same_bits(g.cpu().numpy(), ref)
+
+
+# frames of fewer channels than a workgroup's 32 columns, around 128 samples a chunk
+@pytest.mark.parametrize("nchan,nsamp,nf", [(1, 1, 1), (1, 300, 2), (2, 127, 1), (3, 128, 3), (4, 129, 1),
+                                            (7, 257, 2), (16, 513, 1), (30, 33, 2), (31, 256, 1)])
+def test_time_major_zdot_of_few_channels(nchan, nsamp, nf):
+    import torch
+
+    from transientx_amd import rfi
+
+    say("case time-major nchan", nchan, "nsamp", nsamp, "frames", nf)
+    rng = np.random.default_rng(nchan * 1000 + nsamp)
+    x = (rng.normal(size=(nf, nchan, nsamp)) + rng.normal(size=(nf, 1, nsamp)) * 2).astype(np.float32)
+    if nchan > 3:
+        x[0, 1] = 5.0
+        x[0, 2, nsamp // 2] = np.nan
+    ref = np.stack([oracle.zdot(x[f]) for f in range(nf)])
+    # guard samples around the frames stay as they are
+    buf = torch.full((nf * nchan * nsamp + 8,), 7.0, device="cuda")
+    t = buf[4:-4].view(nf, nsamp, nchan)
+    t.copy_(torch.from_numpy(np.ascontiguousarray(x.transpose(0, 2, 1))))
+    rfi.zdot(t, layout="time")
+    assert same_bits(np.ascontiguousarray(t.cpu().numpy().transpose(0, 2, 1)), ref)
+    assert torch.all(buf[:4] == 7.0) and torch.all(buf[-4:] == 7.0)
+
+
+def duration(f, x0):
+    """Seconds of f on a fresh copy of x0: the shortest of seven runs."""
+    import time
+
+    import torch
+
+    best = np.inf
+    for _ in range(8):
+        x = x0.clone()
+        torch.cuda.synchronize()
+        t = time.perf_counter()
+        f(x)
+        torch.cuda.synchronize()
+        best = min(best, time.perf_counter() - t)
+    return best
+
+
+def test_few_channels_take_no_longer_than_more():
+    """A block of 31 channels takes what one of 32 does (the same chains; three
+    times is allowed, one lane per channel loading for itself took 20)."""
+    import torch
+
+    from transientx_amd import rfi
+
+    g = torch.Generator(device="cuda").manual_seed(3)
+    t = {c: duration(lambda x: rfi.zdot(x, layout="time"), torch.randn((26123, c), generator=g, device="cuda"))
+         for c in (31, 32)}
+    say("zdot of 26123 samples:", {c: round(1e6 * v) for c, v in t.items()}, "us")
+    assert t[31] <= 3 * t[32]

@@ -603,21 +603,29 @@ typedef float f4u __attribute__((ext_vector_type(4), aligned(4))); // 4-byte ali
 // The streaming part: chunks of kColT samples of 32 columns (ts floats from
 // sample to sample, N samples) pass through buf; put(k, v) of a helper
 // thread (h < 256) stores columns q4 .. q4 + 3 of its samples r0 + 32*u
-// of chunk k, chain(k) of wave 0 works on chunk k, buf half k & 1.
+// of chunk k, chain(k) of wave 0 works on chunk k, buf half k & 1.  NARROW:
+// only nc < 32 columns exist, the last one stands in for those past it.
 struct ColChunk {
     f4u v[4];
     double s;
 };
-template <class Put, class Chain>
+template <bool NARROW, class Put, class Chain>
 __device__ __forceinline__ void stream_columns(const float *__restrict__ col, const double *__restrict__ sf, long N,
-                                               long ts, Put put, Chain chain)
+                                               long ts, int nc, Put put, Chain chain)
 {
     const int tid = threadIdx.x, h = tid - 64, q4 = (h & 7) * 4, r0 = h >> 3;
     const int nk = (int)((N + kColT - 1) / kColT);
     auto load = [&](int k, ColChunk &c) { // past the end: a sample that exists, unused
         const long t0 = (long)k * kColT;
 #pragma unroll
-        for (int u = 0; u < 4; u++) c.v[u] = *(const f4u *)(col + min(t0 + r0 + 32 * u, N - 1) * ts + q4);
+        for (int u = 0; u < 4; u++) {
+            const float *row = col + min(t0 + r0 + 32 * u, N - 1) * ts;
+            if (NARROW)
+                c.v[u] = f4u{row[min(q4, nc - 1)], row[min(q4 + 1, nc - 1)], row[min(q4 + 2, nc - 1)],
+                             row[min(q4 + 3, nc - 1)]};
+            else
+                c.v[u] = *(const f4u *)(row + q4);
+        }
         if (sf) c.s = sf[min(t0 + (h & (kColT - 1)), N - 1)];
     };
     ColChunk A, B;
@@ -655,7 +663,10 @@ __device__ __forceinline__ void stream_columns(const float *__restrict__ col, co
 // extra workgroup per frame, sum s and sum s^2 into sess.  4096 channels x
 // 26,123 samples (428 MB): 177 us and 214 us, 16 and 20 cycles a sample; one
 // lane per channel loading for itself took 1.9 and 1.4 ms (with the update).
-template <bool FIT>
+// NARROW: frames of fewer than 32 channels, whose chains are as long: zdot of
+// 31 x 26,123 samples takes 407 us (32: 394), with one lane per channel 3.7 ms
+// where it keeps 32 loads in flight and 12.6 ms where it does not.
+template <bool FIT, bool NARROW>
 __global__ __launch_bounds__(kColThreads) void k_zdot_chain(Frames F, const double *__restrict__ s, double *stat,
                                                             double *sess)
 {
@@ -702,7 +713,8 @@ __global__ __launch_bounds__(kColThreads) void k_zdot_chain(Frames F, const doub
 
     // the last group ends at the last channel (the channels it shares with
     // the group before come out the same in both)
-    const int c0 = min(g * kColCh, F.nchan - kColCh);
+    const int c0 = NARROW ? 0 : min(g * kColCh, F.nchan - kColCh);
+    const int nc = NARROW ? F.nchan : kColCh;
     const int h = tid - 64, q4 = (h & 7) * 4, r0 = h >> 3;
     double acc = 0.;
     const int sel = lane >> 5;
@@ -736,11 +748,11 @@ __global__ __launch_bounds__(kColThreads) void k_zdot_chain(Frames F, const doub
                 acc = FIT ? fma((double)b[i * RS], mult[k & 1][i][sel], acc) : acc + (double)b[i * RS];
         }
     };
-    stream_columns(F.x + f * F.fstride + c0, FIT ? sf : nullptr, N, F.tstride, put, chain);
+    stream_columns<NARROW>(F.x + f * F.fstride + c0, FIT ? sf : nullptr, N, F.tstride, nc, put, chain);
     if (tid >= 64) return;
     double *out = stat + 2 * (f * F.nchan + c0);
     if (FIT) {
-        out[2 * ls + sel] = acc;
+        if (ls < nc) out[2 * ls + sel] = acc;
     } else {
         const double other = __shfl_xor(acc, 32, 64);
         const double m = acc / N;
@@ -748,7 +760,7 @@ __global__ __launch_bounds__(kColThreads) void k_zdot_chain(Frames F, const doub
         sd = fma(-m, m, sd); // tmpstd -= tmpmean*tmpmean
         sd = sqrt(sd);
         if (sd == 0.) sd = 1.;
-        if (lane < kColCh) {
+        if (lane < nc) {
             out[2 * lane] = m;
             out[2 * lane + 1] = sd;
         }
@@ -1022,7 +1034,7 @@ __global__ __launch_bounds__(kColThreads) void k_kad_scan_tm(int ncd, long nsd, 
             for (int i = 0; i < n; i++) p.step(i0 + i, sg, b[i * kColCh]);
         }
     };
-    stream_columns(ds + f * nsd * ncd + c0, nullptr, nsd, ncd, put, chain);
+    stream_columns<false>(ds + f * nsd * ncd + c0, nullptr, nsd, ncd, kColCh, put, chain);
     if (tid < 64) p.zap(td, fd, wnlimit[f], thre, zap + 4 * (f * ncd + c0 + (lane & 31)) + (lane < 32 ? 0 : 2));
 }
 
@@ -1195,14 +1207,16 @@ extern "C" int tx_rfi_zdot(void *stream, float *data, int nframes, long fstride,
             hipLaunchKernelGGL(k_zdot_ss, dim3(blocks_for(nframes)), dim3(256), 0, st, F, cs, sess);
             hipLaunchKernelGGL(k_zdot_rows<true>, dim3(nb), dim3(256), 0, st, F, cs, css);
         }
-    } else if (cstride == 1 && fstride == (long)nchan * nsamp && tstride == nchan && nchan >= kColCh) {
+    } else if (cstride == 1 && fstride == (long)nchan * nsamp && tstride == nchan) {
         // the DataBuffer layout [nframes][nsamp][nchan]
         const unsigned ng = (unsigned)((nchan + kColCh - 1) / kColCh);
-        hipLaunchKernelGGL(k_zdot_chain<false>, dim3(ng * nframes), dim3(kColThreads), 0, st, F, cs, stat, sess);
+        const bool narrow = nchan < kColCh;
+        const auto stats = narrow ? k_zdot_chain<false, true> : k_zdot_chain<false, false>;
+        const auto fit = narrow ? k_zdot_chain<true, true> : k_zdot_chain<true, false>;
+        hipLaunchKernelGGL(stats, dim3(ng * nframes), dim3(kColThreads), 0, st, F, cs, stat, sess);
         hipLaunchKernelGGL(k_zdot_norm_s, dim3((unsigned)((nsamp + kNsT - 1) / kNsT * nframes)), dim3(320), 0, st,
                            F, (const double *)stat, s);
-        hipLaunchKernelGGL(k_zdot_chain<true>, dim3((ng + 1) * nframes), dim3(kColThreads), 0, st, F, cs, stat,
-                           sess);
+        hipLaunchKernelGGL(fit, dim3((ng + 1) * nframes), dim3(kColThreads), 0, st, F, cs, stat, sess);
         hipLaunchKernelGGL(k_zdot_update,
                            dim3((unsigned)(((nchan + 255) / 256) * ((nsamp + kUpT - 1) / kUpT) * nframes)), dim3(256),
                            0, st, F, cs, (const double *)stat, css);
