@@ -198,3 +198,21 @@ def test_few_channels_take_no_longer_than_more():
          for c in (31, 32)}
     say("zdot of 26123 samples:", {c: round(1e6 * v) for c, v in t.items()}, "us")
     assert t[31] <= 3 * t[32]
+
+
+@pytest.mark.parametrize("nchan,nbin,nf", [(5, 1, 3), (33, 1, 2), (40, 1, 130), (7, 2, 1), (3, 3, 1), (2, 5, 128)])
+def test_channel_major_zdot_at_the_end_of_an_allocation(nchan, nbin, nf):
+    """Frames that end where their allocation ends, with rows shorter than the
+    16-byte lines that the tiles are read in."""
+    import torch
+
+    from transientx_amd import rfi
+
+    say("case end of allocation nchan", nchan, "nbin", nbin, "frames", nf)
+    x = np.random.default_rng(nchan).normal(size=(nf, nchan, nbin)).astype(np.float32)
+    ref = np.stack([oracle.zdot(x[f]) for f in range(nf)])
+    buf = torch.zeros(8 << 20, device="cuda")  # 32 MiB, its own segment
+    g = buf[-x.size:].view(nf, nchan, nbin)
+    g.copy_(torch.from_numpy(x))
+    rfi.zdot(g)
+    assert same_bits(g.cpu().numpy(), ref)

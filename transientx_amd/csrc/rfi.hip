@@ -321,15 +321,17 @@ inline RowTile row_tile(long nsamp)
 }
 
 // Rows j0 .. j0 + nr of frame f into LDS.  Whole 16-byte lines: up to 3
-// floats past a row's end are read from the next row, never past the frames.
+// floats past a row's end are read from the rows after it; rows so near the
+// frames' end that those would lie past it take 4-byte loads.
 __device__ __forceinline__ void tile_load(const Frames &F, long f, int j0, int nr, const RowTile &R, float *T)
 {
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int n = (int)F.nsamp;
+    const long total = (long)F.nframes * F.nchan * n;
     for (int r = w; r < nr; r += kTileWaves) {
         const long g = f * F.nchan + j0 + r;
         const uint32_t *src = (const uint32_t *)(F.x + g * n);
-        if ((n & 3) && g + 1 == (long)F.nframes * F.nchan)
+        if (g * n + ((n + 3) & ~3) > total)
             lds_fill(src, (uint32_t *)(T + r * R.st), n, 0, 1, lane);
         else
             lds_fill16(src, (uint32_t *)(T + r * R.st), n, 0, 1, lane);
