@@ -216,3 +216,33 @@ def test_channel_major_zdot_at_the_end_of_an_allocation(nchan, nbin, nf):
     g.copy_(torch.from_numpy(x))
     rfi.zdot(g)
     assert same_bits(g.cpu().numpy(), ref)
+
+
+# a frame per workgroup from max(64, nbin / 2) frames on with 32-row tiles, from 512 with fewer rows
+@pytest.mark.parametrize("nchan,nbin,nf", [(35, 100, 63), (35, 100, 64), (33, 301, 149), (33, 301, 150),
+                                           (17, 557, 511), (17, 557, 512), (9, 1700, 512)])
+def test_channel_major_zdot_frame_counts(nchan, nbin, nf):
+    import torch
+
+    from transientx_amd import rfi
+
+    say("case channel-major nchan", nchan, "nbin", nbin, "frames", nf)
+    x = frames(nchan + nbin + nf, nf, nchan, nbin)
+    ref = np.stack([oracle.zdot(x[f]) for f in range(nf)])
+    g = torch.from_numpy(x).cuda()
+    rfi.zdot(g)
+    assert same_bits(g.cpu().numpy(), ref)
+
+
+def test_one_frame_more_takes_little_longer():
+    """128 frames of long rows against 127 (one workgroup per frame, on half of
+    the CUs, took 1.8 times as long from 128 on; half as long again is allowed)."""
+    import torch
+
+    from transientx_amd import rfi
+
+    g = torch.Generator(device="cuda").manual_seed(4)
+    x = torch.randn((128, 256, 1013), generator=g, device="cuda")
+    t = {n: duration(rfi.zdot, x[:n]) for n in (127, 128)}
+    say("zdot of 256 x 1013:", {n: round(1e6 * v) for n, v in t.items()}, "us")
+    assert t[128] <= 1.5 * t[127]

@@ -19,6 +19,7 @@
 // bit-identical to the oracle's restatement.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <string>
 
@@ -1187,9 +1188,13 @@ extern "C" int tx_rfi_zdot(void *stream, float *data, int nframes, long fstride,
             const unsigned nt = (unsigned)((nchan + R.RB - 1) / R.RB) * nframes;
             auto fit = k_zdot_tile_fit;
             (void)hipFuncSetAttribute((const void *)fit, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kTileLds);
-            // a frame per workgroup reads the frames once less; with fewer
-            // frames than fill the CUs, a tile per workgroup is the faster
-            if (nframes >= 128) {
+            // a frame per workgroup reads the frames once less, but with
+            // fewer frames than fill the CUs twice over a tile per workgroup
+            // is the faster, the more so the longer the rows (at 1024
+            // channels, tile and frame per workgroup: 128 frames of 192
+            // samples 219 and 222 us, 256 of 512 609 and 560, 128 of 1012 783
+            // and 1261, 512 of 1012 2803 and 2543, 256 of 1700 3465 and 4242)
+            if (nframes >= (R.RB == 32 ? std::max(64L, nsamp / 2) : 512L)) {
                 auto k = k_zdot_tile_stats<true>;
                 (void)hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kTileLds);
                 hipLaunchKernelGGL(k, dim3((unsigned)nframes), dim3(kTileThreads), shm, st, F, R, stat, s, sess);
