@@ -246,3 +246,34 @@ def test_one_frame_more_takes_little_longer():
     t = {n: duration(rfi.zdot, x[:n]) for n in (127, 128)}
     say("zdot of 256 x 1013:", {n: round(1e6 * v) for n, v in t.items()}, "us")
     assert t[128] <= 1.5 * t[127]
+
+
+# both sides of the line to the row kernels: 750 channels for each 64 samples, 192 frames of 64 samples
+@pytest.mark.parametrize("nchan,nbin,nf", [(749, 64, 1), (750, 64, 1), (750, 65, 2), (1500, 65, 2), (750, 16, 192),
+                                           (750, 16, 193)])
+def test_channel_major_zdot_of_short_rows(nchan, nbin, nf):
+    import torch
+
+    from transientx_amd import rfi
+
+    say("case channel-major nchan", nchan, "nbin", nbin, "frames", nf)
+    x = frames(nchan + nbin + nf, nf, nchan, nbin)
+    ref = np.stack([oracle.zdot(x[f]) for f in range(nf)])
+    g = torch.from_numpy(x).cuda()
+    rfi.zdot(g)
+    assert same_bits(g.cpu().numpy(), ref)
+
+
+def test_a_frame_of_many_channels_and_short_rows():
+    """One frame of 4096 x 64 against four of 1024 x 64, the same samples (a lane
+    per sample walking all channels took 4.1 times as long; three times is
+    allowed)."""
+    import torch
+
+    from transientx_amd import rfi
+
+    g = torch.Generator(device="cuda").manual_seed(5)
+    x = torch.randn((4, 1024, 64), generator=g, device="cuda")
+    t = {n: duration(rfi.zdot, x.view(n, -1, 64)) for n in (1, 4)}
+    say("zdot of 4096 rows of 64:", {n: round(1e6 * v) for n, v in t.items()}, "us by frames")
+    assert t[1] <= 3 * t[4]

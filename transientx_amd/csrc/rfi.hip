@@ -321,6 +321,20 @@ inline RowTile row_tile(long nsamp)
     return {0, 0};
 }
 
+// Few frames of many channels and short rows: k_zdot_norm_mean, whose lanes
+// each walk all channels (0.115 us a channel), takes longer than the row
+// kernels, whose time goes with the tiles of 64 samples (65 us each) until
+// there are more rows than they keep in flight.  Row kernels and tiles, us:
+// 1 frame of 1024 x 64 94 and 129, 128 frames 118 and 153, 256 frames 197 and
+// 190; 1 frame of 4096 x 64 157 and 474, of 4096 x 192 301 and 486, 100 frames
+// of 4096 x 128 662 and 668; 1 frame of 1024 x 128 159 and 132, 8 frames of
+// 2048 x 192 262 and 229.
+inline bool short_rows(int nframes, int nchan, long nsamp)
+{
+    const long T = (nsamp + 63) / 64;
+    return T * 750 <= nchan && T * nframes <= 192;
+}
+
 // Rows j0 .. j0 + nr of frame f into LDS.  Whole 16-byte lines: up to 3
 // floats past a row's end are read from the rows after it; rows so near the
 // frames' end that those would lie past it take 4-byte loads.
@@ -1182,7 +1196,8 @@ extern "C" int tx_rfi_zdot(void *stream, float *data, int nframes, long fstride,
     const double *cs = s, *css = sess;
     if (tstride == 1 && fstride == (long)nchan * nsamp && cstride == nsamp) {
         // the Candidate layout [nframes][nchan][nsamp]
-        const RowTile R = row_tile(nsamp);
+        RowTile R = row_tile(nsamp);
+        if (short_rows(nframes, nchan, nsamp)) R.RB = 0;
         if (R.RB) {
             const size_t shm = tile_lds(R.RB, nsamp);
             const unsigned nt = (unsigned)((nchan + R.RB - 1) / R.RB) * nframes;
