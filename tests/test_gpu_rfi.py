@@ -218,9 +218,11 @@ def test_channel_major_zdot_at_the_end_of_an_allocation(nchan, nbin, nf):
     assert same_bits(g.cpu().numpy(), ref)
 
 
-# a frame per workgroup from max(64, nbin / 2) frames on with 32-row tiles, from 512 with fewer rows
-@pytest.mark.parametrize("nchan,nbin,nf", [(35, 100, 63), (35, 100, 64), (33, 301, 149), (33, 301, 150),
-                                           (17, 557, 511), (17, 557, 512), (9, 1700, 512)])
+# both sides of the line to a frame per workgroup: 64 frames and a third of the row or 8 per tile of 32 rows, 18 per
+# tile of fewer, 512 at most
+@pytest.mark.parametrize("nchan,nbin,nf", [(35, 301, 79), (35, 301, 80), (65, 30, 73), (65, 30, 74), (17, 557, 99),
+                                           (17, 557, 100), (9, 1700, 99), (9, 1700, 100), (401, 557, 511),
+                                           (401, 557, 512)])
 def test_channel_major_zdot_frame_counts(nchan, nbin, nf):
     import torch
 

@@ -335,6 +335,21 @@ inline bool short_rows(int nframes, int nchan, long nsamp)
     return T * 750 <= nchan && T * nframes <= 192;
 }
 
+// Frames from which a frame per workgroup is faster than a tile per workgroup.
+// It reads the frames once less and needs two launches fewer, but a workgroup
+// walks its frame's tiles one after the other while, with fewer frames than
+// fill the CUs twice over, others idle: the later, the more tiles a frame has
+// and the longer its rows.  Frame and tile per workgroup, us: 1024 channels,
+// 128 frames of 192 samples 222 and 219, 256 of 512 560 and 609, 128 of 1012
+// 1261 and 783, 512 of 1012 2543 and 2803, 256 of 1700 4242 and 3465; 256
+// channels, 128 of 512 115 and 114, 400 of 1012 574 and 617; 64 channels, 200
+// of 557 75 and 90, 128 of 1700 233 and 171, 256 of 1700 295 and 318.
+inline long frame_per_group(int nchan, long nsamp, int RB)
+{
+    const long nt = (nchan + RB - 1) / RB;
+    return RB == 32 ? 64 + std::min(nsamp / 3, 8 * nt) : std::min(512L, 64 + 18 * nt);
+}
+
 // Rows j0 .. j0 + nr of frame f into LDS.  Whole 16-byte lines: up to 3
 // floats past a row's end are read from the rows after it; rows so near the
 // frames' end that those would lie past it take 4-byte loads.
@@ -1203,13 +1218,7 @@ extern "C" int tx_rfi_zdot(void *stream, float *data, int nframes, long fstride,
             const unsigned nt = (unsigned)((nchan + R.RB - 1) / R.RB) * nframes;
             auto fit = k_zdot_tile_fit;
             (void)hipFuncSetAttribute((const void *)fit, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kTileLds);
-            // a frame per workgroup reads the frames once less, but with
-            // fewer frames than fill the CUs twice over a tile per workgroup
-            // is the faster, the more so the longer the rows (at 1024
-            // channels, tile and frame per workgroup: 128 frames of 192
-            // samples 219 and 222 us, 256 of 512 609 and 560, 128 of 1012 783
-            // and 1261, 512 of 1012 2803 and 2543, 256 of 1700 3465 and 4242)
-            if (nframes >= (R.RB == 32 ? std::max(64L, nsamp / 2) : 512L)) {
+            if (nframes >= frame_per_group(nchan, nsamp, R.RB)) {
                 auto k = k_zdot_tile_stats<true>;
                 (void)hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kTileLds);
                 hipLaunchKernelGGL(k, dim3((unsigned)nframes), dim3(kTileThreads), shm, st, F, R, stat, s, sess);
