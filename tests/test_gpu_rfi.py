@@ -279,3 +279,49 @@ def test_a_frame_of_many_channels_and_short_rows():
     t = {n: duration(rfi.zdot, x.view(n, -1, 64)) for n in (1, 4)}
     say("zdot of 4096 rows of 64:", {n: round(1e6 * v) for n, v in t.items()}, "us by frames")
     assert t[1] <= 3 * t[4]
+
+
+# channel-major kadaneF on both sides of each change of rows per workgroup (64 to 151 downsampled samples, 32 to 303, 16
+# to 607, 8 to 1,215 where td*fd is 8 or more, then the three kernels), with whole and broken groups of td and fd
+@pytest.mark.parametrize("nsd,td,fd", [(151, 1, 1), (152, 1, 1), (303, 2, 1), (304, 2, 1), (607, 1, 2), (608, 1, 2),
+                                       (607, 4, 2), (608, 4, 2), (1215, 4, 2), (1216, 4, 2), (2559, 1, 1), (640, 8, 1),
+                                       (151, 4, 1), (303, 4, 1), (304, 4, 3)])
+@pytest.mark.parametrize("rest", [0, 1])
+def test_channel_major_kadanef_row_groups(nsd, td, fd, rest):
+    import torch
+
+    from transientx_amd import rfi
+
+    nf, nchan, nbin = 2, 67 if nsd <= 304 else 19, nsd * td + (td - 1 if rest else 0)
+    if rest and td == 1:
+        nchan += fd - 1  # channels that no group takes
+    say("case channel-major kadaneF nsd", nsd, "td", td, "fd", fd, "nbin", nbin, "nchan", nchan)
+    rng = np.random.default_rng(nsd * 10 + td)
+    x = rng.normal(size=(nf, nchan, nbin)).astype(np.float32)
+    for f in range(nf):  # runs at both ends, in the middle, of both signs; the whole row; a channel that only falls
+        x[f, 0, :nbin // 3] += 2
+        x[f, 1, -(nbin // 4):] -= 2
+        x[f, nchan // 2, nbin // 3:nbin // 2] += 3
+        x[f, nchan - 2] = 1
+        x[f, 4] = -np.abs(x[f, 4])
+    x[1, 5, nbin // 2] = np.inf
+    wl = [0, 3]
+    ref = np.stack([oracle.kadanef(x[f], td, fd, 6.0, wl[f]) for f in range(nf)])
+    assert np.count_nonzero(ref == 0) > nbin
+    g = torch.from_numpy(x).cuda()
+    rfi.kadane_f(g, td, fd, 6.0, wl)
+    assert same_bits(g.cpu().numpy(), ref)
+
+
+def test_one_sample_more_takes_little_longer():
+    """kadaneF of rows of 2559 samples against 2560 (four rows a workgroup took
+    2.7 times as long as the three kernels; half as long again is allowed)."""
+    import torch
+
+    from transientx_amd import rfi
+
+    g = torch.Generator(device="cuda").manual_seed(6)
+    t = {n: duration(lambda x: rfi.kadane_f(x, 1, 1, 50.0, 0), torch.randn((64, 256, n), generator=g, device="cuda"))
+         for n in (2559, 2560)}
+    say("kadaneF of 64 x 256:", {n: round(1e6 * v) for n, v in t.items()}, "us")
+    assert t[2559] <= 1.5 * t[2560]

@@ -1070,17 +1070,27 @@ __global__ __launch_bounds__(kColThreads) void k_kad_scan_tm(int ncd, long nsd, 
     if (tid < 64) p.zap(td, fd, wnlimit[f], thre, zap + 4 * (f * ncd + c0 + (lane & 31)) + (lane < 32 ? 0 : 2));
 }
 
-// kadaneF of channel-major frames in one pass: a workgroup takes 64
+// kadaneF of channel-major frames in one pass: a workgroup takes up to 64
 // downsampled channels (fd rows each), reads their samples once (lane = a
 // downsampled sample), keeps the downsampled rows in LDS, scans them (wave 0
 // the positive runs, wave 1 the negative ones, a lane per row) and zeroes
 // what is zapped.  Reading the frames is all that is left: 0.49 ms for 2.1 GB
 // (1024 frames of 1024 x 512, td 4, fd 2), 0.82 ms with the downsampled
 // frames in memory and a kernel per step.
-constexpr size_t kKrLds = 40 * 1024; // four workgroups per CU
-inline int kad_rows(long nsd) // rows per workgroup, 0: a row does not fit
+//
+// A workgroup's G rows fill at most 38 KB (with the 2 KB of zap ranges four
+// workgroups per CU): 64 rows to 151 downsampled samples, 32 to 303, 16 to 607
+// and 8 to 1,215.  The scan keeps G lanes of two waves busy, so that longer rows
+// pay for the frames read once with chains that leave the CU idle, the sooner
+// the fewer samples go into a downsampled one.  k_kad_rows over the three
+// kernels, 1024 channels, 64 frames and td = fd = 1: 0.70 at 128 samples, 0.89
+// at 256, 1.21 at 512 (256 channels 0.71), 1.32 at 900 and 2.2 at 1800; 32
+// frames and td = 4, fd = 2: 0.62 at 512, 0.83 at 900, 1.08 at 1800.  So 8 rows
+// only for td*fd >= 8 and never fewer.
+constexpr size_t kKrLds = 38 * 1024;
+inline int kad_rows(long nsd, int td, int fd) // rows per workgroup, 0: the three kernels
 {
-    for (int G = 64; G >= 4; G >>= 1)
+    for (int G = 64; G >= ((long)td * fd >= 8 ? 8 : 16); G >>= 1)
         if (nsd <= 65536 && (size_t)G * (nsd | 1) * 4 <= kKrLds) return G;
     return 0;
 }
@@ -1289,7 +1299,7 @@ extern "C" int tx_rfi_kadanef(void *stream, float *data, int nframes, long fstri
                            st, ncd, nsd, td, fd, threshold, wnlimit, (const float *)ds, zap);
         hipLaunchKernelGGL(k_kad_zero_tm, dim3((unsigned)(nzt * ((nsamp + kKzT - 1) / kKzT) * nframes)), dim3(256), 0,
                            st, F, fd, ncd, (const long *)zap);
-    } else if (const int G = tstride == 1 && fstride == (long)nchan * nsamp && cstride == nsamp ? kad_rows(nsd) : 0) {
+    } else if (const int G = tstride == 1 && fstride == (long)nchan * nsamp && cstride == nsamp ? kad_rows(nsd, td, fd) : 0) {
         // the Candidate layout [nframes][nchan][nsamp]
         hipLaunchKernelGGL(k_kad_rows, dim3((unsigned)((ncd + G - 1) / G * nframes)), dim3(256),
                            (size_t)G * (nsd | 1) * 4, st, F, td, fd, ncd, (int)nsd, G, threshold, wnlimit);
