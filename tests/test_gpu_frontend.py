@@ -272,3 +272,49 @@ def test_frontend_word_loads(ns, nch, shift):
         out = frontend.apply(g, 1, 1, off, gain, chan_mask=mask).cpu().numpy()
         ref = oracle.frontend_u8(x, 1, 1, ro, rg, mask if mask is not None else np.ones(nch, np.uint8))
         assert np.array_equal(out.view(np.uint32), ref.view(np.uint32))
+
+
+# the statistics' 32-bit loads, from 256 channels and 2^24 samples in the block on: whole and broken workgroups of 256
+# channels and 512 samples
+@pytest.mark.parametrize("ns,nch,shift", [(65536, 256, 0), (65535, 256, 0), (67000, 252, 0), (64600, 260, 0),
+                                          (32771, 516, 0), (65536, 256, 1)])
+def test_frontend_word_statistics(ns, nch, shift):
+    import torch
+
+    from transientx_amd import frontend
+
+    say("case front end statistics ns", ns, "nch", nch, "shift", shift)
+    rng = np.random.default_rng(ns + nch)
+    x = rng.integers(0, 256, size=(ns, nch)).astype(np.uint8)
+    x[:, 3] = 255
+    x[:, nch - 1] = 7
+    buf = torch.zeros(ns * nch + shift, dtype=torch.uint8, device="cuda")
+    g = buf[shift:].view(ns, nch)
+    g.copy_(torch.from_numpy(x))
+    off, gain = frontend.stats(g, 1, 1)
+    ro, rg = oracle.frontend_stats(x, 1, 1)
+    assert np.array_equal(off.cpu().numpy().view(np.uint32), ro.view(np.uint32))
+    assert np.array_equal(gain.cpu().numpy().view(np.uint32), rg.view(np.uint32))
+
+
+def test_statistics_of_few_channels():
+    """2,000,000 samples of 16 channels against 252 (the same time with a workgroup
+    for 256 channels; 0.7 of it is allowed)."""
+    import time
+
+    import torch
+
+    from transientx_amd import frontend
+
+    t = {}
+    for nch in (16, 252):
+        x = torch.full((2000000, nch), 100, dtype=torch.uint8, device="cuda")
+        t[nch] = np.inf
+        for _ in range(8):
+            torch.cuda.synchronize()
+            t0 = time.perf_counter()
+            frontend.stats(x)
+            torch.cuda.synchronize()
+            t[nch] = min(t[nch], time.perf_counter() - t0)
+    say("statistics:", {n: round(1e6 * v) for n, v in t.items()}, "us")
+    assert t[16] <= 0.7 * t[252]

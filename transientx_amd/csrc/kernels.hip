@@ -329,7 +329,11 @@ __global__ __launch_bounds__(256) void k_frontend_sums(const uint8_t *__restrict
 // td = fd = 1 with a multiple of 4 channels and a 4-byte aligned block: a
 // thread sums 4 channels (one 32-bit load per sample) over 128 samples of the
 // workgroup's 512, 16 loads in flight; 128 * 255^2 fits 32 bits.  44 us for
-// 4096 channels x 26,123 samples (66 us with byte loads).
+// 4096 channels x 26,123 samples (66 us with byte loads).  A workgroup takes
+// 256 channels, so that fewer leave its lanes idle: 2,000,000 samples of 16
+// channels 679 us (342 by bytes), of 128 682 (530), of 252 695 (773), of 512 781
+// (1197).  Small blocks are all launches and tails: 512 x 26,123 21.7 us (20.2
+// by bytes), 1024 x 26,123 23.2 (28.4).  Hence 256 channels and 2^24 samples.
 constexpr int kFsT = 512;
 __global__ __launch_bounds__(256) void k_frontend_sums4(const uint32_t *__restrict__ blk, long ns, int C4,
                                                         unsigned long long *acc)
@@ -438,7 +442,7 @@ void launch_frontend_stats(hipStream_t st, const uint8_t *blk, long ns, int Cin,
 {
     const int C = Cin / fd;
     hipLaunchKernelGGL(k_frontend_zero, dim3((unsigned)((2L * C + 255) / 256)), dim3(256), 0, st, acc, 2L * C);
-    if (td == 1 && fd == 1 && C % 4 == 0 && (uintptr_t)blk % 4 == 0) {
+    if (td == 1 && fd == 1 && C % 4 == 0 && (uintptr_t)blk % 4 == 0 && C >= 256 && ns * C >= 1L << 24) {
         const long nwg = ((C / 4 + 63) / 64) * ((ns + kFsT - 1) / kFsT);
         hipLaunchKernelGGL(k_frontend_sums4, dim3((unsigned)nwg), dim3(256), 0, st, (const uint32_t *)blk, ns, C / 4,
                            acc);
