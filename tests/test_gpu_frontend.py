@@ -318,3 +318,38 @@ def test_statistics_of_few_channels():
             t[nch] = min(t[nch], time.perf_counter() - t0)
     say("statistics:", {n: round(1e6 * v) for n, v in t.items()}, "us")
     assert t[16] <= 0.7 * t[252]
+
+
+# the applied front end's rows of 1 to 256 threads: channel counts around the powers of two, lengths around the 8 steps of
+# 256, 128, ... rows
+@pytest.mark.parametrize("ns,nch", [(2047, 4), (2049, 4), (1025, 8), (513, 12), (257, 20), (255, 64), (65, 132),
+                                    (33, 256), (31, 516), (17, 1024), (9, 1028)])
+def test_frontend_rows_of_threads(ns, nch):
+    import torch
+
+    from transientx_amd import frontend
+
+    say("case front end rows ns", ns, "nch", nch)
+    rng = np.random.default_rng(ns * nch)
+    x = rng.integers(0, 256, size=(ns, nch)).astype(np.uint8)
+    off, gain = oracle.frontend_stats(x, 1, 1)
+    mask = (rng.random(nch) > 0.2).astype(np.uint8)
+    out = frontend.apply(torch.from_numpy(x).cuda(), 1, 1, off, gain, chan_mask=mask).cpu().numpy()
+    ref = oracle.frontend_u8(x, 1, 1, off, gain, mask)
+    assert np.array_equal(out.view(np.uint32), ref.reshape(out.shape).view(np.uint32))
+
+
+def test_frontend_of_few_channels_and_many_samples():
+    """2^27 samples of 4 channels: with a row of 256 threads for every 8 samples
+    they were more threads than a launch holds."""
+    import torch
+
+    from transientx_amd import frontend
+
+    ns, nch = (1 << 27) + 11, 4
+    x = torch.randint(0, 256, (ns, nch), dtype=torch.uint8, device="cuda")
+    off = torch.tensor([100.0, 0.5, 3.25, -7.0], device="cuda")
+    gain = torch.tensor([0.1, 1.0, -2.5, 0.37], device="cuda")
+    out = frontend.apply(x, 1, 1, off, gain)
+    for a in range(0, ns, 1 << 25):
+        assert torch.equal(out[a:a + (1 << 25)], (x[a:a + (1 << 25)].float() - off) * gain)

@@ -242,16 +242,20 @@ __global__ __launch_bounds__(256) void k_frontend_tm(const uint8_t *__restrict__
 // thread takes 4 channels of 8 samples, each one 32-bit load and one 16-byte
 // store, all loads in flight at once.  Bound by the block's read and write
 // (5 bytes a sample): 95 us for 4096 channels x 26,123 samples, 5.6 TB/s,
-// against 190 us with a byte load per thread.
+// against 190 us with a byte load per thread.  A row of fewer than 1024
+// channels takes 2^lg threads and a workgroup 256 >> lg rows at a time, so that
+// few channels leave no lanes idle: 2,000,000 samples of 32 channels 59 us (262
+// with 256 threads per row, 204 by bytes), of 4 channels 11 (170, 206).
 constexpr int kFtT = 8;
-__global__ __launch_bounds__(256) void k_frontend_tm4(const uint32_t *__restrict__ blk, long ns, int C4,
+__global__ __launch_bounds__(256) void k_frontend_tm4(const uint32_t *__restrict__ blk, long ns, int C4, int lg,
                                                       const float4 *__restrict__ off,
                                                       const float4 *__restrict__ gain,
                                                       const uint8_t *__restrict__ mask, float4 *__restrict__ out)
 {
-    const long nct = (C4 + 255) / 256;
-    const int c = (int)(blockIdx.x % nct) * 256 + threadIdx.x;
-    const long t0 = blockIdx.x / nct * kFtT;
+    const long nct = (C4 + (1 << lg) - 1) >> lg;
+    const int c = ((int)(blockIdx.x % nct) << lg) + (threadIdx.x & ((1 << lg) - 1));
+    const int R = 256 >> lg; // rows of a workgroup's step
+    const long t0 = blockIdx.x / nct * kFtT * R + (threadIdx.x >> lg);
     if (c >= C4) return;
     const float4 o = off[c], g = gain[c];
     bool live[4];
@@ -259,16 +263,16 @@ __global__ __launch_bounds__(256) void k_frontend_tm4(const uint32_t *__restrict
     for (int i = 0; i < 4; i++) live[i] = !mask || mask[4 * c + i];
     uint32_t y[kFtT];
 #pragma unroll
-    for (int u = 0; u < kFtT; u++) y[u] = (blk + min(t0 + u, ns - 1) * C4)[c]; // past the end: unused
+    for (int u = 0; u < kFtT; u++) y[u] = (blk + min(t0 + u * R, ns - 1) * C4)[c]; // past the end: unused
 #pragma unroll
     for (int u = 0; u < kFtT; u++) {
-        if (t0 + u >= ns) break;
+        if (t0 + u * R >= ns) break;
         float4 v;
         v.x = live[0] ? ((float)(y[u] & 0xFFu) - o.x) * g.x : 0.f;
         v.y = live[1] ? ((float)((y[u] >> 8) & 0xFFu) - o.y) * g.y : 0.f;
         v.z = live[2] ? ((float)((y[u] >> 16) & 0xFFu) - o.z) * g.z : 0.f;
         v.w = live[3] ? ((float)(y[u] >> 24) - o.w) * g.w : 0.f;
-        (out + (t0 + u) * C4)[c] = v;
+        (out + (t0 + u * R) * C4)[c] = v;
     }
 }
 
@@ -428,8 +432,11 @@ void launch_frontend_tm(hipStream_t st, const uint8_t *blk, long ns, int Cin, in
     const int C = Cin / fd;
     if (td == 1 && fd == 1 && C % 4 == 0 && (uintptr_t)blk % 4 == 0 && (uintptr_t)off % 16 == 0 &&
         (uintptr_t)gain % 16 == 0 && (uintptr_t)out % 16 == 0) {
-        const long nwg = ((C / 4 + 255) / 256) * ((ns + kFtT - 1) / kFtT);
-        hipLaunchKernelGGL(k_frontend_tm4, dim3((unsigned)nwg), dim3(256), 0, st, (const uint32_t *)blk, ns, C / 4,
+        int lg = 0;
+        while (lg < 8 && (1 << lg) < C / 4) lg++;
+        const long nr = (long)kFtT << (8 - lg); // samples of a workgroup
+        const long nwg = ((C / 4 + (1 << lg) - 1) >> lg) * ((ns + nr - 1) / nr);
+        hipLaunchKernelGGL(k_frontend_tm4, dim3((unsigned)nwg), dim3(256), 0, st, (const uint32_t *)blk, ns, C / 4, lg,
                            (const float4 *)off, (const float4 *)gain, mask, (float4 *)out);
         return;
     }
