@@ -491,3 +491,91 @@ def test_grid_row_lengths(nchan, nbin):
             assert np.all(np.abs(best[:, r] - top) <= 1e-4 * np.abs(top) + 1e-5), (r, best[:, r], top)
     finally:
         m.close()
+
+
+@pytest.mark.parametrize("nchan,nbin", [(9, 130), (70, 64), (300, 96), (11, 1500)])
+@pytest.mark.parametrize("live", ["every fourth", "one", "last", "few", "all but one"])
+def test_channels_of_weight_zero(nchan, nbin, live):
+    """Weights that leave waves without a channel, with one, or with a ragged
+    step: S and the gradients without dS/dw against the FP64 restatement with
+    the dead channels' samples NaN (they count for nothing), then dS/dw and
+    dS/dx of live and dead channels with finite samples."""
+    import torch
+
+    from transientx_amd.diff import DiffSNR
+
+    f, x, w, dm, t0, W, kf, tbin = make(nbin + nchan, 2, nchan=nchan, nbin=nbin)
+    rng = np.random.default_rng(nchan)
+    on = {"every fourth": np.arange(nchan) % 4 == 2, "one": np.arange(nchan) == nchan // 2,
+          "last": np.arange(nchan) >= nchan - 2, "few": rng.random(nchan) < 0.1,
+          "all but one": np.arange(nchan) != 4}[live]
+    on[3] = on[3] or not on.any()
+    w[:, on] = rng.uniform(0.5, 1.5, (2, int(on.sum()))).astype(np.float32)
+    w[:, ~on] = 0.0
+    say("case nchan", nchan, "nbin", nbin, live)
+    m = DiffSNR(f, nbin, tbin, softness=1.0)
+    F = lambda v: torch.tensor(v, dtype=torch.float32, device="cuda")
+    one, wt = torch.ones(2, device="cuda"), torch.from_numpy(w).cuda()
+    xn = x.copy()
+    xn[:, ~on] = np.nan
+    try:
+        xt, xnt = torch.from_numpy(x).cuda(), torch.from_numpy(xn).cuda()
+        fwd = m.forward(xnt, wt, F(dm), F(t0), F(W)).cpu().numpy()
+        snr, gdm, gt0, gwd = (v.cpu().numpy() for v in m.adjoint(xnt, wt, F(dm), F(t0), F(W), one, need_w=False)[:4])
+        full = [v.cpu().numpy() for v in m.adjoint(xt, wt, F(dm), F(t0), F(W), one, need_x=True)]
+        best = m.grid(xnt, wt, F(dm), F(t0), 1, 0.5, 1, 1.0, F(W[:1]))[0].cpu().numpy()
+        best_x = m.grid(xt, wt, F(dm), F(t0), 1, 0.5, 1, 1.0, F(W[:1]))[0].cpu().numpy()
+    finally:
+        m.close()
+    assert np.array_equal(fwd, snr) and np.array_equal(full[0], snr)
+    assert np.array_equal(full[2], gt0) and np.array_equal(full[3], gwd)
+    assert np.array_equal(best, best_x) and np.all(np.isfinite(best))
+    assert np.all(full[5][:, ~on] == 0)
+    xd, wd = x.astype(np.float64), w.astype(np.float64)
+    for c in range(2):
+        args = [np.float64(np.float32(v[c])) for v in (dm, t0, W)]
+        s64 = snr64(xd[c], wd[c], *args, kf, 1.0)
+        assert abs(snr[c] - s64) <= 2e-5 * max(1.0, abs(s64)), (c, snr[c], s64)
+        a1, a2 = list(args), list(args)
+        a1[0] += 1e-6
+        a2[0] -= 1e-6
+        ref = (snr64(xd[c], wd[c], *a1, kf, 1.0) - snr64(xd[c], wd[c], *a2, kf, 1.0)) / 2e-6
+        for got in (gdm[c], full[1][c]):
+            assert abs(got - ref) <= 2e-3 * abs(ref) + 2e-3, (c, got, ref)
+        for j in range(0, nchan, max(1, nchan // 24)):
+            w1, w2 = wd[c].copy(), wd[c].copy()
+            w1[j] += 1e-6
+            w2[j] -= 1e-6
+            ref = (snr64(xd[c], w1, *args, kf, 1.0) - snr64(xd[c], w2, *args, kf, 1.0)) / 2e-6
+            assert abs(full[4][c, j] - ref) <= 2e-3 * abs(ref) + 2e-4, (c, j, full[4][c, j], ref)
+
+
+def test_dead_channels_cost_little():
+    """S of cutouts with 97% of their channels at weight zero against none (the
+    same time while dead channels' rows are fetched; 0.6 of it is allowed)."""
+    import time
+
+    import torch
+
+    from transientx_amd.diff import DiffSNR
+
+    n, nchan, nbin = 64, 1024, 1024
+    g = torch.Generator(device="cuda").manual_seed(2)
+    x = torch.randn((n, nchan, nbin), generator=g, device="cuda")
+    m = DiffSNR(np.linspace(1500.0, 1200.0, nchan), nbin, 98.304e-6, softness=1.0)
+    v = torch.full((n,), 100.0, device="cuda")
+    t = {}
+    try:
+        for dead in (0.0, 0.97):
+            w = (torch.rand((n, nchan), generator=g, device="cuda") >= dead).float()
+            t[dead] = np.inf
+            for _ in range(10):
+                torch.cuda.synchronize()
+                t0 = time.perf_counter()
+                m.forward(x, w, v, v, v)
+                torch.cuda.synchronize()
+                t[dead] = min(t[dead], time.perf_counter() - t0)
+    finally:
+        m.close()
+    say("S of 64 x 1024 x 1024:", {k: round(1e6 * u) for k, u in t.items()}, "us by dead channels")
+    assert t[0.97] <= 0.6 * t[0.0]

@@ -54,8 +54,8 @@ struct DiffArgs {
 
 __device__ inline float sigm(float z) { return 1.f / (1.f + expf(-z)); }
 
-// Dynamic LDS of k_diff / k_dgrid: 4 wave partials of p, and per channel its
-// whole-sample delay and fraction.
+// Dynamic LDS of k_diff / k_dgrid: 4 wave partials of p, and per channel a list
+// entry and its delay's fraction.
 inline size_t diff_lds(int nbin, int nchan) { return (size_t)16 * nbin + (size_t)8 * nchan; }
 constexpr size_t kDiffMaxLds = 160 * 1024;
 
@@ -70,63 +70,104 @@ __device__ inline double block_sum_d(double v, double *sh)
     return ((sh[0] + sh[1]) + sh[2]) + sh[3];
 }
 
-// f(j, w_j, x0, x1) for the channels j = wave, wave + 4, ... in order: lane l
+// The delays of the wave's channels j = wave, wave + 4, ... at dm: channel j's
+// fraction in sa[j], and in sd the list of them (entry i at wave + 4*i, j << 12
+// with the whole samples mod nbin <= 4096), the channels of non-zero weight
+// first and in order, those of weight zero behind them.  Returns how many are
+// not zero.
+__device__ __forceinline__ int channel_list(double dm, const double *kf, const float *W, int nchan, int nbin, int lane,
+                                            int wave, int *sd, float *sa)
+{
+    const int n = (nchan - wave + 3) / 4;
+    int live = 0, dead = 0;
+    for (int b = 0; b < n; b += 64) {
+        const int j = wave + 4 * (b + lane);
+        const bool in = j < nchan;
+        int d = 0;
+        if (in) {
+            const double tau = dm * kf[j];
+            const double fl = floor(tau);
+            sa[j] = (float)(tau - fl);
+            d = (int)fmod(fl, (double)nbin);
+            if (d < 0) d += nbin;
+        }
+        const bool on = in && W[j] != 0.f;
+        const unsigned long long m = __ballot(on), z = __ballot(in && !on), below = (1ull << lane) - 1;
+        const int i = on ? live + __popcll(m & below) : n - 1 - dead - __popcll(z & below);
+        if (in) sd[wave + 4 * i] = j << 12 | d;
+        live += __popcll(m);
+        dead += __popcll(z);
+    }
+    return __builtin_amdgcn_readfirstlane(live);
+}
+
+// The sample a fraction al of the way from x0 to x1.  The fused operations are
+// written out, here and where profiles are summed: left to the compiler, it
+// fuses the one product or the other with the code around.
+__device__ __forceinline__ float between(float al, float x0, float x1) { return fmaf(1.f - al, x0, al * x1); }
+
+// f(j, d_j, w_j, x0, x1) for the first n channels of the wave's list: lane l
 // gets x0[u] = X_j[(t + d_j) mod nbin] and x1[u], the sample after it, for
 // t = l + 64*u.  Few workgroups share a CU here, so that a channel's weight and
 // row, waited for one after the other, were all the time went to: the rows of
 // the next NB channels (and their weights, through the scalar cache) are
 // fetched before the current ones are used, and x1 comes from the neighbouring
-// lane (wave_shl:1; lane 63's is lane 0's of the next u).  512 evaluations of
-// 1024 x 512: forward 202 us (1069), with the adjoint 505 us (2229);
-// k_dgrid, 128 cutouts and 9 DM trials of that size: 343 us (810).  A
-// pass over the 1.07 GB: at 5.3 and 4.2 TB/s the memory bounds both.
+// lane when it is used (wave_shl:1; lane 63's is lane 0's of the next u): held
+// for the whole row, or with U sample positions kept from row to row, it cost
+// twice the registers.  512 evaluations of 1024 x 512: forward 197 us (1069),
+// with the adjoint 477 us (2229); of 1024 x 1024 374 and 833, 256 of 1024 x
+// 2048 375 and 1029, 128 of 1024 x 4096 540 and 1538; k_dgrid, 128 cutouts of
+// 1024 x 512 and 9 DM trials: 277 us (810).  A pass over the 1.07 GB: at 5.3 and
+// 4.2 TB/s the memory bounds both.  Channels of weight zero are left out where
+// nothing is wanted of them: with 90% of them dead 512 evaluations of 1024 x
+// 512 take 44 us (205 when their rows were fetched too, 178 when each row was
+// waited for), 128 of 1024 x 4096 101 (555, 908).
 template <int U, typename F>
-__device__ __forceinline__ void channel_rows(const float *X, const float *W, const int *sd, int nchan, int nbin,
-                                             int lane, int wave, F f)
+__device__ __forceinline__ void channel_rows(const float *X, const float *W, const int *sd, int n, int nbin, int lane,
+                                             int wave, F f)
 {
     constexpr int NB = U <= 8 ? 4 : U <= 16 ? 2 : 1;
     typedef __attribute__((address_space(4))) const float const_float_t;
-    const int n = (nchan - wave + 3) / 4;
     if (n <= 0) return;
     float nx[NB][U], nw[NB];
-    auto fetch = [&](int s, float (&v)[U], float &w) {
-        const int j = wave + 4 * min(s, n - 1);
+    int nj[NB];
+    auto fetch = [&](int s, float (&v)[U], float &w, int &jd) {
+        jd = __builtin_amdgcn_readfirstlane(sd[wave + 4 * min(s, n - 1)]);
+        const int j = jd >> 12, d = jd & 4095;
         w = ((const_float_t *)W)[j];
-        const int d = __builtin_amdgcn_readfirstlane(sd[j]);
-        const float *row = X + (size_t)j * nbin;
+        const char *row = (const char *)(X + (size_t)j * nbin);
+        const unsigned t = 4u * (unsigned)(lane + d), len = 4u * (unsigned)nbin;
 #pragma unroll
         for (int u = 0; u < U; u++) {
-            int i0 = min(lane + 64 * u, nbin - 1) + d;
-            if (i0 >= nbin) i0 -= nbin;
-            v[u] = row[i0];
+            const unsigned o = t + 256u * u; // wrapped: the smaller of o and o - len, as unsigned numbers
+            v[u] = *(const float *)(row + min(min(o, o - len), len - 4)); // lanes past the row: its last sample
         }
     };
 #pragma unroll
-    for (int b = 0; b < NB; b++) fetch(b, nx[b], nw[b]);
+    for (int b = 0; b < NB; b++) fetch(b, nx[b], nw[b], nj[b]);
     for (int s = 0; s < n; s += NB) {
         float x0[NB][U], w[NB];
+        int jd[NB];
 #pragma unroll
         for (int b = 0; b < NB; b++) {
             w[b] = nw[b];
+            jd[b] = nj[b];
 #pragma unroll
             for (int u = 0; u < U; u++) x0[b][u] = nx[b][u];
         }
 #pragma unroll
-        for (int b = 0; b < NB; b++) fetch(s + NB + b, nx[b], nw[b]);
+        for (int b = 0; b < NB; b++) fetch(s + NB + b, nx[b], nw[b], nj[b]);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int b = 0; b < NB; b++) {
             if (s + b >= n) break;
-            float x1[U];
             const int first = __builtin_amdgcn_readfirstlane(__float_as_int(x0[b][0]));
-#pragma unroll
-            for (int u = 0; u < U; u++) {
+            auto x1 = [&](int u) {
                 const int after = __builtin_amdgcn_readfirstlane(__float_as_int(x0[b][(u + 1) % U]));
-                const int nb =
-                    __builtin_amdgcn_update_dpp(after, __float_as_int(x0[b][u]), 0x130, 0xF, 0xF, false);
-                x1[u] = __int_as_float(lane + 64 * u == nbin - 1 ? first : nb);
-            }
-            f(wave + 4 * (s + b), w[b], x0[b], x1);
+                const int nb = __builtin_amdgcn_update_dpp(after, __float_as_int(x0[b][u]), 0x130, 0xF, 0xF, false);
+                return __int_as_float(lane + 64 * u == nbin - 1 ? first : nb);
+            };
+            f(jd[b] >> 12, jd[b] & 4095, w[b], x0[b], x1);
         }
     }
 }
@@ -138,8 +179,8 @@ __global__ __launch_bounds__(256) void k_diff(DiffArgs A)
     extern __shared__ float smem[];
     float *pw = smem;                  // [4][nbin] wave partials of p, then p, then G
     __shared__ double shd[4];
-    int *sd = (int *)(smem + 4 * A.nbin);   // [nchan] whole-sample delay mod nbin
-    float *sa = (float *)(sd + A.nchan);    // [nchan] its fraction
+    int *sd = (int *)(smem + 4 * A.nbin);   // [nchan] the waves' channel lists
+    float *sa = (float *)(sd + A.nchan);    // [nchan] the delays' fractions
     // logical order: consecutive evaluations (which share a cutout) on one
     // XCD, so the cutout is fetched into one L2 rather than eight
     const int e = (int)txgpu::xcd_logical(blockIdx.x, gridDim.x);
@@ -149,26 +190,18 @@ __global__ __launch_bounds__(256) void k_diff(DiffArgs A)
     const float *X = A.x + (size_t)c * nchan * nbin;
     const float *W = A.w + (size_t)c * nchan;
     const double dm = (double)A.dm[e];
-    // the channels' delays at this DM, once per workgroup, all lanes at once
-    for (int j = tid; j < nchan; j += 256) {
-        const double tau = dm * A.kf[j];
-        const double fl = floor(tau);
-        sa[j] = (float)(tau - fl);
-        int d = (int)fmod(fl, (double)nbin);
-        if (d < 0) d += nbin;
-        sd[j] = d;
-    }
+    // the channels' delays at this DM, once per workgroup
+    const int nlive = channel_list(dm, A.kf, W, nchan, nbin, lane, wave, sd, sa);
     __syncthreads();
 
     // ---- forward: p(t), channel j on wave j % 4
     float acc[U];
 #pragma unroll
     for (int u = 0; u < U; u++) acc[u] = 0.f;
-    channel_rows<U>(X, W, sd, nchan, nbin, lane, wave, [&](int j, float wj, const float(&x0)[U], const float(&x1)[U]) {
-        if (wj == 0.f) return;
+    channel_rows<U>(X, W, sd, nlive, nbin, lane, wave, [&](int j, int, float wj, const float(&x0)[U], auto x1) {
         const float al = sa[j];
 #pragma unroll
-        for (int u = 0; u < U; u++) acc[u] += wj * ((1.f - al) * x0[u] + al * x1[u]);
+        for (int u = 0; u < U; u++) acc[u] = fmaf(wj, between(al, x0[u], x1(u)), acc[u]);
     });
 #pragma unroll
     for (int u = 0; u < U; u++) {
@@ -266,33 +299,36 @@ __global__ __launch_bounds__(256) void k_diff(DiffArgs A)
     double gdm_w = 0.;
     if (!A.gw && !A.gx) {
         double lacc = 0.;
-        channel_rows<U>(X, W, sd, nchan, nbin, lane, wave,
-                        [&](int j, float wj, const float(&x0)[U], const float(&x1)[U]) {
-                            if (wj == 0.f) return;
+        channel_rows<U>(X, W, sd, nlive, nbin, lane, wave,
+                        [&](int j, int, float wj, const float(&x0)[U], auto x1) {
                             double b = 0.;
 #pragma unroll
-                            for (int u = 0; u < U; u++)
-                                if (lane + 64 * u < nbin) b += (double)G[u] * (double)(x1[u] - x0[u]);
+                            for (int u = 0; u < U; u++) {
+                                const float dx = x1(u) - x0[u];
+                                if (lane + 64 * u < nbin) b += (double)G[u] * (double)dx;
+                            }
                             lacc += (double)wj * A.kf[j] * b;
                         });
         gdm_w = wave_sum_d(lacc);
     } else
-    channel_rows<U>(X, W, sd, nchan, nbin, lane, wave, [&](int j, float wj, const float(&x0)[U], const float(&x1)[U]) {
+    channel_rows<U>(X, W, sd, (nchan - wave + 3) / 4, nbin, lane, wave,
+                    [&](int j, int d, float wj, const float(&x0)[U], auto x1) {
         const float al = sa[j];
         double a = 0., b = 0.;
 #pragma unroll
-        for (int u = 0; u < U; u++)
+        for (int u = 0; u < U; u++) {
+            const float y = x1(u);
             if (lane + 64 * u < nbin) {
-                a += (double)G[u] * (double)((1.f - al) * x0[u] + al * x1[u]);
-                b += (double)G[u] * (double)(x1[u] - x0[u]);
+                a += (double)G[u] * (double)between(al, x0[u], y);
+                b += (double)G[u] * (double)(y - x0[u]);
             }
+        }
         a = wave_total_d(a);
         b = wave_total_d(b);
         if (A.gw && lane == 0) A.gw[(size_t)e * nchan + j] = (float)(gs * (a - S * (double)wj / sw2));
         gdm_w += (double)wj * A.kf[j] * b; // identical on every lane
         if (A.gx) {
             // dS/dx_j[k] = w_j*((1-a_j)*G(k-d_j) + a_j*G(k-d_j-1))
-            const int d = sd[j];
             float *gxr = A.gx + ((size_t)e * nchan + j) * nbin;
             for (int k = lane; k < nbin; k += 64) {
                 int t0i = k - d;
@@ -590,8 +626,8 @@ __global__ __launch_bounds__(256) void k_dgrid(GridArgs A)
     __shared__ double shd[4];
     __shared__ float sbS[4];
     __shared__ int sbI[4];
-    int *sd = (int *)(smem + 4 * A.nbin);   // [nchan] whole-sample delay mod nbin
-    float *sa = (float *)(sd + A.nchan);    // [nchan] its fraction
+    int *sd = (int *)(smem + 4 * A.nbin);   // [nchan] the waves' channel lists
+    float *sa = (float *)(sd + A.nchan);    // [nchan] the delays' fractions
     const unsigned lid = txgpu::xcd_logical(blockIdx.x, gridDim.x);
     const int c = (int)(lid / A.ndm), m = (int)(lid % A.ndm);
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -599,24 +635,16 @@ __global__ __launch_bounds__(256) void k_dgrid(GridArgs A)
     const float *X = A.x + (size_t)c * nchan * nbin;
     const float *W = A.w + (size_t)c * nchan;
     const double dm = (double)(A.dm0[c] + (float)m * A.ddm);
-    for (int j = tid; j < nchan; j += 256) {
-        const double tau = dm * A.kf[j];
-        const double fl = floor(tau);
-        sa[j] = (float)(tau - fl);
-        int d = (int)fmod(fl, (double)nbin);
-        if (d < 0) d += nbin;
-        sd[j] = d;
-    }
+    const int nlive = channel_list(dm, A.kf, W, nchan, nbin, lane, wave, sd, sa);
     __syncthreads();
 
     float acc[U];
 #pragma unroll
     for (int u = 0; u < U; u++) acc[u] = 0.f;
-    channel_rows<U>(X, W, sd, nchan, nbin, lane, wave, [&](int j, float wj, const float(&x0)[U], const float(&x1)[U]) {
-        if (wj == 0.f) return;
+    channel_rows<U>(X, W, sd, nlive, nbin, lane, wave, [&](int j, int, float wj, const float(&x0)[U], auto x1) {
         const float al = sa[j];
 #pragma unroll
-        for (int u = 0; u < U; u++) acc[u] += wj * ((1.f - al) * x0[u] + al * x1[u]);
+        for (int u = 0; u < U; u++) acc[u] = fmaf(wj, between(al, x0[u], x1(u)), acc[u]);
     });
 #pragma unroll
     for (int u = 0; u < U; u++) {
