@@ -128,3 +128,9 @@ def test_refine_row_lengths(nchan, nbin):
         assert np.array_equal(wid[c], W), f"width map cand {c}"
         assert (res[c]["maxdmid"], res[c]["maxtid"], res[c]["wn"]) == (j, i, W[j, i])
         assert res[c]["snr"] == np.float32(s)
+
+
+@pytest.mark.parametrize("nchan,nbin", [(9, 1280), (8, 1281), (8, 1536), (9, 1537)])
+def test_refine_row_lengths_past_1024(nchan, nbin):
+    """The same around the tree's 20 and 24 columns a lane."""
+    test_refine_row_lengths(nchan, nbin)

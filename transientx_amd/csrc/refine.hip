@@ -225,6 +225,9 @@ __global__ __launch_bounds__(256) void k_tree_pass(TreeArgs A)
 // ncol allows.  P2: ncol is a power of two, and a wrap is a mask.
 // 256 cutouts of 1024 x 512, five levels a pass: 258 us a pass, k_tree_pass 865;
 // 1.07 GB read and written, 216 us at a copy's rate, bounds it.
+// U steps close enough that few of a wave's steps lie past the row's end: whole
+// grids with maps, 48 cutouts of 1024 x 1025, 1838 us with 20 columns a lane, 2309
+// with 32, 2152 with k_tree_pass.
 template <int U, bool P2>
 __global__ __launch_bounds__(512) void k_tree_rows(TreeArgs A)
 {
@@ -341,6 +344,8 @@ auto tree_rows_kernel(int ncol) -> void (*)(TreeArgs)
     if (ncol <= 256) return p2 ? k_tree_rows<4, true> : k_tree_rows<4, false>;
     if (ncol <= 512) return p2 ? k_tree_rows<8, true> : k_tree_rows<8, false>;
     if (ncol <= 1024) return p2 ? k_tree_rows<16, true> : k_tree_rows<16, false>;
+    if (ncol <= 1280) return k_tree_rows<20, false>;
+    if (ncol <= 1536) return k_tree_rows<24, false>;
     return p2 ? k_tree_rows<32, true> : k_tree_rows<32, false>;
 }
 
