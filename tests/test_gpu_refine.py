@@ -134,3 +134,30 @@ def test_refine_row_lengths(nchan, nbin):
 def test_refine_row_lengths_past_1024(nchan, nbin):
     """The same around the tree's 20 and 24 columns a lane."""
     test_refine_row_lengths(nchan, nbin)
+
+
+@pytest.mark.parametrize("nbin", [1537, 1536])
+def test_refine_many_long_rows(nbin):
+    """Batches on both sides of 18 x 1024 rows, where rows of no whole 16-byte
+    lines change kernels: the same results, and the oracle's for a few."""
+    import torch
+
+    nchan, n, tbin = 64, 289, 98.304e-6
+    f = np.linspace(1500.0, 1200.0, nchan)
+    g = torch.Generator(device="cuda").manual_seed(nbin)
+    x = torch.randn((n, nchan, nbin), generator=g, device="cuda")
+    dm = np.random.default_rng(nbin).uniform(20, 300, n)
+    say("case", n, nchan, nbin)
+    res = []
+    for batch in (n, n - 1):  # 18,496 rows, then 18,432 and 64
+        R = Refiner(f, nbin, tbin, 0.1, max_batch=batch)
+        try:
+            res.append(R.run(x, dm))
+        finally:
+            R.close()
+    assert res[0].tobytes() == res[1].tobytes()
+    for c in (0, 7, n - 1):
+        odmt = oracle.refine_optimize(oracle.cand_dedisperse(x[c].cpu().numpy(), f, dm[c], tbin), f, tbin, dm[c])[0]
+        S, W, j, i, s = oracle.refine_mf(odmt, 0.1)
+        assert (res[0][c]["maxdmid"], res[0][c]["maxtid"], res[0][c]["wn"]) == (j, i, W[j, i])
+        assert res[0][c]["snr"] == np.float32(s)

@@ -68,6 +68,17 @@ constexpr int kMfRowsMax = 2048, kMfMapsMax = 512;
 // Bytes of LDS per k_mf_rows workgroup: three to a CU (512 samples, 256 cutouts:
 // 824 us; four to a CU 843, two 939).
 constexpr int kMfRowsLds = 52 * 1024;
+// Rows of no whole 16-byte lines read LDS a word at a time; over 1536 samples
+// four or three such rows fit a workgroup, and k_mf_scan, which does not
+// depend on it, is the faster from about 18 x 1024 rows on: 1901 samples 1.04
+// of its time at 20 x 1024 rows, 1.23 at 64, 0.82 at 8; 1601 samples 0.97, 1.18
+// and 0.76; 1501 samples 0.91 at 64.  Where four rows fit and k_mf_box's rows
+// leave room for two workgroups per CU, not three, only from 64 x 1024 rows on
+// (1801 samples 0.89 at 24, 1.00 at 64).
+inline bool mf_word_rows(int nbin, int rows, long nrows)
+{
+    return nbin <= 1536 || nrows <= (rows < 4 || 3 * (32 * nbin + 2048) <= 160 * 1024 ? 18 : 64) * 1024L;
+}
 
 // include/candidate.h:116-119, no contraction (the reference computes it as written)
 __device__ __host__ inline double dmdelay(double dm, double fh, double fl)
@@ -1053,17 +1064,20 @@ extern "C" int tx_refine_run(tx_refiner *r, int ncand, const float *cutouts, con
         M.nrows = (long)nc * nrow;
         M.ncol = nbin;
         M.pick = nullptr;
-        bool picked = false; // the results' times and widths are there
+        const auto argmax = [&](const int *rowarg, const int *rowwid) {
+            hipLaunchKernelGGL(k_argmax, dim3((unsigned)nc), dim3(256), 0, r->stream, (const float *)r->d_rowmax, rowarg,
+                               rowwid, nrow, r->d_res_i, r->d_res_i + r->batch, r->d_res_s, r->d_res_i + 2 * r->batch);
+        };
         const bool maps = M.snr || M.wid;
-        if (nbin <= (maps ? kMfMapsMax : kMfRowsMax)) {
-            const bool v4 = nbin % 4 == 0 && ((uintptr_t)dmt_out & 15) == 0;
-            const int nu = (nbin + 63) / 64;
-            MfRow T;
-            T.nchunk = (nu + 7) / 8;
-            const int cu = (nu + T.nchunk - 1) / T.nchunk;
-            T.W = v4 ? (r->vwn.back() + 3) / 4 * 4 : r->vwn.back();
-            T.pitch = v4 ? ((nbin + T.W) / 4 | 1) * 4 : (nbin + T.W) | 1;
-            T.nrows = std::max(1, std::min(64, (kMfRowsLds / 4 - 64 * cu * T.nchunk) / (T.pitch + 64)));
+        const bool v4 = nbin % 4 == 0 && ((uintptr_t)dmt_out & 15) == 0;
+        const int nu = (nbin + 63) / 64;
+        MfRow T;
+        T.nchunk = (nu + 7) / 8;
+        const int cu = (nu + T.nchunk - 1) / T.nchunk;
+        T.W = v4 ? (r->vwn.back() + 3) / 4 * 4 : r->vwn.back();
+        T.pitch = v4 ? ((nbin + T.W) / 4 | 1) * 4 : (nbin + T.W) | 1;
+        T.nrows = std::max(1, std::min(64, (kMfRowsLds / 4 - 64 * cu * T.nchunk) / (T.pitch + 64)));
+        if (nbin <= (maps ? kMfMapsMax : kMfRowsMax) && (v4 || mf_word_rows(nbin, T.nrows, M.nrows))) {
             // reads past a row's last sample (whose results do not count) stay in the allocation
             const auto shm = [&] { return ((size_t)T.nrows * (T.pitch + 64) + 64 * cu * T.nchunk) * 4; };
             auto kernel = [&](bool m) {
@@ -1073,12 +1087,9 @@ extern "C" int tx_refine_run(tx_refiner *r, int ncand, const float *cutouts, con
             hipLaunchKernelGGL(kernel(maps), dim3((unsigned)((M.nrows + T.nrows - 1) / T.nrows)), dim3(256), shm(),
                                r->stream, M, T);
             RCHK(hipGetLastError());
-            if (!maps) {
-                hipLaunchKernelGGL(k_argmax, dim3((unsigned)nc), dim3(256), 0, r->stream, r->d_rowmax,
-                                   (const int *)nullptr, (const int *)nullptr, nrow, r->d_res_i,
-                                   r->d_res_i + r->batch, r->d_res_s, r->d_res_i + 2 * r->batch);
-                RCHK(hipGetLastError());
-                picked = true;
+            argmax(maps ? r->d_rowarg : nullptr, maps ? r->d_rowwid : nullptr);
+            RCHK(hipGetLastError());
+            if (!maps) { // the best rows once more, for their times and widths
                 M.pick = r->d_res_i;
                 M.nrows = nrow;
                 M.rowarg = r->d_res_i + r->batch;
@@ -1102,11 +1113,7 @@ extern "C" int tx_refine_run(tx_refiner *r, int ncand, const float *cutouts, con
             else
                 hipLaunchKernelGGL(k_mf_box<64>, mg, dim3(256), shm, r->stream, M);
             RCHK(hipGetLastError());
-        }
-        if (!picked) {
-            hipLaunchKernelGGL(k_argmax, dim3((unsigned)nc), dim3(256), 0, r->stream, r->d_rowmax,
-                               r->d_rowarg, r->d_rowwid, nrow, r->d_res_i, r->d_res_i + r->batch, r->d_res_s,
-                               r->d_res_i + 2 * r->batch);
+            argmax(r->d_rowarg, r->d_rowwid);
             RCHK(hipGetLastError());
         }
         std::vector<int> ri(3 * (size_t)r->batch);
