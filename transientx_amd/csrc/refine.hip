@@ -1104,9 +1104,7 @@ extern "C" int tx_refine_run(tx_refiner *r, int ncand, const float *cutouts, con
             RCHK(hipGetLastError());
             const size_t shm = 4 * 2 * (size_t)nbin * 4;
             const dim3 mg((unsigned)((M.nrows + 3) / 4));
-            if (nbin <= 512)
-                hipLaunchKernelGGL(k_mf_box<8>, mg, dim3(256), shm, r->stream, M);
-            else if (nbin <= 1024)
+            if (nbin <= 1024) // over kMfMapsMax: shorter rows never come here
                 hipLaunchKernelGGL(k_mf_box<16>, mg, dim3(256), shm, r->stream, M);
             else if (nbin <= 2048)
                 hipLaunchKernelGGL(k_mf_box<32>, mg, dim3(256), shm, r->stream, M);
