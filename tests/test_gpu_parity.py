@@ -665,3 +665,30 @@ def test_stage2_passes_of_many_and_few_rows(shape, dtype):
             assert "does not fit" in str(e) and lds == 20480, e
             continue
         assert len(seen) == nblocks
+
+
+@pytest.mark.parametrize("in_load", [False, True])
+@pytest.mark.parametrize("q", [1, 2])
+@pytest.mark.parametrize("ncc", [1, 2, 4, 8])
+def test_stage1_shapes_of_float_rows(ncc, q, in_load):
+    """Every stage-1 shape of float rows, from an f32 ring and with the front
+    end in the load: several passes of several channels per sub-band, slots past
+    the last coarse DM, tiles past the block's end."""
+    C, ndump, nblocks = 160, 1037, 4
+    obs, raw, vwn, kw = small_case(seed=ncc + 10 * q, C=C, ndump=ndump, nblocks=nblocks)
+    kw.update(nsub=5, ndm=45, group=9)
+    op = oracle_plan(obs, ndump, kw)
+    say("case stage 1 ncc", ncc, "q", q, "front end in load", in_load, "coarse DMs", op.info().ndmc)
+    off, gain = oracle.frontend_stats(raw[:ndump], 1, 1)
+    x = oracle.frontend_u8(raw, 1, 1, off, gain)
+    beam = Beam(C, ndump, dtype="f32")
+    try:
+        if in_load:
+            beam.set_frontend(C, 1, 1, off, gain, in_load=True)
+        plan = Plan(beam, **kw, shapes={"s1_ncc": ncc, "s1_q": q})
+        for b in range(1, nblocks + 1):
+            beam.push((raw if in_load else x)[(b - 1) * ndump:b * ndump])
+            plan.dedisp_run()
+            assert np.array_equal(all_tim(plan), op.dedisperse(x, op.window_start(b))), f"block {b}"
+    finally:
+        beam.close()

@@ -620,12 +620,12 @@ __global__ __launch_bounds__(256) void k_stage1_u8(Stage1Args a)
 // Adds n staged rows into SL slots (fine DMs in stage 2, coarse DMs in the f32
 // stage 1) of R samples each, STEP words apart from buf on: row i of slot d
 // starts at lane table off[j]'s entry (i - j*SC)*SL + d, SC = 64/SL rows per
-// table, taken with v_readlane (no memory wait between rows).  Only the first
-// NA slots read and add.  A slot's samples are added and the slot is at once
-// read for the next row, so that the other slots' adds cover the reads.
+// table, NT tables, taken with v_readlane (no memory wait between rows).  Only
+// the first NA slots read and add.  A slot's samples are added and the slot is
+// at once read for the next row, so that the other slots' adds cover the reads.
 // Rows are added in ascending order.
-template <int SL, int NA, int R, int STEP>
-__device__ __forceinline__ void add_rows(const float *buf, int n, const int (&off)[4], float (&acc)[SL][R])
+template <int SL, int NA, int R, int STEP, int NT>
+__device__ __forceinline__ void add_rows(const float *buf, int n, const int (&off)[NT], float (&acc)[SL][R])
 {
     constexpr int SC = 64 / SL;
     float v[NA][R];
@@ -649,12 +649,12 @@ __device__ __forceinline__ void add_rows(const float *buf, int n, const int (&of
 #pragma unroll
     for (int d = 0; d < NA; d++) get(d, off[0], 0);
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
+    for (int j = 0; j < NT; j++) {
         const int cn = min(SC, n - j * SC);
 #pragma unroll 1
         for (int q = 1; q < cn; q++) step(off[j], q * SL);
-        if (j == 3 || (j + 1) * SC >= n) break;
-        step(off[j < 3 ? j + 1 : 3], 0);
+        if (j == NT - 1 || (j + 1) * SC >= n) break;
+        step(off[j < NT - 1 ? j + 1 : NT - 1], 0);
     }
 #pragma unroll
     for (int d = 0; d < NA; d++)
@@ -696,22 +696,15 @@ __global__ __launch_bounds__(256) void k_stage1_f32(Stage1Args a)
     constexpr bool kScalar = NCC >= 8;
     auto mins = [&](int jc) { return (d1min + s * a.cps)[min(jc + lane, a.cps - 1)]; }; // as in k_stage1_u8
     int dml = kScalar ? 0 : mins(0);
-    // where coarse DM k of channel row i starts in LDS: lane (i % SC)*NCC + k of
-    // table i / SC (CH <= 16 rows in 4 tables)
-    constexpr int SC = 64 / NCC;
-    auto offs = [&](int jc, int(&o)[4]) {
-#pragma unroll
-        for (int t = 0; t < 4; t++) {
-            const int i = t * SC + lane / NCC;
-            o[t] = 0;
-            if (i < a.CH && jc + i < a.cps) {
-                const int j = s * a.cps + jc + i;
-                o[t] = i * a.RS + a.d1[(long)j * a.d1pitch + k0 + lane % NCC] - d1min[j];
-            }
-        }
+    // where coarse DM k of channel row i starts in LDS: lane i*NCC + k (a pass
+    // has at most 16 rows)
+    auto offs = [&](int jc) {
+        const int i = lane / NCC;
+        if (i >= a.CH || jc + i >= a.cps) return 0;
+        const int j = s * a.cps + jc + i;
+        return (int)(i * a.RS + a.d1[(long)j * a.d1pitch + k0 + lane % NCC] - d1min[j]);
     };
-    int off[4], noff[4];
-    if (!kScalar) offs(0, off);
+    int off[1] = {kScalar ? 0 : offs(0)}, noff = 0;
     float acc[NCC][U];
 #pragma unroll
     for (int k = 0; k < NCC; k++)
@@ -749,7 +742,7 @@ __global__ __launch_bounds__(256) void k_stage1_f32(Stage1Args a)
                 lds_fill_rows((const uint32_t *)(ring + j0), a.pitch, lane * a.RS, (int)start, nch, nch * a.RS,
                               (uint32_t *)lds_f, wave, 4, lane);
             dml = mins(jc + a.CH);
-            offs(jc + a.CH, noff);
+            noff = offs(jc + a.CH);
         }
         lds_fill_done();
         if (FE) {
@@ -801,9 +794,8 @@ __global__ __launch_bounds__(256) void k_stage1_f32(Stage1Args a)
                     for (int u = 0; u < U; u++) acc[k][u] += v[k][u];
             }
         } else {
-            add_rows<NCC, NCC, U, 256>(lds_f + tid, nch, off, acc);
-#pragma unroll
-            for (int t = 0; t < 4; t++) off[t] = noff[t];
+            add_rows<NCC, NCC, U, 256, 1>(lds_f + tid, nch, off, acc);
+            off[0] = noff;
         }
     }
 
@@ -986,9 +978,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
         const float *buf = lds2 + (p & 1) * a.half;
         // only the wave's live DM slots (a prefix of d) read and add
         if (nact == DPW) {
-            add_rows<DPW, DPW, R, 64>(buf + lane, s1 - s0, cur, acc);
+            add_rows<DPW, DPW, R, 64, 4>(buf + lane, s1 - s0, cur, acc);
         } else if (DPW > 1 && nact == DPW - 1) {
-            add_rows<DPW, (DPW > 1 ? DPW - 1 : 1), R, 64>(buf + lane, s1 - s0, cur, acc);
+            add_rows<DPW, (DPW > 1 ? DPW - 1 : 1), R, 64, 4>(buf + lane, s1 - s0, cur, acc);
         } else if (nact > 0) { // ragged group ends
             for (int s = s0; s < s1; s++) {
 #pragma unroll
