@@ -2,14 +2,17 @@
 
 The plan's built-in cost model picks the stage-1 tile (coarse DMs per
 workgroup, output quads per thread) and the stage-2 tile (fine DMs per wave,
-samples per lane, LDS per workgroup).  The autotuner times the
-alternatives on synthetic 8-bit blocks of the row's real shape, stage by
-stage (the two stages are independent), and returns the fastest; shapes
-never change results, only speed.  Results are cached per (device, row
-shape) in a JSON file ($TX_AUTOTUNE_CACHE or ~/.cache/transientx_amd/autotune.json).
+samples per lane, LDS per workgroup).  The autotuner times that choice and
+the alternatives on synthetic 8-bit blocks of the row's real shape, stage by
+stage (the two stages are independent), and returns the fastest; a stage is
+left to the plan unless another shape is measurably faster.  Shapes never
+change results, only speed.  Results are cached per (device, library, row
+shape) in a JSON file ($TX_AUTOTUNE_CACHE or ~/.cache/transientx_amd/autotune.json):
+another build of the kernels is timed anew.
 """
 from __future__ import annotations
 
+import hashlib
 import json
 import os
 from pathlib import Path
@@ -19,9 +22,9 @@ import numpy as np
 from . import _lib
 from .search import Beam, Plan
 
-S1_CANDIDATES = [(16, 2), (16, 1), (8, 2), (8, 1), (4, 2)]
-# float rows take 4x the LDS of 8-bit rows (and 8 coarse DMs at most): narrower tiles
-S1_CANDIDATES_F32 = [(8, 2), (8, 1), (4, 2), (4, 1), (2, 2), (2, 1)]
+S1_CANDIDATES = [(16, 2), (16, 1), (8, 2), (8, 1), (4, 2), (4, 1), (2, 2), (2, 1), (1, 2), (1, 1)]
+# float rows take 4x the LDS of 8-bit rows and 8 coarse DMs at most
+S1_CANDIDATES_F32 = S1_CANDIDATES[2:]
 # per-workgroup stage-2 LDS budgets: one, two, three or four workgroups per
 # 160 KB CU (clamped to the device's per-workgroup maximum)
 S2_LDS = (163840, 81920, 53248, 40960)
@@ -30,6 +33,35 @@ S2_LDS = (163840, 81920, 53248, 40960)
 def _cache_path() -> Path:
     p = os.environ.get("TX_AUTOTUNE_CACHE")
     return Path(p) if p else Path.home() / ".cache" / "transientx_amd" / "autotune.json"
+
+
+# a shape has to beat the plan's own choice by more than two runs of one shape differ
+GAIN = 0.99
+
+
+def _library_id() -> str:
+    """Which kernels were timed: a digest of the library."""
+    return hashlib.sha1(_lib.LIBPATH.read_bytes()).hexdigest()[:12]
+
+
+def _device_id() -> str:
+    """The device kind: the marketing name can read empty (e.g. under a
+    profiler), the ISA and CU count identify it."""
+    import torch
+
+    props = torch.cuda.get_device_properties(0)
+    return f"{getattr(props, 'gcnArchName', '')}/{props.multi_processor_count}CU"
+
+
+def _blocks(nchans, ndump, dtype):
+    """Two synthetic blocks on the device."""
+    import torch
+
+    g = torch.Generator(device="cuda")
+    g.manual_seed(12345)
+    data = [(torch.randn((ndump, nchans), generator=g, device="cuda") * 12 + 128).round().clamp(0, 255)
+            .to(torch.uint8) for _ in range(2)]
+    return data if dtype == "u8" else [d.float() - 128.0 for d in data]
 
 
 def _key(nchans, freqs, tsamp, ndump, overlap, dms, ddm, ndm, nsub, device_name):
@@ -66,14 +98,10 @@ def tune_row(nchans, freqs, tsamp, ndump, row, vwn, overlap=0.0, nblocks=8, use_
              verbose=False, dtype="u8"):
     """Fastest launch shapes for a row (dms, ddm, ndm, nsub) of 8-bit
     (dtype "u8") or float (dtype "f32", a different stage-1 kernel) data:
-    a dict of PlanDesc overrides (s1_ncc, s1_q, s2_shape, s2_lds)."""
-    import torch
-
-    # the marketing name can read empty (e.g. under a profiler); the ISA and
-    # CU count identify the device kind
-    props = torch.cuda.get_device_properties(0)
-    name = f"{getattr(props, 'gcnArchName', '')}/{props.multi_processor_count}CU"
-    key = _key(nchans, freqs, tsamp, ndump, overlap, *row, name) + ("" if dtype == "u8" else f"|{dtype}")
+    a dict of PlanDesc overrides (s1_ncc, s1_q, s2_shape, s2_lds), without a
+    stage's where the plan's own choice is the fastest."""
+    key = (_key(nchans, freqs, tsamp, ndump, overlap, *row, f"{_device_id()}|{_library_id()}")
+           + ("" if dtype == "u8" else f"|{dtype}"))
     path = _cache_path()
     cache = {}
     if use_cache and path.exists():
@@ -83,29 +111,28 @@ def tune_row(nchans, freqs, tsamp, ndump, row, vwn, overlap=0.0, nblocks=8, use_
             cache = {}
         if key in cache:
             return dict(cache[key]["shapes"])
-    g = torch.Generator(device="cuda")
-    g.manual_seed(12345)
-    data = [(torch.randn((ndump, nchans), generator=g, device="cuda") * 12 + 128).round().clamp(0, 255)
-            .to(torch.uint8) for _ in range(2)]
-    if dtype != "u8":
-        data = [d.float() - 128.0 for d in data]
+    data = _blocks(nchans, ndump, dtype)
     res = {}
-    best1, t1 = {}, None
-    for ncc, q in (S1_CANDIDATES if dtype == "u8" else S1_CANDIDATES_F32):
-        t = _time_stage(nchans, freqs, tsamp, ndump, row, vwn, overlap, {"s1_ncc": ncc, "s1_q": q}, data,
-                        "stage1", nblocks, dtype)
-        res[f"s1 {ncc},{q}"] = t
-        if t is not None and (t1 is None or t < t1):
-            best1, t1 = {"s1_ncc": ncc, "s1_q": q}, t
+
+    def best(stage, candidates):
+        """The plan's choice ({}) or the fastest candidate, and its time."""
+        def timed(shapes):
+            t = _time_stage(nchans, freqs, tsamp, ndump, row, vwn, overlap, shapes, data, stage, nblocks, dtype)
+            res[f"{stage} " + (",".join(str(v) for v in shapes.values()) or "plan")] = t
+            return t
+
+        own = timed({})
+        shape, t = {}, own
+        for c in candidates:
+            tc = timed(c)
+            if tc is not None and (t is None or tc < (t if shape else GAIN * own)):
+                shape, t = c, tc
+        return shape, t
+
+    best1, t1 = best("stage1", [{"s1_ncc": n, "s1_q": q} for n, q in
+                                (S1_CANDIDATES if dtype == "u8" else S1_CANDIDATES_F32)])
     nshape = _lib.lib().tx_stage2_shapes(None, 0)
-    best2, t2 = {}, None
-    for sh in range(1, nshape + 1):
-        for lds in S2_LDS:
-            t = _time_stage(nchans, freqs, tsamp, ndump, row, vwn, overlap, {"s2_shape": sh, "s2_lds": lds},
-                            data, "stage2", nblocks, dtype)
-            res[f"s2 {sh},{lds}"] = t
-            if t is not None and (t2 is None or t < t2):
-                best2, t2 = {"s2_shape": sh, "s2_lds": lds}, t
+    best2, t2 = best("stage2", [{"s2_shape": sh, "s2_lds": lds} for sh in range(1, nshape + 1) for lds in S2_LDS])
     shapes = {**best1, **best2}
     if verbose:
         print(json.dumps({"row": list(row), "times_ms": res, "best": shapes}), flush=True)
