@@ -958,10 +958,11 @@ __global__ __launch_bounds__(256) void k_kad_down_tm(Frames F, int td, int fd, i
 // XLibs kadane<float>; declared: the running sum restarts after it drops
 // below zero, strict '>' keeps the earliest maximum).  sg is 1, or -1 for the
 // strongest negative run (the product is exact, so the FMA is one add).
-struct Kadane {
+// I: the type that holds a sample's number.
+template <class I> struct Kadane {
     float best = -INFINITY, cur = 0.f;
-    int s = 0, bs = 0, be = 0;
-    __device__ __forceinline__ void step(int i, float sg, float v)
+    I s = 0, bs = 0, be = 0;
+    __device__ __forceinline__ void step(I i, float sg, float v)
     {
         cur = fmaf(sg, v, cur);
         const bool up = cur > best;
@@ -989,13 +990,14 @@ struct Kadane {
 // kadaneF 2: per (frame, downsampled channel) the strongest positive and
 // negative runs.  zap[4*g..]: positive then negative range, empty when not
 // zapped.  ds as k_kad_down leaves it.
+template <class I>
 __global__ void k_kad_scan(int nframes, int ncd, long nsd, int td, int fd, float thre, const int *wnlimit,
                            const float *ds, long *zap)
 {
     const long g = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (g >= (long)nframes * ncd) return;
     const float *ch = ds + g * nsd;
-    Kadane p, m;
+    Kadane<I> p, m;
     long i = 0;
     for (; i + 16 <= nsd; i += 16) { // 16 loads in flight
         float v[16];
@@ -1003,13 +1005,13 @@ __global__ void k_kad_scan(int nframes, int ncd, long nsd, int td, int fd, float
         for (int u = 0; u < 16; u++) v[u] = ch[i + u];
 #pragma unroll
         for (int u = 0; u < 16; u++) {
-            p.step((int)(i + u), 1.f, v[u]);
-            m.step((int)(i + u), -1.f, v[u]);
+            p.step((I)(i + u), 1.f, v[u]);
+            m.step((I)(i + u), -1.f, v[u]);
         }
     }
     for (; i < nsd; i++) {
-        p.step((int)i, 1.f, ch[i]);
-        m.step((int)i, -1.f, ch[i]);
+        p.step((I)i, 1.f, ch[i]);
+        m.step((I)i, -1.f, ch[i]);
     }
     const int wl = wnlimit[g / ncd];
     p.zap(td, fd, wl, thre, zap + 4 * g);
@@ -1033,7 +1035,7 @@ __global__ __launch_bounds__(kColThreads) void k_kad_scan_tm(int ncd, long nsd, 
     const int c0 = min((int)(blockIdx.x % per) * kColCh, ncd - kColCh);
     const int h = tid - 64, q4 = (h & 7) * 4, r0 = h >> 3;
     const float sg = lane < 32 ? 1.f : -1.f;
-    Kadane p;
+    Kadane<int> p;
     auto put = [&](int k, const ColChunk &c) {
 #pragma unroll
         for (int u = 0; u < 4; u++)
@@ -1135,7 +1137,7 @@ __global__ __launch_bounds__(256) void k_kad_rows(Frames F, int td, int fd, int 
     if (w < 2 && lane < ng) {
         const float sg = w ? -1.f : 1.f;
         const float *row = ds + lane * pitch;
-        Kadane p;
+        Kadane<int> p;
 #pragma unroll 8
         for (int i = 0; i < nsd; i++) p.step(i, sg, row[i]);
         p.zap(td, fd, wnlimit[f], thre, &z[lane][2 * w]);
@@ -1182,6 +1184,17 @@ __global__ __launch_bounds__(256) void k_kad_zero_tm(Frames F, int fd, int ncd, 
 
 inline unsigned blocks_for(long n) { return (unsigned)((n + 255) / 256); }
 
+// A launch holds fewer than 2^32 threads.  Frames of which each of the kernels
+// here takes at most `threads` a frame go in slices of this many, one after the
+// other on the stream.
+inline int frames_per_launch(int nframes, long threads)
+{
+    return (int)std::max(1L, std::min((long)nframes, (1L << 31) / threads));
+}
+// Longest time-major frames of the kernels that take several threads a sample
+// there (and number samples in 32 bits); longer ones take the general kernels.
+constexpr long kMaxTmZdot = 1L << 28, kMaxTmKad = 1L << 26;
+
 int check_frames(const Frames &F)
 {
     if (!F.x || F.nframes < 0 || F.nchan < 1 || F.nsamp < 1 || F.cstride < 1 || F.tstride < 1 ||
@@ -1215,6 +1228,14 @@ extern "C" int tx_rfi_zdot(void *stream, float *data, int nframes, long fstride,
     if (nframes == 0) return TX_OK;
     if (!work || work_bytes < tx_rfi_work_bytes(TX_RFI_ZDOT, nframes, nchan, nsamp, 1, 1))
         return set_error(TX_EINVAL, "rfi: work buffer smaller than tx_rfi_work_bytes");
+    // at most 512 threads for 8 rows, 10 a sample, one for 32 samples of a channel
+    const int most = frames_per_launch(nframes, 64L * nchan + 10 * nsamp + (nchan + 255L) * (nsamp + 31) / 32 + 1024);
+    if (nframes > most) {
+        for (int f = 0; f < nframes && rc == TX_OK; f += std::min(most, nframes - f))
+            rc = tx_rfi_zdot(stream, data + f * fstride, std::min(most, nframes - f), fstride, nchan, nsamp, cstride,
+                             tstride, work, work_bytes);
+        return rc;
+    }
     hipStream_t st = (hipStream_t)stream;
     double *s = (double *)work, *sess = s + (size_t)nframes * nsamp, *stat = sess + 2 * (size_t)nframes;
     const long nfc = (long)nframes * nchan, nfs = (long)nframes * nsamp;
@@ -1248,7 +1269,7 @@ extern "C" int tx_rfi_zdot(void *stream, float *data, int nframes, long fstride,
             hipLaunchKernelGGL(k_zdot_ss, dim3(blocks_for(nframes)), dim3(256), 0, st, F, cs, sess);
             hipLaunchKernelGGL(k_zdot_rows<true>, dim3(nb), dim3(256), 0, st, F, cs, css);
         }
-    } else if (cstride == 1 && fstride == (long)nchan * nsamp && tstride == nchan) {
+    } else if (cstride == 1 && fstride == (long)nchan * nsamp && tstride == nchan && nsamp <= kMaxTmZdot) {
         // the DataBuffer layout [nframes][nsamp][nchan]
         const unsigned ng = (unsigned)((nchan + kColCh - 1) / kColCh);
         const bool narrow = nchan < kColCh;
@@ -1287,10 +1308,19 @@ extern "C" int tx_rfi_kadanef(void *stream, float *data, int nframes, long fstri
     if (!wnlimit) return set_error(TX_EINVAL, "rfi: null wnlimit");
     if (!work || work_bytes < tx_rfi_work_bytes(TX_RFI_KADANEF, nframes, nchan, nsamp, td, fd))
         return set_error(TX_EINVAL, "rfi: work buffer smaller than tx_rfi_work_bytes");
+    // a thread for each downsampled sample or for 64 samples of a channel, 256 for 8 downsampled channels
+    const int most = frames_per_launch(nframes, ncd * nsd + (ncd + 255L) * (nsd + 7) / 8 +
+                                                    (nchan + 255L) * (nsamp + 63) / 64 + 33L * nchan + 1024);
+    if (nframes > most) {
+        for (int f = 0; f < nframes && rc == TX_OK; f += std::min(most, nframes - f))
+            rc = tx_rfi_kadanef(stream, data + f * fstride, std::min(most, nframes - f), fstride, nchan, nsamp,
+                                cstride, tstride, td, fd, threshold, wnlimit + f, work, work_bytes);
+        return rc;
+    }
     hipStream_t st = (hipStream_t)stream;
     float *ds = (float *)work;
     long *zap = (long *)((char *)work + ((size_t)nframes * ncd * nsd * sizeof(float) + 255) / 256 * 256);
-    if (cstride == 1 && fstride == (long)nchan * nsamp && tstride == nchan && ncd >= kColCh) {
+    if (cstride == 1 && fstride == (long)nchan * nsamp && tstride == nchan && ncd >= kColCh && nsamp <= kMaxTmKad) {
         // the DataBuffer layout [nframes][nsamp][nchan]
         const long nct = (ncd + 255) / 256, nzt = ((long)ncd * fd + 255) / 256;
         hipLaunchKernelGGL(k_kad_down_tm, dim3((unsigned)(nct * ((nsd + kKdT - 1) / kKdT) * nframes)), dim3(256), 0,
@@ -1306,7 +1336,8 @@ extern "C" int tx_rfi_kadanef(void *stream, float *data, int nframes, long fstri
     } else {
         hipLaunchKernelGGL(k_kad_down, dim3(blocks_for((long)nframes * ncd * nsd)), dim3(256), 0, st, F, td, fd,
                            ncd, nsd, ds);
-        hipLaunchKernelGGL(k_kad_scan, dim3(blocks_for((long)nframes * ncd)), dim3(256), 0, st, nframes, ncd, nsd,
+        const auto scan = nsd < 1L << 31 ? k_kad_scan<int> : k_kad_scan<long>;
+        hipLaunchKernelGGL(scan, dim3(blocks_for((long)nframes * ncd)), dim3(256), 0, st, nframes, ncd, nsd,
                            td, fd, threshold, wnlimit, (const float *)ds, zap);
         hipLaunchKernelGGL(k_kad_zero, dim3(blocks_for((long)nframes * ncd * fd)), dim3(256), 0, st, F, fd, ncd,
                            (const long *)zap);
