@@ -242,7 +242,7 @@ __global__ __launch_bounds__(256) void k_tree_pass(TreeArgs A)
 template <int U, bool P2>
 __global__ __launch_bounds__(512) void k_tree_rows(TreeArgs A)
 {
-    extern __shared__ float rows[]; // [G][ncol], then the shifts: G a level (or G row delays)
+    extern __shared__ __attribute__((aligned(16))) float rows[]; // [G][ncol], then the shifts: G a level (or G row delays)
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int c = blockIdx.y;
     const int G = 1 << (A.b - A.a);
@@ -609,7 +609,7 @@ template <bool V4> __device__ __forceinline__ void mf_csum(const float *x, float
 template <int CU, bool V4, bool MAPS>
 __global__ __launch_bounds__(256) void k_mf_rows(MfArgs M, MfRow T)
 {
-    extern __shared__ float smem[];
+    extern __shared__ __attribute__((aligned(16))) float smem[];
     __shared__ double smean[64], svar[64];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int ncol = M.ncol, W = T.W;
