@@ -126,9 +126,8 @@ def test_time_major_zdot_and_kadanef_edges(nchan, nsamp, nf):
         assert same_bits(np.ascontiguousarray(t.cpu().numpy().transpose(0, 2, 1)), r), (td, fd)
 
 
-# channel-major zdot around the tiles of rows in LDS: 32 rows to 600 samples,
-# fewer for longer rows, none past about 2,400 (the row kernels), and rows of no
-# whole 16-byte lines; few frames (a tile per workgroup) and many (a frame each)
+# channel-major zdot in and past the tiles of rows in LDS (32 rows to 556 samples, 16 to 1012, 8 to 1700, then the row
+# kernels; the edges themselves below) and rows of no whole 16-byte lines; few frames (a tile per workgroup) and many
 @pytest.mark.parametrize("nchan,nbin,nf", [(33, 31, 2), (32, 32, 130), (5, 1, 3), (70, 601, 1), (40, 605, 129),
                                            (20, 1023, 2), (9, 2049, 1), (4, 2600, 1), (37, 65, 128)])
 def test_channel_major_zdot_tiles(nchan, nbin, nf):
@@ -355,3 +354,10 @@ def test_more_frames_than_a_launch_holds(op, layout, nf, nchan, nsamp):
     f(x)
     # zero samples of zdot's single channels may be NaN: equal bits
     assert torch.equal(x.view(torch.int32), ref.view(torch.int32))
+
+
+# both sides of each change of rows per tile, the last sample of the 80 KB of LDS, with a tile and a frame per workgroup
+@pytest.mark.parametrize("nbin", [556, 557, 1012, 1013, 1700, 1701])
+@pytest.mark.parametrize("nchan,nf", [(37, 2), (9, 130)])
+def test_channel_major_zdot_tile_edges(nbin, nchan, nf):
+    test_channel_major_zdot_frame_counts(nchan, nbin, nf)
