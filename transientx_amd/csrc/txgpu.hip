@@ -716,6 +716,27 @@ static void plan_free(tx_plan *p)
     hipFree(p->d_sess_n);
 }
 
+// The lowest and highest delay of each channel among the coarse DMs of chunk kc
+// (NCC of them).  The lowest, where the channel's LDS row starts, is rounded
+// down: rows start on whole 32-bit words of an 8-bit ring (tiles start on
+// multiples of 4 samples and the ring length is one); f32 rows too, so that an
+// f32 plan also serves the front end in the stage-1 load over an 8-bit ring.
+// (Channels in the inner loop: every shape's tables are formed at each plan.)
+static void stage1_extents(const PlanMath &pm, int NCC, int kc, int *lo, int *hi)
+{
+    const int *d = pm.d1.data() + (size_t)kc * NCC * pm.nchans;
+    std::copy(d, d + pm.nchans, lo);
+    std::copy(d, d + pm.nchans, hi);
+    for (int k = kc * NCC + 1; k < std::min(pm.ndmc, (kc + 1) * NCC); k++) {
+        d += pm.nchans;
+        for (int j = 0; j < pm.nchans; j++) {
+            lo[j] = std::min(lo[j], d[j]);
+            hi[j] = std::max(hi[j], d[j]);
+        }
+    }
+    for (int j = 0; j < pm.nchans; j++) lo[j] &= ~3;
+}
+
 // Stage-1 shape: NCC coarse DMs per workgroup (one input pass serves them
 // all), Q quads per thread, CH channel rows per LDS pass within an LDS budget
 // (f32 rows, four times the 8-bit ones: 24, 32 or 40 KB; 8-bit rows 24 KB, six
@@ -737,28 +758,15 @@ static bool choose_stage1(tx_plan *p, std::vector<int> &d1min, int force_ncc, in
     if (force_ncc > maxncc) return false;
     ncc0 = force_ncc > 0 ? force_ncc : std::min(ncc0, 8);
     double best = 1e300;
+    std::vector<int> lo(pm.nchans), hi(pm.nchans);
     for (int NCC = ncc0; NCC >= 1; NCC >>= 1) {
         if (force_ncc > 0 && NCC != force_ncc) continue;
         const int nkc = (pm.ndmc + NCC - 1) / NCC;
-        std::vector<int> mn((size_t)nkc * pm.nchans);
         int spread = 0;
-        for (int kc = 0; kc < nkc; kc++)
-            for (int j = 0; j < pm.nchans; j++) {
-                int lo = 1 << 30, hi = -(1 << 30);
-                for (int k = kc * NCC; k < std::min(pm.ndmc, (kc + 1) * NCC); k++) {
-                    const int d = pm.d1[(size_t)k * pm.nchans + j];
-                    lo = std::min(lo, d);
-                    hi = std::max(hi, d);
-                }
-                // rows start on whole 32-bit words of an 8-bit ring (tiles
-                // start on multiples of 4 samples and the ring length is
-                // one); f32 rows too, so that an f32 plan also serves the
-                // front end in the stage-1 load over an 8-bit ring
-                lo -= ((lo % 4) + 4) % 4;
-                mn[(size_t)kc * pm.nchans + j] = lo;
-                spread = std::max(spread, hi - lo);
-            }
-        bool kept = false;
+        for (int kc = 0; kc < nkc; kc++) {
+            stage1_extents(pm, NCC, kc, lo.data(), hi.data());
+            for (int j = 0; j < pm.nchans; j++) spread = std::max(spread, hi[j] - lo[j]);
+        }
         for (int Q = 2; Q >= 1; Q--) {
             if (force_q > 0 && Q != force_q) continue;
             // u8: words covering spread (from the word-aligned row start) +
@@ -799,45 +807,44 @@ static bool choose_stage1(tx_plan *p, std::vector<int> &d1min, int force_ncc, in
                 p->RS = RS;
                 p->nkc = nkc;
                 p->read1 = u8 ? (long)RS * 4 + 4 : (long)RS + 1;
-                kept = true;
             }
         }
-        if (kept) d1min = mn;
     }
-    return best < 1e300;
+    if (best == 1e300) return false;
+    d1min.resize((size_t)p->nkc * pm.nchans);
+    for (int kc = 0; kc < p->nkc; kc++)
+        stage1_extents(pm, p->NCC, kc, d1min.data() + (size_t)kc * pm.nchans, hi.data());
+    return true;
 }
 
 // Stage-2 delay extents of every DM block for blocks of `blk` fine DMs.
-static int stage2_extents(const PlanMath &pm, int blk, int nblk, std::vector<int> &d2min,
-                          std::vector<int> &d2span, std::vector<int> *nact)
+static void stage2_extents(const PlanMath &pm, int blk, int nblk, std::vector<int> &d2min,
+                           std::vector<int> &d2span, std::vector<int> &nact)
 {
     d2min.assign((size_t)pm.ndmc * nblk * pm.nsub, 0);
     d2span.assign(d2min.size(), 0);
-    if (nact) nact->assign((size_t)pm.ndmc * nblk, 0);
-    int span = 0;
+    nact.assign((size_t)pm.ndmc * nblk, 0);
     for (int k = 0; k < pm.ndmc; k++)
         for (int b = 0; b < nblk; b++) {
+            const size_t w = (size_t)k * nblk + b;
             const long i0 = (long)k * pm.group + (long)b * blk;
             const long i1 =
                 std::min<long>(std::min<long>((long)(k + 1) * pm.group, pm.ndm), i0 + blk);
-            if (nact) (*nact)[(size_t)k * nblk + b] = (int)std::max<long>(0, i1 - i0);
-            for (int s = 0; s < pm.nsub; s++) {
-                int lo = 0, hi = 0;
-                if (i1 > i0) {
-                    lo = 1 << 30;
-                    hi = -(1 << 30);
-                    for (long i = i0; i < i1; i++) {
-                        const int d = pm.d2[(size_t)i * pm.nsub + s];
-                        lo = std::min(lo, d);
-                        hi = std::max(hi, d);
-                    }
+            nact[w] = (int)std::max<long>(0, i1 - i0);
+            if (i1 <= i0) continue;
+            int *lo = d2min.data() + w * pm.nsub, *hi = d2span.data() + w * pm.nsub;
+            const int *d = pm.d2.data() + (size_t)i0 * pm.nsub;
+            std::copy(d, d + pm.nsub, lo);
+            std::copy(d, d + pm.nsub, hi);
+            for (long i = i0 + 1; i < i1; i++) {
+                d += pm.nsub;
+                for (int s = 0; s < pm.nsub; s++) {
+                    lo[s] = std::min(lo[s], d[s]);
+                    hi[s] = std::max(hi[s], d[s]);
                 }
-                d2min[((size_t)k * nblk + b) * pm.nsub + s] = lo;
-                d2span[((size_t)k * nblk + b) * pm.nsub + s] = hi - lo;
-                span = std::max(span, hi - lo);
             }
+            for (int s = 0; s < pm.nsub; s++) hi[s] -= lo[s];
         }
-    return span;
 }
 
 // Pass plan of stage 2 for one shape: each DM block's sub-band rows (its
@@ -847,16 +854,14 @@ static int stage2_extents(const PlanMath &pm, int blk, int nblk, std::vector<int
 struct Stage2Plan {
     std::vector<int> ldsoff, npass, pstart, pused;
     int pstride = 0, maxrow = 0;
-    long passes = 0;
 };
-static bool stage2_passes(const PlanMath &pm, int nblkall, int T, const std::vector<int> &sp,
-                          const std::vector<int> &nact, int half, int maxsub, Stage2Plan &pl)
+static bool stage2_passes(const PlanMath &pm, int nblkall, int T, const std::vector<int> &sp, int half, int maxsub,
+                          Stage2Plan &pl)
 {
     pl.ldsoff.assign((size_t)nblkall * pm.nsub, 0);
     pl.npass.assign(nblkall, 0);
     std::vector<std::vector<int>> starts(nblkall), fills(nblkall);
     pl.maxrow = 0;
-    pl.passes = 0;
     for (int w = 0; w < nblkall; w++) {
         int used = 0;
         starts[w].push_back(0);
@@ -875,7 +880,6 @@ static bool stage2_passes(const PlanMath &pm, int nblkall, int T, const std::vec
         starts[w].push_back(pm.nsub);
         fills[w].push_back(used);
         pl.npass[w] = (int)starts[w].size() - 1;
-        if (nact[w]) pl.passes += pl.npass[w];
     }
     pl.pstride = 0;
     for (auto &v : starts) pl.pstride = std::max(pl.pstride, (int)v.size());
@@ -886,6 +890,30 @@ static bool stage2_passes(const PlanMath &pm, int nblkall, int T, const std::vec
         std::copy(fills[w].begin(), fills[w].end(), pl.pused.begin() + (size_t)w * pl.pstride);
     }
     return true;
+}
+
+// The passes of the DM blocks with DMs in them that stage2_passes would make, -1
+// if a row does not fit.
+static long stage2_count(const PlanMath &pm, int T, const std::vector<int> &sp, const std::vector<int> &nact, int half,
+                         int maxsub)
+{
+    long passes = 0;
+    for (size_t w = 0; w < nact.size(); w++) {
+        const int *span = sp.data() + w * pm.nsub;
+        int used = 0, first = 0, n = 1;
+        for (int s = 0; s < pm.nsub; s++) {
+            const int len = span[s] + T;
+            if (len > half) return -1;
+            if (used + len > half || s - first >= maxsub) {
+                first = s;
+                used = 0;
+                n++;
+            }
+            used += (len + 3) & ~3;
+        }
+        if (nact[w]) passes += n;
+    }
+    return passes;
 }
 
 static int stage2_maxsub(int DPW) { return std::min(64, 4 * (64 / DPW)); }
@@ -908,14 +936,15 @@ static bool choose_stage2(tx_plan *p, std::vector<int> &d2min, std::vector<int> 
     const PlanMath &pm = p->pm;
     const int max_lds = p->beam->max_lds;
     double best = 1e300;
-    int bi = -1;
+    int bi = -1, have = 0;
+    std::vector<int> mn, sp, nact;
     for (int c = 0; c < kNumStage2Shapes; c++) {
         if (force_shape > 0 && force_shape - 1 != c) continue;
         const int DPW = kStage2Shapes[c][0], R = kStage2Shapes[c][1];
         const int blk = kS2Waves * DPW, T = 64 * R;
         const int nblk = (pm.group + blk - 1) / blk;
-        std::vector<int> mn, sp, nact;
-        stage2_extents(pm, blk, nblk, mn, sp, &nact);
+        if (blk != have) stage2_extents(pm, blk, nblk, mn, sp, nact);
+        have = blk;
         double adds = 0, fill = 0, wgs = 0;
         for (size_t w = 0; w < nact.size(); w++) {
             if (!nact[w]) continue;
@@ -927,11 +956,11 @@ static bool choose_stage2(tx_plan *p, std::vector<int> &d2min, std::vector<int> 
         const double ntile = (double)((pm.nsamples + T - 1) / T);
         for (int kb : {160, 80, 52, 40}) {
             const int lds = force_lds > 0 ? std::min(max_lds, force_lds) : std::min(max_lds, kb * 1024);
-            Stage2Plan pl;
-            if (stage2_passes(pm, pm.ndmc * nblk, T, sp, nact, (lds / 8) & ~3, stage2_maxsub(DPW), pl)) {
+            const long passes = stage2_count(pm, T, sp, nact, (lds / 8) & ~3, stage2_maxsub(DPW));
+            if (passes >= 0) {
                 const bool few = DPW * R < 32;
                 const double share = kb == 160 ? 1.15 : kb == 80 ? 1. : kb == 52 ? (few ? 0.86 : 1.03) : few ? 0.81 : 1.08;
-                const double cost = ntile * (adds * shape + 1.08 * fill + 14900. * pl.passes + 87000. * wgs) *
+                const double cost = ntile * (adds * shape + 1.08 * fill + 14900. * passes + 87000. * wgs) *
                                     (share + 220. / (ntile * wgs));
                 if (cost < best) {
                     best = cost;
@@ -947,9 +976,8 @@ static bool choose_stage2(tx_plan *p, std::vector<int> &d2min, std::vector<int> 
     p->R = kStage2Shapes[bi][1];
     const int blk = kS2Waves * p->DPW;
     p->nblk = (pm.group + blk - 1) / blk;
-    std::vector<int> nact;
-    stage2_extents(pm, blk, p->nblk, d2min, d2span, &nact);
-    return stage2_passes(pm, pm.ndmc * p->nblk, 64 * p->R, d2span, nact, p->half2, stage2_maxsub(p->DPW), plan);
+    stage2_extents(pm, blk, p->nblk, d2min, d2span, nact);
+    return stage2_passes(pm, pm.ndmc * p->nblk, 64 * p->R, d2span, p->half2, stage2_maxsub(p->DPW), plan);
 }
 
 template <typename T>
