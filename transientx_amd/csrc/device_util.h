@@ -51,6 +51,22 @@ __device__ __forceinline__ void lds_fill_rows(const uint32_t *__restrict__ src, 
     }
 }
 
+// The same row by row, for rows of at least a chunk per wave: finding a
+// chunk's row costs more instructions than walking such rows.  The waves go on
+// where the row before left off, so that their shares stay equal.
+__device__ __forceinline__ void lds_fill_long_rows(const uint32_t *__restrict__ src, long pitch, int off, int first,
+                                                   int nr, int used, uint32_t *buf, int wave, int nw, int lane)
+{
+    int turn = 0; // the wave whose chunk is a row's first
+    for (int r = 0; r < nr; r++) {
+        const int a = __builtin_amdgcn_readlane(off, r);
+        const int len = (r + 1 < nr ? __builtin_amdgcn_readlane(off, r + 1) : used) - a;
+        const int mine = wave - turn + (wave < turn ? nw : 0);
+        lds_fill16(src + (long)r * pitch + __builtin_amdgcn_readlane(first, r), buf + a, len, mine, nw, lane);
+        turn = (turn + (len + 255) / 256) % nw;
+    }
+}
+
 __device__ inline void lds_fill_done()
 {
     __builtin_amdgcn_s_waitcnt(0); // vmcnt(0): every global->LDS load has landed

@@ -956,8 +956,18 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
         const int s0 = ldc(a.pstart, pb + p), nr = ldc(a.pstart, pb + p + 1) - s0;
         int x = base + t.min;
         x -= x >= Lsub ? Lsub : 0;
-        lds_fill_rows((const uint32_t *)(grp + (long)s0 * a.spitch), a.spitch, t.off, x, nr, ldc(a.pused, pb + p),
-                      (uint32_t *)(lds2 + (p & 1) * a.half), wave, nw, lane);
+        const int used = ldc(a.pused, pb + p);
+        const uint32_t *src = (const uint32_t *)(grp + (long)s0 * a.spitch);
+        uint32_t *buf = (uint32_t *)(lds2 + (p & 1) * a.half);
+        // Rows of two chunks a wave or more are staged row by row: stage 2 of
+        // 2048 channels, 128 sub-bands, 200 DMs from 3000 by 10 (16 us) takes
+        // 200 us so and 237 us with the chunks dealt over the rows, 4096
+        // channels, 64 sub-bands, 100 DMs from 4000 by 10 57 us and 65 us.
+        // Shorter rows: two DMs a wave lose 2-3% from one chunk a wave.
+        if (used > nw * 512 * nr)
+            lds_fill_long_rows(src, a.spitch, t.off, x, nr, used, buf, wave, nw, lane);
+        else
+            lds_fill_rows(src, a.spitch, t.off, x, nr, used, buf, wave, nw, lane);
     };
     int cur[4], nxt[4] = {0, 0, 0, 0};
     Rows rows;
