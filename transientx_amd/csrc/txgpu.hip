@@ -746,8 +746,9 @@ static void stage1_extents(const PlanMath &pm, int NCC, int kc, int *lo, int *hi
 // 1 + W/workgroups for the end of a launch that does not fill the CUs.  The
 // constants are fitted to the measured times of every shape on 23 rows (64 to
 // 4096 channels, 512 to 31,250 samples, 24 to 2500 DMs): the choice is within
-// 1% of the best shape on average, 8% at worst, where the widest NCC that
-// fits, the rule before, is 1.5 times slower on average.
+// 1% of the best shape on average, 8% at worst (on 78 others within 2%, 21% at
+// worst), where the widest NCC that fits, the rule before, is 1.5 times slower
+// on average.
 static bool choose_stage1(tx_plan *p, std::vector<int> &d1min, int force_ncc, int force_q)
 {
     const PlanMath &pm = p->pm;
@@ -920,16 +921,23 @@ static int stage2_maxsub(int DPW) { return std::min(64, 4 * (64 / DPW)); }
 
 // Stage-2 shape (DPW fine DMs per wave, R samples per lane) and LDS per
 // workgroup: force_shape and force_lds, or where those are 0 every shape with
-// one to four workgroups' LDS per CU.  The cost of a choice counts, per time
-// tile and DM block: one LDS read and add per sample of its live DMs, each
-// sub-band row staged (the block's delay extent + the tile), its passes
-// (barrier and fill latency the double buffer does not cover) and its start
-// and end; times a factor for the workgroups that share a CU (shapes of 16
-// accumulators have the registers for three or four) plus the end of a launch
-// that does not fill the CUs.  Fitted to the measured times of every choice on
-// 23 rows (as for stage 1): within 2.5% of the best on average; one LDS size and
-// no cost for workgroups, the rule before, were 19% off on average and 1.9
-// times slower on the 16 us row.
+// one to four workgroups' LDS per CU.  The cost of a choice is a workgroup's
+// work and waits times the rounds of workgroups that the CUs run.  Work: the
+// sub-band rows staged (the block's delay extent + the tile), and per sample
+// of each DM an LDS read and add, by shape (nothing beyond the staging where
+// each wave adds 16 samples of one DM; most for waves of fewer than DPW - 1
+// DMs, which take the kernel's loop for ragged group ends); a workgroup with
+// uneven waves ends with its busiest.  Waits: a barrier and fill latency per
+// pass.  Both shrink as workgroups share a CU (its LDS, or the shape's
+// registers, allow one to four).  Workgroups that nearly fill the CUs already
+// run into a second round (0.93), and a round begun costs a third of what it
+// lacks.  Fitted to the measured times of every choice on 168 rows (8 to 4096
+// channels, 300 to 31,250 samples, 1 to 2500 DMs, DM steps of 0.2 to 10): within
+// 2% of the best on average, 28% at worst.  The rule before, linear in these
+// and fitted on 23 rows, was 8% off on average and 59% at worst, on rows of
+// large DM steps: stage 2 of 992 channels, 62 sub-bands, 830 DMs from 1500 by 5
+// took 256 us and takes 195 us, of 1520 channels, 95 sub-bands, 316 DMs from
+// 1500 by 5 213 us and 153 us.
 static bool choose_stage2(tx_plan *p, std::vector<int> &d2min, std::vector<int> &d2span,
                           Stage2Plan &plan, int force_shape, int force_lds)
 {
@@ -945,23 +953,33 @@ static bool choose_stage2(tx_plan *p, std::vector<int> &d2min, std::vector<int> 
         const int nblk = (pm.group + blk - 1) / blk;
         if (blk != have) stage2_extents(pm, blk, nblk, mn, sp, nact);
         have = blk;
-        double adds = 0, fill = 0, wgs = 0;
+        const double add = DPW == 8 ? 6.5 : DPW == 4 ? 2.6 : DPW == 2 ? (R == 16 ? 2.6 : 2.1) : R == 32 ? 1.1 : 0.;
+        double work = 0, wgs = 0;
         for (size_t w = 0; w < nact.size(); w++) {
             if (!nact[w]) continue;
-            adds += (double)nact[w] * T * pm.nsub;
+            double sum = 0, busiest = 0, fill = 0;
+            for (int wave = 0; wave < std::min(kS2Waves, nact[w]); wave++) {
+                const int live = (nact[w] - wave + kS2Waves - 1) / kS2Waves; // the wave's DMs
+                const double c1 = live * (live >= DPW - 1 ? add : 13.);
+                sum += c1;
+                busiest = std::max(busiest, c1);
+            }
             for (int s = 0; s < pm.nsub; s++) fill += (sp[w * pm.nsub + s] + T + 3) & ~3;
+            work += 41. * fill + (0.4 * sum + 0.6 * kS2Waves * busiest) * T * pm.nsub;
             wgs++;
         }
-        const double shape = DPW == 8 ? 1.97 : DPW * R < 32 ? 1. : DPW == 1 ? 0.93 : DPW == 2 ? 1.065 : 1.;
-        const double ntile = (double)((pm.nsamples + T - 1) / T);
+        const double n = wgs * ((pm.nsamples + T - 1) / T);           // workgroups of the launch
+        const int regs = DPW * R == 32 ? 2 : DPW == 2 ? 3 : 4;        // those a CU's registers hold
         for (int kb : {160, 80, 52, 40}) {
             const int lds = force_lds > 0 ? std::min(max_lds, force_lds) : std::min(max_lds, kb * 1024);
             const long passes = stage2_count(pm, T, sp, nact, (lds / 8) & ~3, stage2_maxsub(DPW));
             if (passes >= 0) {
-                const bool few = DPW * R < 32;
-                const double share = kb == 160 ? 1.15 : kb == 80 ? 1. : kb == 52 ? (few ? 0.86 : 1.03) : few ? 0.81 : 1.08;
-                const double cost = ntile * (adds * shape + 1.08 * fill + 14900. * passes + 87000. * wgs) *
-                                    (share + 220. / (ntile * wgs));
+                const int occ = std::max(1, std::min(regs, 160 * 1024 / lds));
+                const double rounds = n / (256 * 0.93 * occ);
+                const double share = std::min(std::max(1., n / 256), (double)occ); // workgroups on a CU
+                const double times = rounds <= 1 ? share : occ * (rounds + 0.35 * (std::ceil(rounds) - rounds));
+                const double cost = (work * std::pow(share, -0.3) + 200000. * passes / share) / wgs * times *
+                                    std::pow(std::min(1., n / 256), 0.2);
                 if (cost < best) {
                     best = cost;
                     bi = c;
